@@ -14,10 +14,12 @@
 // few that crossed into a neighbour's cells are added with LDS float atomics
 // afterwards.  The tile goes to HBM, and the grid operator (MODE 2) sums the
 // tiles of the 3^d neighbouring blocks into the output grid.  The same pass
-// writes the next substep's binning hints (direction codes and ranks).
+// takes its particles from the previous substep's direction lists and writes
+// the next one's, and now and then moves the particles into the sorted order
+// (mpm_binning.h, as k_p2g and k_g2p do).
 #pragma once
 
-#include "mpm_device.h"
+#include "mpm_binning.h"
 
 namespace mpm {
 
@@ -27,15 +29,16 @@ struct G2P2GGeo {
   static constexpr int kNodes = D == 3 ? kEdge * kEdge * kEdge : kEdge * kEdge;
 };
 
-template <int D, bool Q>
+template <int D, bool Q, int ORDER = kOrderGiven>
 __global__ __launch_bounds__(kThreads) void k_g2p2g(
-    const Params* __restrict__ scenes, const int* __restrict__ slab, float* __restrict__ pf,
-    const int* __restrict__ pi, int64_t cap, const int* __restrict__ perm,
+    const Params* __restrict__ scenes, const int* __restrict__ slab, const float* pf,
+    const int* __restrict__ pi, int64_t cap, int* __restrict__ perm,
     const int4* __restrict__ chunks, const int* __restrict__ totals,
     const float4* __restrict__ grid_in, float4* __restrict__ tiles, int n_final,
     unsigned* __restrict__ maxv, const int* __restrict__ step, int stride,
-    int* __restrict__ code, int* __restrict__ nkey,
-    int* __restrict__ dcount, int* __restrict__ count_next, int* __restrict__ err) {
+    int* members, int* dseg, int* __restrict__ count_next, int* __restrict__ err,
+    PrevBinning prev, const int* __restrict__ pstart, float* pf_out, int* __restrict__ pi_out,
+    int n, int nw) {
   using L = Layout<D>;
   constexpr int NPB = Geo<D>::kNodesPerBlock, TN = Geo<D>::kTileNodes;
   constexpr int E8 = G2P2GGeo<D>::kEdge, TN8 = G2P2GGeo<D>::kNodes;
@@ -51,6 +54,7 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
   __shared__ int cstart[CELLS], ccount[CELLS];
   __shared__ unsigned char order[kBatch];
   __shared__ int dwcnt[WAVES][32];
+  __shared__ int dstart[32];
   __shared__ float red[WAVES];
 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -71,6 +75,13 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
     for (int i = threadIdx.x; i < TN8; i += kThreads) stile[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     for (int i = threadIdx.x; i < WAVES * CELLS; i += kThreads) (&wcnt[0][0])[i] = 0;
     for (int i = threadIdx.x; i < WAVES * 32; i += kThreads) (&dwcnt[0][0])[i] = 0;
+    int ids[1] = {-1};
+    if (ORDER == kOrderLists) {
+      const int first = pstart[ck.x];
+      wave_members<D, 1>(lb, ck.y - first + threadIdx.x, 0, ck.z - first, scenes[0], prev, ids);
+    } else if (threadIdx.x < nc) {
+      ids[0] = perm[ck.y + threadIdx.x];
+    }
     for (int i = threadIdx.x; i < TN; i += kThreads) {
       const int tl[3] = {i % kTile, (i / kTile) % kTile, i / (kTile * kTile)};
       int q[3], ln[3];
@@ -91,13 +102,16 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
 
     // ---- phase 1: G2P, advection, constitutive update, staging ----
     const int t = threadIdx.x;
-    const bool live = t < nc;
+    const int p = ids[0];
+    if (t < nc && p < 0) atomicOr(err, 16);  // counts and lists disagree (cannot happen)
+    const bool live = p >= 0;
+    const int po = ORDER == kOrderMove ? ck.y + t : p;  // slot of the new state
     bool inner = false;
     int cell = 0, shell = -1;  // shell: output-tile node of the new base (crossed particles)
-    int dir = 13, key_new = ck.x;
+    int dir = 13;
     if (live) {
       using PS = Particles<D, Q, true>;
-      const int p = perm[ck.y + t];
+      if (ORDER != kOrderGiven) perm[ck.y + t] = po;
       const int mat = pi[(int64_t)L::MAT * cap + p];
       float xp[3] = {0, 0, 0}, fx[3] = {0, 0, 0}, w[3][3], vp[3] = {0, 0, 0};
       int l[3] = {0, 0, 0};
@@ -114,6 +128,11 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
       }
       float nv[3] = {0.0f, 0.0f, 0.0f}, nC[3][3] = {{0.0f}};
       const bool fresh = pi[(int64_t)L::ORIG * cap + p] >= n_final;  // mpm:396-399
+      if (ORDER == kOrderMove) {
+        PS::move_xvC(pf, pf_out, cap, p, po);
+        for (int w = 0; w < L::NI; w++)
+          pi_out[(int64_t)w * cap + po] = pi[(int64_t)w * cap + p];
+      }
       if (!fresh) {  // G2P, mpm:386-394 (tensor-product form of k_g2p)
         float pe[3][3] = {{0.0f}}, wd[3][3];
 #pragma unroll
@@ -163,13 +182,13 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
       }
       float xn[3] = {xp[0], xp[1], xp[2]};
       if (mat != kStationary) {  // mpm:401-403: x advances by the stored v
-        PS::store_v(pf, cap, p, nv);
+        PS::store_v(pf_out, cap, po, nv);
 #pragma unroll
         for (int a = 0; a < D; a++) {
           vp[a] = nv[a];
           xn[a] = xp[a] + P.dt * nv[a];
         }
-        PS::store_x(pf, cap, p, xn);  // xn: the stored x, scattered around below
+        PS::store_x(pf_out, cap, po, xn);  // xn: the stored x, scattered around below
       }
 #pragma unroll
       for (int a = 0; a < D; a++) vmax = fmaxf(vmax, fabsf(vp[a]));
@@ -201,8 +220,11 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
       PS::load_F(pf, cap, p, F);
       float Jp = P.plastic ? PS::load_Jp(pf, cap, p) : 1.0f;
       constitutive<D, true, Q>(mat, P, P.mu_0, P.lambda_0, F, nC, Jp, stress);
-      PS::store_F(pf, cap, p, F);
-      if (P.plastic) PS::store_Jp(pf, cap, p, Jp);
+      PS::store_F(pf_out, cap, po, F);
+      if (P.plastic)
+        PS::store_Jp(pf_out, cap, po, Jp);
+      else if (!Q && ORDER == kOrderMove)
+        PS::store_Jp(pf_out, cap, po, PS::load_Jp(pf, cap, p));
       const float mass = P.p_mass;  // mpm:474-483 (no water density here)
       float Ad[3][3] = {{0.0f}}, q[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -243,8 +265,6 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
       }
       if (fits && near) {
         dir = (dd[2] + 1) * 9 + (dd[1] + 1) * 3 + (dd[0] + 1);
-        qb[D - 1] += P.zoff;
-        key_new = encode_local<D>(qb, P);
       } else if (fits) {
         atomicOr(err, 1);  // left the window
       }
@@ -341,7 +361,7 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
           }
     }
 
-    // ---- next substep's binning hints (as k_g2p) ----
+    // ---- next substep's direction lists (as k_g2p) ----
     unsigned long long dpeers = __ballot(live);
 #pragma unroll
     for (int bit = 0; bit < 5; bit++) {
@@ -352,20 +372,17 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
     const int drank = (int)__popcll(dpeers & lt);
     if (live && drank == 0) dwcnt[wave][dir] = (int)__popcll(dpeers);
     __syncthreads();
-    if (threadIdx.x < 27) {
-      const int d = threadIdx.x;
+    if (threadIdx.x < 64) {
       int run = 0;
+      if (lane < 27) {
 #pragma unroll
-      for (int w = 0; w < WAVES; w++) {
-        const int cnt = dwcnt[w][d];
-        dwcnt[w][d] = run;
-        run += cnt;
+        for (int w = 0; w < WAVES; w++) {
+          const int cnt = dwcnt[w][lane];
+          dwcnt[w][lane] = run;
+          run += cnt;
+        }
       }
-      dcount[(int64_t)c * 27 + d] = run;
-      if (run > 0) {
-        int q[3] = {lb[0] + d % 3 - 1, lb[1] + (d / 3) % 3 - 1, lb[2] + d / 9 - 1};
-        atomicAdd(&count_next[encode_local<D>(q, P)], run);
-      }
+      write_groups<D>(c, lb, P, run, dstart, dseg, count_next);
     }
 
     // ---- phase 4: sum the private tiles, write the node tile ----
@@ -396,12 +413,18 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
       out[i] = acc;
     }
     __syncthreads();
-    if (live) {
-      code[ck.y + t] = dir | ((dwcnt[wave][dir] + drank) << 8);
-      nkey[ck.y + t] = key_new;
-    }
+    if (live) members[ck.y + dstart[dir] + dwcnt[wave][dir] + drank] = po;
     __syncthreads();
   }
+  // particles outside the window (sorted to the end, frozen) move as they are
+  if (ORDER == kOrderMove)
+    for (int j = totals[kTotValid] + blockIdx.x * kThreads + threadIdx.x; j < n;
+         j += gridDim.x * kThreads) {
+      const int p = perm[j];
+      for (int w = 0; w < nw; w++) pf_out[(int64_t)w * cap + j] = pf[(int64_t)w * cap + p];
+      for (int w = 0; w < L::NI; w++) pi_out[(int64_t)w * cap + j] = pi[(int64_t)w * cap + p];
+      perm[j] = j;
+    }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, off));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = vmax;

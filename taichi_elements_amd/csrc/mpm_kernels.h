@@ -30,10 +30,16 @@ struct LBState {
 // Totals written on the device by the block scan (read by persistent kernels).
 enum Total : int { kTotValid = 0, kTotChunks = 1, kTotActive = 2, kTotPBlocks = 3, kTotCount = 4 };
 
+// Source of a transfer's particle order (k_p2g, k_g2p2g).
+enum Order : int { kOrderGiven = 0, kOrderLists = 1, kOrderMove = 2 };
+
 struct SubstepBuffers {
   float* pf;  // particle float components
   float* pf_out;  // where p2g / g2p write the new state (== pf: in place)
   int* pi;    // particle int components
+  float* pf_alt;  // the same arrays again: a substep with move set writes
+  int* pi_alt;    // the particles there, in sorted order, and the two swap
+  bool move;
   int64_t cap;
   int n;
   int* keys;        // [n] block key per slot
@@ -66,17 +72,16 @@ struct SubstepBuffers {
   int persistent_groups;
   int g2p_waves;  // g2p's occupancy target: 0 = the compiler's choice, 6 = six waves per SIMD
   int parity;  // substep counter parity (selects the digit-histogram copy)
-  // neighbour-bounded sort: the previous substep's chunks and block tables,
-  // direction codes / new keys per previous sorted position, per-chunk
-  // direction counts and output offsets
+  // steady-state binning (mpm_binning.h): the previous substep's chunks and
+  // block tables, and the direction lists its last transfer left; this
+  // substep's own (use_g2p2g reads the one and writes the other in one kernel)
   int4* chunks_prev;
   int* pchunk_begin_prev;
   int* pchunk_cnt_prev;
-  int* totals_prev;
-  int* code;
-  int* nkey;
-  int* dcount;      // [chunk_cap][27]
-  int* doff;        // [chunk_cap][27]
+  const int* members_prev;
+  const int* dseg_prev;
+  int* members;     // [cap] slots, grouped by direction (null: g2p leaves no lists)
+  int* dseg;        // [chunk_cap][27] count | start << 16
   int4* tile_prefix;  // two-level block scan
   // use_g2p2g mode: the fused transfer reads grid_in and writes grid;
   // particles with an insertion index >= n_final skip the G2P
@@ -86,8 +91,6 @@ struct SubstepBuffers {
   bool quant;         // packed particle layout (PackedLayout<D>)
   int nw;             // particle float-buffer words per slot
   bool full_sort;     // radix-sort the slots (first substep / positions set by the host)
-  bool perm_identity; // the slots were just reordered into the previous order
-  int* keys_sorted;   // output: block keys in sorted order
 };
 
 class Timer;
@@ -127,8 +130,9 @@ void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const f
                     const float* gout, float* gin, float* gE, float4* gbar, float* abuf,
                     float* nu_part, float* gnu, hipStream_t st, Timer* timer);
 
-template <int D>
-void launch_reorder(SubstepBuffers& B, float* pf_alt, int* pi_alt, hipStream_t st, Timer* timer);
+// Block keys in sorted order (of the binning whose chunks and totals are given).
+void launch_sorted_keys(const int4* chunks, const int* totals, int n, int total_blocks, int* keys,
+                        hipStream_t st);
 
 template <int D>
 void launch_append(SubstepBuffers& B, const float* x, const float* v, const int* mat, int k,

@@ -6,21 +6,23 @@
 //   k_bscan*          scan of the dense block window: particle offsets,
 //                     transfer work items (chunks), active grid blocks  (replaces the pointer
 //                                                                        SNodes and deactivate_all)
-//   k_onesweep        stable LSD radix sort of slots by block key (with k_keys), or
-//   k_offsets,        the steady-state neighbour sort: the previous order
-//   k_nscatter        stably re-sorted from g2p's direction codes
-//   k_p2g             per chunk: constitutive update + scatter into an
-//                     LDS tile of (4+2)^d nodes, tile written to HBM     (p2g, mpm:487-584)
+//   k_onesweep        stable LSD radix sort of slots by block key (with k_keys)
+//   k_p2g             per chunk: its particles (from the sort, or in the
+//                     steady state from g2p's direction lists),
+//                     constitutive update + scatter into an
+//                     LDS tile of (4+2)^d nodes, tile written to HBM     (p2g, mpm:487-584);
+//                     every few substeps the particle state also moves
+//                     into the sorted order
 //   k_grid_op         per active node: sum of the overlapping tiles,
 //                     normalisation, gravity, post-process              (mpm:586-692)
 //   k_g2p             per chunk: LDS tile of grid velocity, gather,
-//                     advection, max |v|, next binning's hints          (g2p, mpm:694-735)
-//   k_reorder         every few substeps: particle state moved into the sorted order
+//                     advection, max |v|, next binning's lists          (g2p, mpm:694-735)
 // use_g2p2g replaces p2g / grid op / g2p with k_g2p2g + k_grid_op_g2p2g
 // (mpm_g2p2g.h); the differentiable backward runs the adjoints of
 // mpm_adjoint.h.  Particles are read and written through Particles<D, Q>
 // (mpm_particles.h), instantiated for the float and the packed layout.
 #include "mpm_kernels.h"
+#include "mpm_binning.h"
 #include "mpm_adjoint.h"
 #include "mpm_g2p2g.h"
 
@@ -532,12 +534,22 @@ __global__ __launch_bounds__(kThreads) void k_onesweep(
 // At most 128 VGPRs (4 waves per SIMD): the latency of the particle loads
 // and of the LDS scatter is hidden better than at 3 waves with no spills
 // (measured: 85 -> 75 us per 1M-particle substep, a few spilled registers).
-template <int D, int MODE, bool Q = false>
+// ORDER: where the chunk's particles come from and what p2g does to their
+// order.  kOrderGiven: perm.  kOrderLists: the previous substep's direction
+// lists (wave_members); p2g writes perm.  kOrderMove: perm, and the particle
+// state moves into the sorted order on the way (position j becomes slot j of
+// pf_out / pi_out): p2g reads every field but two integers anyway and is
+// bound by the vector ALU and LDS, so the extra writes cost less than a pass
+// of their own (1M particles: 76 -> 98 us instead of 76 + 65; 16M: 1.15 ->
+// 2.24 ms instead of 1.15 + 1.64).
+template <int D, int MODE, bool Q = false, int ORDER = kOrderGiven>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_p2g(
-    const Params* __restrict__ scenes, const int* __restrict__ slab, float* __restrict__ pf,
-    const int* __restrict__ pi, int64_t cap, const int* __restrict__ perm,
+    const Params* __restrict__ scenes, const int* __restrict__ slab, const float* __restrict__ pf,
+    const int* __restrict__ pi, int64_t cap, int* __restrict__ perm,
     const int4* __restrict__ chunks, const int* __restrict__ totals, float4* __restrict__ tiles,
-    const float* __restrict__ gf, float* __restrict__ pf_out) {
+    const float* __restrict__ gf, float* __restrict__ pf_out, PrevBinning prev,
+    const int* __restrict__ pstart, int* __restrict__ pi_out, int n, int nw,
+    int* __restrict__ err) {
   using L = Layout<D>;
   constexpr int TN = Geo<D>::kTileNodes;
   constexpr int CELLS = Geo<D>::kNodesPerBlock;  // cells of a block (64 / 16)
@@ -558,6 +570,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     int lbc[3], b[3];
     decode_local<D>(ck.x, scenes[0], lbc);
     const Params& P = scenes[scene_of<D>(lbc, slab)];
+    int ids[kChunkMax / kThreads];  // slots of this thread's particle of each batch
+    if (ORDER == kOrderLists) {
+      const int first = pstart[ck.x];
+      wave_members<D, kChunkMax / kThreads>(lbc, ck.y - first + threadIdx.x, kThreads,
+                                            ck.z - first, scenes[0], prev, ids);
+#pragma unroll
+      for (int k = 0; k < kChunkMax / kThreads; k++) {
+        const int j = ck.y + threadIdx.x + k * kThreads;
+        if (j >= ck.z) continue;
+        if (ids[k] < 0) atomicOr(err, 16);  // counts and lists disagree (cannot happen)
+        perm[j] = max(ids[k], 0);
+      }
+    }
+    if (ORDER == kOrderMove)
+      for (int j = ck.y + threadIdx.x; j < ck.z; j += kThreads) {
+        const int p = perm[j];
+        for (int w = 0; w < L::NI; w++) pi_out[(int64_t)w * cap + j] = pi[(int64_t)w * cap + p];
+        if (P.skip)  // the scene sits the substep out: its state moves unchanged
+          for (int w = 0; w < nw; w++) pf_out[(int64_t)w * cap + j] = pf[(int64_t)w * cap + p];
+        if (P.skip) perm[j] = j;
+      }
     if (P.skip) continue;  // workgroup-uniform: the whole chunk belongs to one scene
     to_local<D>(lbc, P, b);
 #pragma unroll
@@ -571,10 +604,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 
       // ---- phase 1: constitutive update and staging ----
       const int t = threadIdx.x;
-      const bool valid = t < nc;
+      int p = -1;
+      if (ORDER == kOrderLists) {
+#pragma unroll
+        for (int k = 0; k < kChunkMax / kThreads; k++)
+          if (b0 - ck.y == k * kThreads) p = ids[k];
+      } else if (t < nc) {
+        p = perm[b0 + t];
+      }
+      const bool valid = p >= 0;
       int cell = 0;
       if (MODE == 1 && valid) {
-        const int p = perm[b0 + t];
         const int mat = pi[(int64_t)L::MAT * cap + p];
         float fx[3] = {0.0f, 0.0f, 0.0f};
         int l[3] = {0, 0, 0};
@@ -610,13 +650,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         }
       } else if (MODE == 0 && valid) {
         using PS = Particles<D, Q>;
-        const int p = perm[b0 + t];
         const int mat = pi[(int64_t)L::MAT * cap + p];
         float xp[3], vp[3], C[3][3], F[3][3], stress[3][3];
         PS::load_x(pf, cap, p, xp);
         PS::load_v(pf, cap, p, vp);
         PS::load_C(pf, cap, p, C);
         PS::load_F(pf, cap, p, F);
+        const int po = ORDER == kOrderMove ? b0 + t : p;  // slot of the new state
+        if (ORDER == kOrderMove) {
+          PS::move_xvC(pf, pf_out, cap, p, po);
+          perm[po] = po;
+        }
         float Jp = P.plastic ? PS::load_Jp(pf, cap, p) : 1.0f;
         float fx[3] = {0.0f, 0.0f, 0.0f};
         int l[3] = {0, 0, 0};
@@ -635,8 +679,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
           lambda_0 = E * P.kla;
         }
         constitutive<D>(mat, P, mu_0, lambda_0, F, C, Jp, stress);
-        PS::store_F(pf_out, cap, p, F);  // the stress already used F before rounding (mpm:567)
-        if (P.plastic) PS::store_Jp(pf_out, cap, p, Jp);
+        PS::store_F(pf_out, cap, po, F);  // the stress already used F before rounding (mpm:567)
+        if (P.plastic)
+          PS::store_Jp(pf_out, cap, po, Jp);
+        else if (!Q && ORDER == kOrderMove)
+          PS::store_Jp(pf_out, cap, po, PS::load_Jp(pf, cap, p));
         float mass = P.p_mass;  // mpm_solver.py:571-573
         if (mat == kWater) mass *= P.water_density;
         // contribution to node o: w_o * (mass v + A (o - fx) dx) = w_o * (q + Adx o)
@@ -728,6 +775,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     }
     lds_barrier();
   }
+  // particles outside the window (sorted to the end, frozen) move as they are
+  if (ORDER == kOrderMove)
+    for (int j = totals[kTotValid] + blockIdx.x * kThreads + threadIdx.x; j < n;
+         j += gridDim.x * kThreads) {
+      const int p = perm[j];
+      for (int w = 0; w < nw; w++) pf_out[(int64_t)w * cap + j] = pf[(int64_t)w * cap + p];
+      for (int w = 0; w < L::NI; w++) pi_out[(int64_t)w * cap + j] = pi[(int64_t)w * cap + p];
+      perm[j] = j;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -861,8 +917,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
                                                   const float4* __restrict__ grid,
                                                   unsigned* __restrict__ maxv,
                                                   const int* __restrict__ step, int stride,
-                                                  int* __restrict__ code, int* __restrict__ nkey,
-                                                  int* __restrict__ dcount,
+                                                  int* __restrict__ members,
+                                                  int* __restrict__ dseg,
                                                   int* __restrict__ count_next,
                                                   int* __restrict__ err,
                                                   float* __restrict__ pf_out, int n) {
@@ -875,6 +931,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
   __shared__ float red[kThreads / 64];
   __shared__ int dwcnt[kThreads / 64][32];
   __shared__ int dbase[32];  // particles per direction in the chunk's earlier batches
+  __shared__ int dstart[32];
+  // the particles of the earlier batches: direction | rank << 8, slot
+  __shared__ int lcode[kChunkMax - kBatch], lid[kChunkMax - kBatch];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   float vmax = 0.0f;
@@ -911,15 +970,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
     for (int a = 0; a < D; a++) b[a] = (lbl[a] + P.blo[a]) * kBlock;
     // one particle per thread, kBatch particles of the chunk at a time
     for (int b0 = ck.y; b0 < ck.z; b0 += kBatch) {
-      for (int i = threadIdx.x; i < (kThreads / 64) * 32; i += kThreads) (&dwcnt[0][0])[i] = 0;
-      lds_barrier();
       const int j = b0 + threadIdx.x;
       const bool live = j < ck.z;
       int dir = 13;  // block offset of the particle after advection, (dz+1)*9 + (dy+1)*3 + (dx+1)
-      int key_new = ck.x;
+      const int p = live ? perm[j] : 0;
       if (live) {
         using PS = Particles<D, Q>;
-        const int p = perm[j];
         const int mat = pi[(int64_t)L::MAT * cap + p];
         float xp[3] = {0.0f, 0.0f, 0.0f}, fx[3], w[3][3];
         int l[3];
@@ -1029,8 +1085,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
         }
         if (near) {
           dir = (dd[2] + 1) * 9 + (dd[1] + 1) * 3 + (dd[0] + 1);
-          q[D - 1] += P.zoff;
-          key_new = encode_local<D>(q, P);
         } else {
           // left the window (bit 0) or moved more than one block (bit 3): the
           // particle stays binned in its old block and the caller is told
@@ -1040,8 +1094,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
                             : 8);
         }
       }
+      if (!members) continue;  // no binning follows from this substep
       // stable rank of the particle among the chunk's particles with the same
-      // direction; per-chunk direction counts; block counts of the next substep
+      // direction
+      if (lane < 32) dwcnt[wave][lane] = 0;  // the wave's own row, in program order
       unsigned long long peers = __ballot(live);
   #pragma unroll
       for (int bit = 0; bit < 5; bit++) {
@@ -1052,35 +1108,37 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
       const int rank = (int)__popcll(peers & lt);
       if (live && rank == 0) dwcnt[wave][dir] = (int)__popcll(peers);
       lds_barrier();
-      if (threadIdx.x < 27) {
-        const int d = threadIdx.x;
-        int run = dbase[d];
+      const bool last = b0 + kBatch >= ck.z;
+      if (threadIdx.x < 64) {
+        int run = 0;
+        if (lane < 27) {
+          run = dbase[lane];
   #pragma unroll
-        for (int w = 0; w < kThreads / 64; w++) {
-          const int cnt = dwcnt[w][d];
-          dwcnt[w][d] = run;
-          run += cnt;
+          for (int w = 0; w < kThreads / 64; w++) {
+            const int cnt = dwcnt[w][lane];
+            dwcnt[w][lane] = run;
+            run += cnt;
+          }
+          dbase[lane] = run;
         }
-        dbase[d] = run;
+        if (last) write_groups<D>(c, lb, P, run, dstart, dseg, count_next);
       }
       lds_barrier();
       if (live) {
-        code[j] = dir | ((dwcnt[wave][dir] + rank) << 8);
-        nkey[j] = key_new;
+        const int r = dwcnt[wave][dir] + rank;
+        if (last) {
+          members[ck.y + dstart[dir] + r] = p;
+        } else {
+          lcode[j - ck.y] = dir | (r << 8);
+          lid[j - ck.y] = p;
+        }
       }
+      if (last)  // the earlier batches' particles (this thread's own entries)
+        for (int i = threadIdx.x; i < b0 - ck.y; i += kThreads)
+          members[ck.y + dstart[lcode[i] & 255] + (lcode[i] >> 8)] = lid[i];
       lds_barrier();
     }  // batches of the chunk
-    // per-chunk direction counts; block counts of the next substep
-    if (threadIdx.x < 27) {
-      const int d = threadIdx.x;
-      const int run = dbase[d];
-      dcount[(int64_t)c * 27 + d] = run;
-      if (run > 0) {
-        int q[3] = {lb[0] + d % 3 - 1, lb[1] + (d / 3) % 3 - 1, lb[2] + d / 9 - 1};
-        atomicAdd(&count_next[encode_local<D>(q, P)], run);
-      }
-    }
-    lds_barrier();
+    if (!members) lds_barrier();  // the node tile is rewritten for the next chunk
   }
   // out of place: particles outside every chunk (escaped the window; sorted
   // to the end) keep their whole state
@@ -1108,130 +1166,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
 }
 
 // ---------------------------------------------------------------------------
-// neighbour-bounded counting sort (steady-state binning)
-//
-// The order of a substep is the previous order stably sorted by the new
-// block key.  Particles move less than one block per substep, so the members
-// of new block k come from the 3^d old blocks k - d; in the previous order
-// they are grouped by old block (ascending key), then by old chunk, then by
-// position.  k_g2p already gave every particle its direction d and its
-// stable rank among its old chunk's particles with the same d; k_offsets
-// walks each new block's 3^d old neighbours in ascending key order and hands
-// every (old chunk, d) pair its first output position; k_nscatter moves the
-// particle indices.
-// ---------------------------------------------------------------------------
-template <int D>
-__global__ __launch_bounds__(kThreads) void k_offsets(
-    const Params* __restrict__ scenes, const int4* __restrict__ chunks,
-    const int* __restrict__ totals,
-    const int* __restrict__ pstart, const int* __restrict__ count,
-    const int* __restrict__ pchunk_begin_prev, const int* __restrict__ pchunk_cnt_prev,
-    const int* __restrict__ dcount, int* __restrict__ doff, int* __restrict__ err) {
-  // one wave per new chunk; the wave of a block's first chunk does the block:
-  // lane t < 3^d takes old neighbour t in ascending key order, sums its
-  // chunks' counts toward this block, and a wave scan orders the neighbours
-  const Params& P = scenes[0];  // the combined window extents
-  const int nch = totals[kTotChunks];
-  const int lane = threadIdx.x & 63;
-  const int waves = gridDim.x * (kThreads / 64);
-  for (int c = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6); c < nch; c += waves) {
-    const int4 ck = chunks[c];
-    const int bid = ck.x;
-    if (ck.y != pstart[bid]) continue;  // not the first chunk of its block (wave-uniform)
-    int lb[3];
-    decode_local<D>(bid, P, lb);
-    constexpr int NB = D == 3 ? 27 : 9;
-    int c0 = 0, cn = 0, dir = 0, mine = 0;
-    if (lane < NB) {
-      // ascending old key <=> descending offset (dz, dy, dx) in lexicographic order
-      const int dx = 1 - lane % 3, dy = 1 - (lane / 3) % 3, dz = D == 3 ? 1 - lane / 9 : 0;
-      const int q[3] = {lb[0] - dx, lb[1] - dy, lb[2] - dz};
-      if (q[0] >= 0 && q[0] < P.bn[0] && q[1] >= 0 && q[1] < P.bn[1] &&
-          (D == 2 || (q[2] >= 0 && q[2] < P.bn[2]))) {
-        const int ob = encode_local<D>(q, P);
-        c0 = pchunk_begin_prev[ob];
-        cn = pchunk_cnt_prev[ob];
-        dir = (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1);
-        for (int oc = c0; oc < c0 + cn; oc++) mine += dcount[(int64_t)oc * 27 + dir];
-      }
-    }
-    int inc = mine;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int y = __shfl_up(inc, off);
-      if (lane >= off) inc += y;
-    }
-    int run = ck.y + inc - mine;
-    for (int oc = c0; oc < c0 + cn; oc++) {
-      doff[(int64_t)oc * 27 + dir] = run;
-      run += dcount[(int64_t)oc * 27 + dir];
-    }
-    const int total = __shfl(inc, 63);
-    if (lane == 0 && total != count[bid]) atomicOr(err, 16);  // counts disagree (cannot happen)
-  }
-}
-
-__global__ __launch_bounds__(kThreads) void k_nscatter(
-    const int4* __restrict__ chunks_prev, const int* __restrict__ totals_prev,
-    const int* __restrict__ code, const int* __restrict__ nkey, const int* __restrict__ doff,
-    const int* __restrict__ perm_old, int* __restrict__ perm_new, int* __restrict__ keys_new,
-    int n, int total_blocks, int* __restrict__ err) {
-  const int nch = totals_prev[kTotChunks];
-  for (int c = blockIdx.x; c < nch; c += gridDim.x) {
-    const int4 ck = chunks_prev[c];
-    for (int j = ck.y + threadIdx.x; j < ck.z; j += kThreads) {
-      const int cd = code[j];
-      const int pos = doff[(int64_t)c * 27 + (cd & 255)] + (cd >> 8);
-      if (pos >= 0 && pos < n) {
-        perm_new[pos] = perm_old ? perm_old[j] : j;
-        keys_new[pos] = nkey[j];
-      } else {
-        atomicOr(err, 16);
-      }
-    }
-  }
-  // particles outside the window (frozen since an earlier full sort) keep
-  // their places at the end
-  for (int j = totals_prev[kTotValid] + blockIdx.x * kThreads + threadIdx.x; j < n;
-       j += gridDim.x * kThreads) {
-    perm_new[j] = perm_old ? perm_old[j] : j;
-    keys_new[j] = total_blocks;
-  }
-}
-
-// ---------------------------------------------------------------------------
 // particle bookkeeping kernels
 // ---------------------------------------------------------------------------
-template <int D>
-__global__ __launch_bounds__(kThreads) void k_reorder(const float* __restrict__ pf,
-                                                      float* __restrict__ pf2,
-                                                      const int* __restrict__ pi,
-                                                      int* __restrict__ pi2,
-                                                      const int* __restrict__ perm, int n,
-                                                      int64_t cap) {
-  using L = Layout<D>;
-  for (int j = blockIdx.x * kThreads + threadIdx.x; j < n; j += gridDim.x * kThreads) {
-    const int p = perm[j];
-#pragma unroll
-    for (int c = 0; c < L::NF; c++) pf2[(int64_t)c * cap + j] = pf[(int64_t)c * cap + p];
-#pragma unroll
-    for (int c = 0; c < L::NI; c++) pi2[(int64_t)c * cap + j] = pi[(int64_t)c * cap + p];
+// Block keys in sorted order, from the chunks (mpm_read_binning).
+__global__ __launch_bounds__(kThreads) void k_sorted_keys(const int4* __restrict__ chunks,
+                                                          const int* __restrict__ totals, int n,
+                                                          int total_blocks,
+                                                          int* __restrict__ keys) {
+  for (int c = blockIdx.x; c < totals[kTotChunks]; c += gridDim.x) {
+    const int4 ck = chunks[c];
+    for (int j = ck.y + threadIdx.x; j < ck.z; j += kThreads) keys[j] = ck.x;
   }
-}
-
-// Packed layout: the word count depends on the mode, so it is a parameter.
-__global__ __launch_bounds__(kThreads) void k_reorder_words(const float* __restrict__ pf,
-                                                            float* __restrict__ pf2,
-                                                            const int* __restrict__ pi,
-                                                            int* __restrict__ pi2,
-                                                            const int* __restrict__ perm, int n,
-                                                            int64_t cap, int nw, int ni) {
-  for (int j = blockIdx.x * kThreads + threadIdx.x; j < n; j += gridDim.x * kThreads) {
-    const int p = perm[j];
-#pragma unroll 4
-    for (int c = 0; c < nw; c++) pf2[(int64_t)c * cap + j] = pf[(int64_t)c * cap + p];
-    for (int c = 0; c < ni; c++) pi2[(int64_t)c * cap + j] = pi[(int64_t)c * cap + p];
-  }
+  for (int j = totals[kTotValid] + blockIdx.x * kThreads + threadIdx.x; j < n;
+       j += gridDim.x * kThreads)
+    keys[j] = total_blocks;
 }
 
 // New particles: seed_particle (mpm_solver.py:823-838).
@@ -1367,18 +1315,36 @@ struct TimerScope {
   }
 };
 
+// The previous substep's direction lists.
+static PrevBinning prev_binning(const SubstepBuffers& B) {
+  PrevBinning p{};
+  p.pchunk_begin = B.pchunk_begin_prev;
+  p.pchunk_cnt = B.pchunk_cnt_prev;
+  p.chunks = B.chunks_prev;
+  p.dseg = B.dseg_prev;
+  p.members = B.members_prev;
+  return p;
+}
+
+// Whether the transfer walks the direction lists itself (mpm_binning.h says
+// what each way costs): with about one chunk per workgroup, which a scene of
+// this many particles has unless they are spread very thinly.  A substep
+// that moves the particles takes the given order.
+constexpr int kListsInTransfer = 160 * 1024;
+static bool order_in_transfer(const SubstepBuffers& B) {
+  return !B.full_sort && !B.move && B.n <= kListsInTransfer;
+}
+
 // binning of one substep: block counts, the dense-window scan (chunks,
 // active blocks) and the sorted order
 template <int D>
 static void launch_binning(const Params* P, SubstepBuffers& B, hipStream_t st, Timer* tm) {
   const int n = B.n;
-  const int G = B.persistent_groups;
   if (n == 0) return;
   const int nparts = div_up(B.total_blocks, kScanTile);
   const int passes = (B.key_bits + 7) / 8;
   int* ghist = B.ghist + (B.parity & 1) * kMaxRadixPasses * kRadixBins;
   int* ghist_next = B.ghist + ((B.parity & 1) ^ 1) * kMaxRadixPasses * kRadixBins;
-  const int chunk_bound = std::min(B.total_blocks, n) + div_up(n, B.chunk);
   if (B.full_sort) {
     // first substep (or positions changed from the host): block counts from
     // scratch, then a stable radix sort of the slots
@@ -1419,21 +1385,20 @@ static void launch_binning(const Params* P, SubstepBuffers& B, hipStream_t st, T
       vin = vbuf[pass & 1];
     }
     if (vin != B.perm) std::swap(B.perm, B.perm_alt);
-    B.keys_sorted = (int*)kin;
-  } else {
-    TimerScope ts(tm, "k_nsort", st);
-    k_offsets<D><<<clamp_groups(div_up(chunk_bound, kThreads / 64), G), kThreads, 0, st>>>(
-        P, B.chunks, B.totals, B.pstart, B.count, B.pchunk_begin_prev, B.pchunk_cnt_prev,
-        B.dcount, B.doff, B.err);
-    // the previous order: the last substep's permutation, or the slots
-    // themselves right after a physical reorder
-    const int* perm_old = B.perm_identity ? nullptr : B.perm;
-    k_nscatter<<<clamp_groups(chunk_bound, G), kThreads, 0, st>>>(
-        B.chunks_prev, B.totals_prev, B.code, B.nkey, B.doff, perm_old, B.perm_alt, B.keys_alt,
-        n, B.total_blocks, B.err);
-    std::swap(B.perm, B.perm_alt);
-    B.keys_sorted = B.keys_alt;
+  } else if (!order_in_transfer(B)) {
+    TimerScope ts(tm, "k_members", st);
+    const int chunk_bound = std::min(B.total_blocks, n) + div_up(n, B.chunk);
+    k_members<D><<<clamp_groups(div_up(chunk_bound, kThreads / 64), 4096), kThreads, 0, st>>>(
+        P, B.chunks, B.totals, B.pstart, prev_binning(B), B.perm, B.err);
   }
+}
+
+// The slots were rewritten in sorted order by the transfer just launched.
+static void take_moved(SubstepBuffers& B) {
+  std::swap(B.pf, B.pf_alt);
+  std::swap(B.pi, B.pi_alt);
+  B.pf_out = B.pf;
+  B.move = false;
 }
 
 // binning, p2g and the grid operator of one substep
@@ -1457,9 +1422,14 @@ static void launch_g2p2g(const Params* P, const int* slab, SubstepBuffers& B, in
   {
     TimerScope ts(tm, "k_g2p2g", st);
     auto kern = B.quant ? k_g2p2g<D, true> : k_g2p2g<D, false>;
+    if (order_in_transfer(B))
+      kern = B.quant ? k_g2p2g<D, true, kOrderLists> : k_g2p2g<D, false, kOrderLists>;
+    if (B.move) kern = B.quant ? k_g2p2g<D, true, kOrderMove> : k_g2p2g<D, false, kOrderMove>;
     kern<<<clamp_groups(chunk_bound, G), kThreads, 0, st>>>(
         P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.grid_in, B.tiles, B.n_final,
-        B.maxv, B.step, B.persistent_groups, B.code, B.nkey, B.dcount, B.count_next, B.err);
+        B.maxv, B.step, B.persistent_groups, B.members, B.dseg, B.count_next, B.err,
+        prev_binning(B), B.pstart, B.move ? B.pf_alt : B.pf, B.move ? B.pi_alt : nullptr, n, B.nw);
+    if (B.move) take_moved(B);
   }
   {
     TimerScope ts(tm, "k_grid_op", st);
@@ -1482,8 +1452,14 @@ void launch_transfer(const Params* P, const int* slab, SubstepBuffers& B, int ra
   {
     TimerScope ts(tm, "k_p2g", st);
     auto kern = B.quant ? k_p2g<D, 0, true> : k_p2g<D, 0, false>;
+    if (order_in_transfer(B))
+      kern = B.quant ? k_p2g<D, 0, true, kOrderLists> : k_p2g<D, 0, false, kOrderLists>;
+    if (B.move) kern = B.quant ? k_p2g<D, 0, true, kOrderMove> : k_p2g<D, 0, false, kOrderMove>;
     kern<<<clamp_groups(chunk_bound, G), kThreads, 0, st>>>(
-        P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.tiles, nullptr, B.pf_out);
+        P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.tiles, nullptr,
+        B.move ? B.pf_alt : B.pf_out, prev_binning(B), B.pstart, B.move ? B.pi_alt : nullptr, n,
+        B.nw, B.err);
+    if (B.move) take_moved(B);
   }
   {
     TimerScope ts(tm, "k_grid_op", st);
@@ -1509,7 +1485,7 @@ void launch_g2p(const Params* P, const int* slab, SubstepBuffers& B, int s_index
                                  : (B.quant ? k_g2p<D, true, 1> : k_g2p<D, false, 1>);
     kern<<<clamp_groups(chunk_bound, G), kThreads, 0, st>>>(
         P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.grid,
-        B.maxv, B.step, B.persistent_groups, B.code, B.nkey, B.dcount, B.count_next, B.err,
+        B.maxv, B.step, B.persistent_groups, B.members, B.dseg, B.count_next, B.err,
         B.pf_out, n);
   }
   std::swap(B.count, B.count_next);
@@ -1556,9 +1532,9 @@ void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const f
     }
     {
       TimerScope ts(tm, "k_g2p_adj_scatter", st);
-      k_p2g<D, 1><<<groups, kThreads, 0, st>>>(P, slab, const_cast<float*>(pf_in), B.pi, B.cap,
-                                               B.perm, B.chunks, B.totals, B.tiles, gout,
-                                               nullptr);
+      k_p2g<D, 1><<<groups, kThreads, 0, st>>>(P, slab, pf_in, B.pi, B.cap, B.perm, B.chunks,
+                                               B.totals, B.tiles, gout, nullptr, PrevBinning{},
+                                               nullptr, nullptr, n, 0, nullptr);
     }
     {
       TimerScope ts(tm, "k_grid_op_adj", st);
@@ -1583,15 +1559,11 @@ void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const f
   k_sum_partials<<<1, kThreads, 0, st>>>(nu_part, pgroups, gnu);
 }
 
-template <int D>
-void launch_reorder(SubstepBuffers& B, float* pf_alt, int* pi_alt, hipStream_t st, Timer* tm) {
-  TimerScope ts(tm, "k_reorder", st);
-  if (B.quant)
-    k_reorder_words<<<clamp_groups(div_up(B.n, kThreads), 8192), kThreads, 0, st>>>(
-        B.pf, pf_alt, B.pi, pi_alt, B.perm, B.n, B.cap, B.nw, Layout<D>::NI);
-  else
-    k_reorder<D><<<clamp_groups(div_up(B.n, kThreads), 8192), kThreads, 0, st>>>(
-        B.pf, pf_alt, B.pi, pi_alt, B.perm, B.n, B.cap);
+void launch_sorted_keys(const int4* chunks, const int* totals, int n, int total_blocks, int* keys,
+                        hipStream_t st) {
+  if (n > 0)
+    k_sorted_keys<<<clamp_groups(div_up(n, kThreads), 2048), kThreads, 0, st>>>(
+        chunks, totals, n, total_blocks, keys);
 }
 
 template <int D>
@@ -1899,8 +1871,6 @@ template void launch_substep_half<2>(const Params*, const int*, SubstepBuffers&,
                                      hipStream_t, Timer*);
 template void launch_substep_half<3>(const Params*, const int*, SubstepBuffers&, int, int,
                                      hipStream_t, Timer*);
-template void launch_reorder<2>(SubstepBuffers&, float*, int*, hipStream_t, Timer*);
-template void launch_reorder<3>(SubstepBuffers&, float*, int*, hipStream_t, Timer*);
 template void launch_append<2>(SubstepBuffers&, const float*, const float*, const int*, int, int,
                                int, int, hipStream_t);
 template void launch_append<3>(SubstepBuffers&, const float*, const float*, const int*, int, int,

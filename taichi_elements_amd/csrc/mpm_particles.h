@@ -177,6 +177,11 @@ struct Particles<D, false, G> {
 #pragma unroll
       for (int e = 0; e < D; e++) pf[(int64_t)(L::F + a * D + e) * cap + p] = F[a][e];
   }
+  // x, v and C of slot p to slot po of dst, as they are
+  __device__ static void move_xvC(const float* pf, float* dst, int64_t cap, int p, int po) {
+#pragma unroll
+    for (int w = 0; w < L::F; w++) dst[(int64_t)w * cap + po] = pf[(int64_t)w * cap + p];
+  }
   __device__ static float load_Jp(const float* pf, int64_t cap, int p) {
     return pf[(int64_t)L::JP * cap + p];
   }
@@ -261,6 +266,12 @@ struct Particles<D, true, G> {
       }
       u[(int64_t)(K::F + k) * cap + p] = w;
     }
+  }
+  __device__ static void move_xvC(const float* pf, float* dst, int64_t cap, int p, int po) {
+#pragma unroll
+    for (int w = 0; w < K::F; w++) dst[(int64_t)w * cap + po] = pf[(int64_t)w * cap + p];
+#pragma unroll
+    for (int w = K::C; w < K::jp(G); w++) dst[(int64_t)w * cap + po] = pf[(int64_t)w * cap + p];
   }
   __device__ static float load_Jp(const float* pf, int64_t cap, int p) {
     return pf[(int64_t)K::jp(G) * cap + p];

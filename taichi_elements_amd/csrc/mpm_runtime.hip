@@ -134,11 +134,8 @@ struct mpm_solver {
   float4* tiles = nullptr;
   int4* chunks = nullptr;  // 2 x chunk_cap (substep parity)
   int64_t chunk_cap = 0;
-  int* code = nullptr;     // cap
-  int* nkey = nullptr;     // cap
-  int* dcount = nullptr;   // 27 x chunk_cap
-  int* doff = nullptr;     // 27 x chunk_cap
-  int* keys_sorted = nullptr;
+  int* members = nullptr;  // 2 x cap (substep parity)
+  int* dseg = nullptr;     // 2 x 27 x chunk_cap (substep parity)
   // buffers sized by the block window
   int* count = nullptr;
   int* count_next = nullptr;
@@ -153,7 +150,6 @@ struct mpm_solver {
   float4* grid = nullptr;
   int* totals = nullptr;  // 2 x 16 (substep parity)
   int last_parity = 0;
-  bool reordered = false;
   int* err = nullptr;
   unsigned* maxv = nullptr;
   int maxv_cap = 0;
@@ -341,10 +337,8 @@ int free_particle_buffers(mpm_solver* s) {
   dfree(s->lb_status_radix);
   dfree(s->tiles);
   dfree(s->chunks);
-  dfree(s->code);
-  dfree(s->nkey);
-  dfree(s->dcount);
-  dfree(s->doff);
+  dfree(s->members);
+  dfree(s->dseg);
   return MPM_OK;
 }
 
@@ -406,8 +400,7 @@ int grow(mpm_solver* s, int64_t need) {
   TRY(dalloc(&s->lb_status_radix, kRadixBins * ntiles));
   HIP_TRY(hipMemsetAsync(s->lb_status_radix, 0, sizeof(unsigned long long) * kRadixBins * ntiles,
                          s->stream));
-  TRY(dalloc(&s->code, ncap));
-  TRY(dalloc(&s->nkey, ncap));
+  TRY(dalloc(&s->members, 2 * ncap));
   TRY(alloc_chunk_buffers(s));
   HIP_TRY(hipStreamSynchronize(s->stream));
   s->have_perm = false;
@@ -420,16 +413,14 @@ int alloc_chunk_buffers(mpm_solver* s) {
   drop_graphs(s);
   dfree(s->tiles);
   dfree(s->chunks);
-  dfree(s->dcount);
-  dfree(s->doff);
+  dfree(s->dseg);
   const int chunk = s->eff_chunk();
   s->chunk_cap = std::min<int64_t>(s->total_blocks, s->cap) + (s->cap + chunk - 1) / chunk;
   int TN = s->D == 3 ? Geo<3>::kTileNodes : Geo<2>::kTileNodes;
   if (s->g2p2g) TN = s->D == 3 ? (kBlock + 4) * (kBlock + 4) * (kBlock + 4) : (kBlock + 4) * (kBlock + 4);
   TRY(dalloc(&s->tiles, s->chunk_cap * TN));
   TRY(dalloc(&s->chunks, 2 * s->chunk_cap));
-  TRY(dalloc(&s->dcount, 27 * s->chunk_cap));
-  TRY(dalloc(&s->doff, 27 * s->chunk_cap));
+  TRY(dalloc(&s->dseg, 2 * 27 * s->chunk_cap));
   return MPM_OK;
 }
 
@@ -437,6 +428,9 @@ void fill_buffers(mpm_solver* s, SubstepBuffers& B) {
   B.pf = s->pf;
   B.pf_out = s->pf;
   B.pi = s->pi;
+  B.pf_alt = s->pf_alt;
+  B.pi_alt = s->pi_alt;
+  B.move = false;
   B.cap = s->cap;
   B.n = (int)s->n;
   B.keys = s->keys;
@@ -454,20 +448,17 @@ void fill_buffers(mpm_solver* s, SubstepBuffers& B) {
   B.pchunk_begin_prev = s->pchunk_begin + prev * tb;
   B.pchunk_cnt_prev = s->pchunk_cnt + prev * tb;
   B.chunks_prev = s->chunks + prev * s->chunk_cap;
-  B.totals_prev = s->totals + prev * 16;
-  B.code = s->code;
-  B.nkey = s->nkey;
-  B.dcount = s->dcount;
-  B.doff = s->doff;
+  B.members = s->members + cur * s->cap;
+  B.members_prev = s->members + prev * s->cap;
+  B.dseg = s->dseg + cur * 27 * s->chunk_cap;
+  B.dseg_prev = s->dseg + prev * 27 * s->chunk_cap;
   B.tile_prefix = s->tile_prefix;
   B.full_sort = !s->have_perm;
-  B.perm_identity = s->reordered;
   B.g2p2g = s->g2p2g != 0;
   B.quant = s->quant != 0;
   B.nw = s->nf();
   B.grid_in = s->g2p2g ? s->grid : nullptr;
   B.n_final = (int)s->n_final;
-  B.keys_sorted = nullptr;
   B.active = s->active;
   B.lb_status_scan = s->lb_status_scan;
   B.lb_status_radix = s->lb_status_radix;
@@ -495,42 +486,37 @@ void take_buffers(mpm_solver* s, const SubstepBuffers& B) {
   }
   s->perm = B.perm;
   s->perm_alt = B.perm_alt;
-  s->keys_sorted = B.keys_sorted;
   s->last_parity = B.parity;
   s->count = B.count;
   s->count_next = B.count_next;
 }
 
-// The physical reorder of the particle slots when one is due, then B for
-// the next substep.
-void begin_buffers(mpm_solver* s, SubstepBuffers& B, Timer* tm) {
+// B for the next substep; the particles move into the sorted order with it
+// when that is due.
+void begin_buffers(mpm_solver* s, SubstepBuffers& B) {
   fill_buffers(s, B);
   if (s->have_perm && s->reorder_interval > 0 && s->since_reorder >= s->reorder_interval) {
-    if (s->D == 3)
-      launch_reorder<3>(B, s->pf_alt, s->pi_alt, s->stream, tm);
-    else
-      launch_reorder<2>(B, s->pf_alt, s->pi_alt, s->stream, tm);
-    std::swap(s->pf, s->pf_alt);
-    std::swap(s->pi, s->pi_alt);
+    B.move = true;
     s->since_reorder = 0;
-    s->reordered = true;
-    fill_buffers(s, B);
   }
 }
 
 // Host bookkeeping after a substep's kernels were launched.
 void end_buffers(mpm_solver* s, const SubstepBuffers& B) {
   take_buffers(s, B);
+  s->pf = B.pf;
+  s->pf_alt = B.pf_alt;
+  s->pi = B.pi;
+  s->pi_alt = B.pi_alt;
   s->substep_counter++;
   s->have_perm = true;
-  s->reordered = false;
   s->since_reorder++;
 }
 
 // One substep launched kernel by kernel (also what a graph captures).
 int eager_substep(mpm_solver* s, int k, Timer* tm) {
   SubstepBuffers B;
-  begin_buffers(s, B, tm);
+  begin_buffers(s, B);
   if (s->D == 3)
     launch_substep<3>(s->d_params, s->d_slab, B, k, s->debug & 1, s->stream, tm);
   else
@@ -540,13 +526,13 @@ int eager_substep(mpm_solver* s, int k, Timer* tm) {
 }
 
 // The next two substeps can run as one HIP graph: binning by the
-// neighbour sort (not the first substep, not right after positions were
+// direction lists (not the first substep, not right after positions were
 // set), even parity (the pair returns every double-buffered pointer to its
 // place), no physical reorder due, g2p2g past its first substep, no
 // per-kernel timing.
 bool steady_pair(const mpm_solver* s, int left, const Timer* tm) {
   if (!s->use_graphs || tm || left < 2 || s->n == 0) return false;
-  if (!s->have_perm || s->reordered || (s->substep_counter & 1)) return false;
+  if (!s->have_perm || (s->substep_counter & 1)) return false;
   if (s->reorder_interval > 0 && s->since_reorder + 1 >= s->reorder_interval) return false;
   if (s->g2p2g && s->n_final != s->n) return false;
   return true;
@@ -556,7 +542,7 @@ std::vector<intptr_t> graph_key(const mpm_solver* s) {
   return {(intptr_t)s->pf, (intptr_t)s->pi, (intptr_t)s->perm, (intptr_t)s->perm_alt,
           (intptr_t)s->count, (intptr_t)s->count_next, (intptr_t)s->grid,
           (intptr_t)s->grid_alt, (intptr_t)s->maxv, (intptr_t)s->tiles, (intptr_t)s->chunks,
-          (intptr_t)s->keys_alt, (intptr_t)s->dcount, (intptr_t)s->doff, (intptr_t)s->n,
+          (intptr_t)s->members, (intptr_t)s->dseg, (intptr_t)s->n,
           (intptr_t)s->cap, (intptr_t)s->debug, (intptr_t)s->chunk,
           (intptr_t)s->persistent_groups, (intptr_t)s->g2p2g, (intptr_t)s->g2p_waves};
 }
@@ -571,7 +557,6 @@ int run_graph_pair(mpm_solver* s) {
     HIP_TRY(hipGraphLaunch(g.exec, s->stream));
     // bookkeeping of two substeps: every swapped pointer is back in place
     s->last_parity = 1;
-    s->keys_sorted = s->keys_alt;
     s->substep_counter += 2;
     s->since_reorder += 2;
     if (s->g2p2g) s->n_final = s->n;
@@ -733,15 +718,13 @@ void carve_diff_workspace(const mpm_solver* s, Carve& c, SubstepBuffers& B) {
   B.chunks = B.chunks_prev = c.take<int4>(chunk_cap);
   B.active = c.take<int>(tb);
   B.tile_prefix = c.take<int4>(nparts);
-  B.totals = B.totals_prev = c.take<int>(16);
+  B.totals = c.take<int>(16);
   B.ghist = c.take<int>(2 * kMaxRadixPasses * kRadixBins);
   B.lb_status_scan = c.take<unsigned long long>(4 * nparts);
   B.lb_status_radix = c.take<unsigned long long>(kRadixBins * rtiles);
   B.lbs = c.take<LBState>(1);
-  B.code = c.take<int>(n);
-  B.nkey = c.take<int>(n);
-  B.dcount = c.take<int>(27 * chunk_cap);
-  B.doff = nullptr;  // steady-state binning only
+  B.members = nullptr;  // steady-state binning only
+  B.dseg = nullptr;
   B.maxv = c.take<unsigned>(s->persistent_groups);
   B.tiles = c.take<float4>(chunk_cap * TN);
   B.grid = c.take<float4>(tb * NPB);
@@ -1250,7 +1233,7 @@ int mpm_substep_begin(mpm_solver* s, float dt) {
     if (s->unbounded) TRY(follow_particles(s, 1));
     Timer* tm = s->timing ? &s->timer : nullptr;
     SubstepBuffers& B = s->half_B;
-    begin_buffers(s, B, tm);
+    begin_buffers(s, B);
     if (s->D == 3)
       launch_substep_half<3>(s->d_params, s->d_slab, B, 0, 0, s->stream, tm);
     else
@@ -1519,7 +1502,12 @@ int mpm_read_binning(mpm_solver* s, int32_t* keys, int32_t* perm, int32_t* slot_
   TRY(check_device_errors(s));
   if (!s->have_perm) return fail(MPM_EINVAL, "no substep has run since the last change");
   if (s->n == 0) return MPM_OK;
-  if (keys) HIP_TRY(hipMemcpy(keys, s->keys_sorted, sizeof(int) * s->n, hipMemcpyDeviceToHost));
+  if (keys) {
+    launch_sorted_keys(s->chunks + s->last_parity * s->chunk_cap, s->totals + s->last_parity * 16,
+                       (int)s->n, s->total_blocks, s->keys, s->stream);
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    HIP_TRY(hipMemcpy(keys, s->keys, sizeof(int) * s->n, hipMemcpyDeviceToHost));
+  }
   if (perm) HIP_TRY(hipMemcpy(perm, s->perm, sizeof(int) * s->n, hipMemcpyDeviceToHost));
   if (slot_to_insertion)
     HIP_TRY(hipMemcpy(slot_to_insertion, s->pi + s->cap, sizeof(int) * s->n,
@@ -1730,7 +1718,7 @@ void diff_buffers(mpm_solver* s, SubstepBuffers& B, float* pf) {
   B.cap = s->diff_n;
   B.n = (int)s->diff_n;
   B.full_sort = true;  // every call is a function of its input state alone
-  B.perm_identity = false;
+  B.members = nullptr;
 }
 
 }  // namespace
@@ -1931,7 +1919,6 @@ int mpm_snapshot(mpm_solver* s, int32_t op) {
                            hipMemcpyDeviceToDevice, s->stream));
   s->n_final = s->snap_n_final;
   s->have_perm = false;  // slots moved: bin from scratch
-  s->reordered = false;
   // the saved slots need not be in block order (a snapshot taken right after
   // particles were added holds insertion order, which makes every transfer's
   // particle loads scattered): reorder at the first opportunity
