@@ -168,7 +168,7 @@ struct mpm_solver {
   std::vector<float> h_aabb;
   // HIP graphs of two steady-state substeps, keyed by the buffer pointers
   // and sizes their kernels were captured with
-  bool use_graphs = true;
+  bool use_graphs = false;  // mpm_set_graphs: eager launches keep ahead of the kernels
   struct GraphEntry {
     std::vector<intptr_t> key;
     hipGraphExec_t exec;
