@@ -438,9 +438,8 @@ __global__ __launch_bounds__(kThreads) void k_p2g_adj(
   constexpr int NPB = Geo<D>::kNodesPerBlock, TN = Geo<D>::kTileNodes;
   __shared__ float4 vt[TN];
   __shared__ float4 gt[TN];
-  const int nchunks = totals[kTotChunks];
-  for (int c = blockIdx.x; c < nchunks; c += gridDim.x) {
-    const int4 ck = chunks[c];
+  for (XcdItems it(totals[kTotChunks], kSpreadChunks); it.valid(); it.next()) {
+    const int4 ck = chunks[it.c];
     int lb[3], lbl[3];
     decode_local<D>(ck.x, scenes[0], lb);
     const Params& P = scenes[scene_of<D>(lb, slab)];

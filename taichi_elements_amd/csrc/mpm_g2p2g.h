@@ -60,8 +60,8 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   float vmax = 0.0f;
-  const int nchunks = totals[kTotChunks];
-  for (int c = blockIdx.x; c < nchunks; c += gridDim.x) {
+  for (XcdItems it(totals[kTotChunks], kSpreadChunks); it.valid(); it.next()) {
+    const int c = it.c;
     const int4 ck = chunks[c];
     const int nc = ck.z - ck.y;
     int lb[3], lbl[3], b[3] = {0, 0, 0};
@@ -450,48 +450,44 @@ __global__ __launch_bounds__(kThreads) void k_grid_op_g2p2g(
   constexpr int E8 = G2P2GGeo<D>::kEdge, TN8 = G2P2GGeo<D>::kNodes;
   // The tile of block q = b - d starts one node below q, so this node sits at
   // tile coordinate l + 1 + 4 d, inside the tile for d = 0 and, per axis,
-  // for d = -1 (l = 3) or d = +1 (l < 3): 2^D source blocks, summed by
-  // node_lanes lanes per node and combined in a fixed tree as in k_grid_op.
+  // for d = -1 (l = 3) or d = +1 (l < 3): 2^D source blocks.  A lane per
+  // node, as in k_grid_op.
   constexpr int SRC = D == 3 ? 8 : 4;
-  const int64_t nodes = (int64_t)totals[kTotActive] * NPB;
-  const int lanes = node_lanes(nodes, SRC);
-  for (int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x; t < nodes * lanes;
-       t += (int64_t)gridDim.x * kThreads) {
-    const int64_t nt = t / lanes;
-    const int sub = (int)(t % lanes);
-    const int blk = (int)(nt / NPB), node = (int)(nt % NPB);
+  constexpr int BPW = 64 / NPB;  // blocks per wave
+  const int nact = totals[kTotActive];
+  const int lane = threadIdx.x & 63, node = lane % NPB;
+  const int l[3] = {node & 3, (node >> 2) & 3, node >> 4};
+  constexpr int BPG = kThreads / NPB;  // blocks per workgroup
+  for (XcdItems it((nact + BPG - 1) / BPG, INT32_MAX); it.valid(); it.next()) {
+    const int w = it.c * (kThreads / 64) + (threadIdx.x >> 6);
+    const int blk = D == 3 ? __builtin_amdgcn_readfirstlane(w) : w * BPW + lane / NPB;
+    if (blk >= nact) continue;
     const int bid = active[blk];
     int lb[3];
     decode_local<D>(bid, scenes[0], lb);
     const Params& P = scenes[scene_of<D>(lb, slab)];
-    if (P.skip) continue;  // uniform over the group
-    const int l[3] = {node & 3, (node >> 2) & 3, node >> 4};
-    const float4 sum = tree_sum<SRC>(lanes, sub, [&](int src) {
-      float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      int q[3] = {lb[0], lb[1], lb[2]}, tl[3] = {0, 0, 0};
-      bool ok = true;
+    if (P.skip) continue;
+    int first[SRC], left[SRC], tn[SRC];
 #pragma unroll
-      for (int a = 0; a < D; a++) {
+    for (int src = 0; src < SRC; src++) {
+      int q[3] = {lb[0], lb[1], lb[2]};
+      bool in = true;
+      tn[src] = 0;
+#pragma unroll
+      for (int a = D - 1; a >= 0; a--) {
         const int d = ((src >> a) & 1) ? (l[a] == kBlock - 1 ? -1 : 1) : 0;
-        tl[a] = l[a] + 1 + kBlock * d;
+        tn[src] = tn[src] * E8 + l[a] + 1 + kBlock * d;
         q[a] = lb[a] - d;
-        ok &= (q[a] >= 0) & (q[a] < scenes[0].bn[a]);
+        in &= (q[a] >= 0) & (q[a] < scenes[0].bn[a]);
       }
-      if (ok) {
+      first[src] = left[src] = 0;
+      if (in) {
         const int nb = encode_local<D>(q, P);
-        const int c0 = pchunk_begin[nb], cn = pchunk_cnt[nb];
-        const int tn = D == 3 ? tl[0] + E8 * (tl[1] + E8 * tl[2]) : tl[0] + E8 * tl[1];
-        for (int k = c0; k < c0 + cn; k++) {
-          const float4 tv = tiles[(int64_t)k * TN8 + tn];
-          acc.x += tv.x;
-          acc.y += tv.y;
-          if (D == 3) acc.z += tv.z;
-          acc.w += tv.w;
-        }
+        first[src] = pchunk_begin[nb];
+        left[src] = pchunk_cnt[nb];
       }
-      return acc;
-    });
-    if (sub != 0) continue;
+    }
+    const float4 sum = sum_tiles<SRC, TN8, D>(tiles, first, left, tn);
     float m = sum.w, p[3] = {sum.x, sum.y, sum.z};
     if (node_has_mass(m)) {  // mpm_solver.py:591-593
       const float inv = 1.0f / m;

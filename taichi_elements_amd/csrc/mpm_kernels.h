@@ -12,6 +12,10 @@ namespace mpm {
 constexpr int kThreads = 256;
 constexpr int kBatch = kThreads;  // particles a transfer workgroup holds at a time
 constexpr int kChunkMax = 1024;  // particles per transfer work item (max), kBatch at a time
+// Up to this many particles a scene has about one chunk per workgroup (unless
+// they are spread very thinly): work that each chunk adds to a transfer then
+// costs its latency once, less than a kernel of its own.
+constexpr int kOneRound = 160 * 1024;
 constexpr int kScanItems = 2;                       // per thread in the block scan
 constexpr int kScanTile = kThreads * kScanItems;    // 512 blocks per workgroup
 constexpr int kRadixItems = 16;
@@ -61,6 +65,7 @@ struct SubstepBuffers {
   LBState* lbs;
   float4* tiles;    // p2g per-chunk node tiles (momentum xyz, mass)
   float4* grid;     // dense block-major grid [total_blocks][nodes] of (v, mass)
+  bool grid_in_g2p; // g2p sums the tiles itself; the grid is not written
   float4* raw_out;  // if set, the grid operator also stores the raw p2g sums here
   int* err;         // error bits
   unsigned* maxv;   // per-substep, per-g2p-workgroup max |v| (float bits)

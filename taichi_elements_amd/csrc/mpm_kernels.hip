@@ -564,8 +564,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  const int nchunks = totals[kTotChunks];
-  for (int c = blockIdx.x; c < nchunks; c += gridDim.x) {
+  for (XcdItems it(totals[kTotChunks], kSpreadChunks); it.valid(); it.next()) {
+    const int c = it.c;
     const int4 ck = chunks[c];
     int lbc[3], b[3];
     decode_local<D>(ck.x, scenes[0], lbc);
@@ -789,6 +789,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 // ---------------------------------------------------------------------------
 // grid operator (mpm_solver.py:586-692)
 // ---------------------------------------------------------------------------
+// Velocity of the node with index I from its p2g sums (momentum, mass):
+// normalisation, gravity (mpm_solver.py:591-595) and the post-processes.
+template <int D>
+__device__ __forceinline__ float4 node_velocity(const Params& P, const int I[3], float4 sum) {
+  float p[3] = {sum.x, sum.y, sum.z};
+  if (node_has_mass(sum.w)) {
+    const float inv = 1.0f / sum.w;
+#pragma unroll
+    for (int a = 0; a < D; a++) p[a] = inv * p[a];
+#pragma unroll
+    for (int a = 0; a < D; a++) p[a] += P.dt * P.gravity[a];
+  }
+  apply_post<D>(P, I, p);
+  return make_float4(p[0], p[1], D == 3 ? p[2] : 0.0f, sum.w);
+}
+
 // Bounding-box walls zero the outward velocity components near the domain
 // faces (mpm_solver.py:600-616); bit a of the result is set when component a
 // of v (before the walls) passes unchanged.
@@ -810,53 +826,52 @@ __global__ __launch_bounds__(kThreads) void k_grid_op(const Params* __restrict__
                                                       float4* __restrict__ gbar,
                                                       float4* __restrict__ raw_out) {
   constexpr int NPB = Geo<D>::kNodesPerBlock, TN = Geo<D>::kTileNodes;
-  // Lanes per node (node_lanes), each summing the tiles of some of the SRC
-  // particle blocks b - d (d in {0,1}^D) whose tiles reach the node; the
-  // partial sums combine in a fixed tree (tree_sum), so the result does not
-  // depend on the lane count.  A sparse window gets a lane per source block:
-  // this latency-bound kernel then has SRC times the loads in flight.
+  // A lane per node, so in 3D a wave per block: its source blocks, chunk
+  // ranges and scene are the same for every lane, and a load instruction
+  // reads the 16-byte nodes of one tile's rows.  Bound by the chain of
+  // dependent loads (block, chunk ranges, tiles) at 1M particles, by the
+  // tiles' bytes at 16M.  Eight lanes per node, one per source block, spread
+  // every load over eight tiles: 1M 20.0 -> 14.0 us, 16M 211 -> 108 us,
+  // use_g2p2g 300k 17.8 -> 12.1 us.
   constexpr int SRC = D == 3 ? 8 : 4;
-  const int64_t nodes = (int64_t)totals[kTotActive] * NPB;
-  const int lanes = node_lanes(nodes, SRC);
-  for (int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x; t < nodes * lanes;
-       t += (int64_t)gridDim.x * kThreads) {
-    // groups of `lanes` lanes are aligned and enter or leave the loop together
-    const int64_t nt = t / lanes;
-    const int sub = (int)(t % lanes);
-    const int blk = (int)(nt / NPB), node = (int)(nt % NPB);
+  constexpr int BPW = 64 / NPB;  // blocks per wave
+  const int nact = totals[kTotActive];
+  const int lane = threadIdx.x & 63, node = lane % NPB;
+  const int l[3] = {node & 3, (node >> 2) & 3, node >> 4};
+  constexpr int BPG = kThreads / NPB;  // blocks per workgroup
+  for (XcdItems it((nact + BPG - 1) / BPG, INT32_MAX); it.valid(); it.next()) {
+    const int w = it.c * (kThreads / 64) + (threadIdx.x >> 6);
+    const int blk = D == 3 ? __builtin_amdgcn_readfirstlane(w) : w * BPW + lane / NPB;
+    if (blk >= nact) continue;
     const int bid = active[blk];
     int lb[3];
     decode_local<D>(bid, scenes[0], lb);
     const Params& P = scenes[scene_of<D>(lb, slab)];
-    if (P.skip) continue;  // uniform over the group: one node, one scene
-    const int l[3] = {node & 3, (node >> 2) & 3, node >> 4};
-    const float4 sum = tree_sum<SRC>(lanes, sub, [&](int src) {
-      float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      const int d[3] = {src & 1, (src >> 1) & 1, src >> 2};
-      int q[3], tl[3];
-      bool ok = true;
+    if (P.skip) continue;
+    int first[SRC], left[SRC], tn[SRC];
 #pragma unroll
-      for (int a = 0; a < D; a++) {
-        tl[a] = l[a] + kBlock * d[a];
+    for (int src = 0; src < SRC; src++) {  // particle block b - d, d in {0, 1}^D
+      const int d[3] = {src & 1, (src >> 1) & 1, src >> 2};
+      int q[3];
+      bool in = true, reach = true;
+      tn[src] = 0;
+#pragma unroll
+      for (int a = D - 1; a >= 0; a--) {
         q[a] = lb[a] - d[a];
-        ok &= (tl[a] < kTile) & (q[a] >= 0);
+        in &= q[a] >= 0;
+        reach &= l[a] + kBlock * d[a] < kTile;
+        tn[src] = tn[src] * kTile + l[a] + kBlock * d[a];
       }
-      if (ok) {
+      first[src] = left[src] = 0;
+      if (in) {
         const int nb = encode_local<D>(q, P);
-        const int c0 = pchunk_begin[nb], cn = pchunk_cnt[nb];
-        const int tn = D == 3 ? tl[0] + kTile * (tl[1] + kTile * tl[2]) : tl[0] + kTile * tl[1];
-        for (int k = c0; k < c0 + cn; k++) {
-          const float4 tv = tiles[(int64_t)k * TN + tn];
-          acc.x += tv.x;
-          acc.y += tv.y;
-          if (D == 3) acc.z += tv.z;
-          acc.w += tv.w;
-        }
+        first[src] = pchunk_begin[nb];
+        left[src] = pchunk_cnt[nb];
       }
-      return acc;
-    });
-    if (sub != 0) continue;
-    float m = sum.w, p[3] = {sum.x, sum.y, sum.z};
+      if (!reach) left[src] = 0;
+    }
+    const float4 sum = sum_tiles<SRC, TN, D>(tiles, first, left, tn);
+    const float p[3] = {sum.x, sum.y, sum.z};
     if (MODE == 0 && raw_out) raw_out[(int64_t)bid * NPB + node] = sum;
     if (MODE == 1) {
       const float4 f = grid[(int64_t)bid * NPB + node];
@@ -882,21 +897,15 @@ __global__ __launch_bounds__(kThreads) void k_grid_op(const Params* __restrict__
       gbar[(int64_t)bid * NPB + node] = make_float4(pb[0], pb[1], D == 3 ? pb[2] : 0.0f, mb);
       continue;
     }
+    float4 out = make_float4(p[0], p[1], D == 3 ? p[2] : 0.0f, sum.w);
     if (!raw) {
-      if (node_has_mass(m)) {  // mpm_solver.py:591-593
-        const float inv = 1.0f / m;
-#pragma unroll
-        for (int a = 0; a < D; a++) p[a] = inv * p[a];
-#pragma unroll
-        for (int a = 0; a < D; a++) p[a] += P.dt * P.gravity[a];
-      }
       int I[3], lbl[3];
       to_local<D>(lb, P, lbl);
 #pragma unroll
       for (int a = 0; a < D; a++) I[a] = (lbl[a] + P.blo[a]) * kBlock + l[a];
-      apply_post<D>(P, I, p);
+      out = node_velocity<D>(P, I, sum);
     }
-    grid[(int64_t)bid * NPB + node] = make_float4(p[0], p[1], D == 3 ? p[2] : 0.0f, m);
+    grid[(int64_t)bid * NPB + node] = out;
   }
 }
 
@@ -906,7 +915,14 @@ __global__ __launch_bounds__(kThreads) void k_grid_op(const Params* __restrict__
 // W: minimum waves per SIMD the register allocation must allow (1: no
 // constraint, 5 waves at its register count; 6: at most 80 registers, more
 // grid-tile gathers in flight where each block holds few particles).
-template <int D, bool Q = false, int W = 1>
+// TILES: the grid operator runs in here.  The workgroup sums the p2g tiles
+// that reach its (4+2)^d nodes itself, in k_grid_op's order (bitwise the same
+// velocities), instead of reading them from the grid: every node is summed by
+// up to 2^d workgroups, out of L2, and a kernel and the grid's round trip
+// through memory go.  Taken in 2D up to kOneRound particles: 20k, g2p 4.8 +
+// grid operator 4.3 -> 6.6 us; at 400k in 2D 22.6 -> 24.6, in 3D 15.4 -> 14.4
+// (50k, no gain over the present grid operator), 51 -> 84 us (1M).
+template <int D, bool Q = false, int W = 1, bool TILES = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) void k_g2p(const Params* __restrict__ scenes,
                                                   const int* __restrict__ slab,
                                                   float* __restrict__ pf,
@@ -921,7 +937,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
                                                   int* __restrict__ dseg,
                                                   int* __restrict__ count_next,
                                                   int* __restrict__ err,
-                                                  float* __restrict__ pf_out, int n) {
+                                                  float* __restrict__ pf_out, int n,
+                                                  const int* __restrict__ pchunk_begin,
+                                                  const int* __restrict__ pchunk_cnt,
+                                                  const float4* __restrict__ tiles) {
   using L = Layout<D>;
   constexpr int NPB = Geo<D>::kNodesPerBlock, TN = Geo<D>::kTileNodes;
   // grid velocity tile as three float arrays: the per-particle gathers hit
@@ -932,13 +951,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
   __shared__ int dwcnt[kThreads / 64][32];
   __shared__ int dbase[32];  // particles per direction in the chunk's earlier batches
   __shared__ int dstart[32];
+  __shared__ int2 nbr[TILES ? 27 : 1];  // chunk ranges of the neighbouring blocks
   // the particles of the earlier batches: direction | rank << 8, slot
   __shared__ int lcode[kChunkMax - kBatch], lid[kChunkMax - kBatch];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   float vmax = 0.0f;
-  const int nchunks = totals[kTotChunks];
-  for (int c = blockIdx.x; c < nchunks; c += gridDim.x) {
+  for (XcdItems it(totals[kTotChunks], kSpreadChunks); it.valid(); it.next()) {
+    const int c = it.c;
     const int4 ck = chunks[c];
     int lb[3], lbl[3];
     decode_local<D>(ck.x, scenes[0], lb);
@@ -948,21 +968,70 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
     // grid was not rebuilt and is not read
     const bool skip = P.skip != 0;
     if (threadIdx.x < 32) dbase[threadIdx.x] = 0;
-    for (int i = skip ? TN : threadIdx.x; i < TN; i += kThreads) {
-      const int tl[3] = {i % kTile, (i / kTile) % kTile, i / (kTile * kTile)};
-      int q[3], ln[3];
+    if (TILES) {
+      constexpr int NB = D == 3 ? 27 : 9, SRC = D == 3 ? 8 : 4;
+      if (threadIdx.x < NB) {  // chunk ranges of the blocks lb + {-1, 0, 1}^d
+        const int q[3] = {lb[0] - 1 + (int)threadIdx.x % 3, lb[1] - 1 + ((int)threadIdx.x / 3) % 3,
+                          D == 3 ? lb[2] - 1 + (int)threadIdx.x / 9 : 0};
+        bool ok = true;  // below the window there is no block; above it is lb + 1 at most
 #pragma unroll
-      for (int a = 0; a < D; a++) {
-        const int hi = tl[a] >= kBlock;
-        q[a] = lb[a] + hi;
-        ln[a] = tl[a] - kBlock * hi;
+        for (int a = 0; a < D; a++) ok &= q[a] >= 0;
+        int2 r = make_int2(0, 0);
+        if (ok) {
+          const int nb = encode_local<D>(q, P);
+          r = make_int2(pchunk_begin[nb], pchunk_cnt[nb]);
+        }
+        nbr[threadIdx.x] = r;
       }
-      const int gb = encode_local<D>(q, P);
-      const int node = D == 3 ? ln[0] + 4 * (ln[1] + 4 * ln[2]) : ln[0] + 4 * ln[1];
-      const float4 g = grid[(int64_t)gb * NPB + node];
-      tile_x[i] = g.x;
-      tile_y[i] = g.y;
-      tile_z[i] = g.z;
+      lds_barrier();
+      for (int i = skip ? TN : threadIdx.x; i < TN; i += kThreads) {
+        const int t[3] = {i % kTile, (i / kTile) % kTile, i / (kTile * kTile)};
+        // source block lb + hi - d, hi the node's own block, d in {0, 1}^d;
+        // its tile holds the node at l + 4 d
+        int first[SRC], left[SRC], tn[SRC];
+#pragma unroll
+        for (int src = 0; src < SRC; src++) {
+          const int d[3] = {src & 1, (src >> 1) & 1, src >> 2};
+          int nb = 0;
+          bool reach = true;
+          tn[src] = 0;
+#pragma unroll
+          for (int a = D - 1; a >= 0; a--) {
+            const int x = (t[a] & (kBlock - 1)) + kBlock * d[a];
+            reach &= x < kTile;
+            tn[src] = tn[src] * kTile + x;
+            nb = nb * 3 + (t[a] >= kBlock ? 1 : 0) - d[a] + 1;
+          }
+          const int2 r = nbr[nb];
+          first[src] = r.x;
+          left[src] = reach ? r.y : 0;
+        }
+        const float4 sum = sum_tiles<SRC, TN, D>(tiles, first, left, tn);
+        int I[3];
+#pragma unroll
+        for (int a = 0; a < D; a++) I[a] = (lbl[a] + P.blo[a]) * kBlock + t[a];
+        const float4 g = node_velocity<D>(P, I, sum);
+        tile_x[i] = g.x;
+        tile_y[i] = g.y;
+        tile_z[i] = g.z;
+      }
+    } else {
+      for (int i = skip ? TN : threadIdx.x; i < TN; i += kThreads) {
+        const int tl[3] = {i % kTile, (i / kTile) % kTile, i / (kTile * kTile)};
+        int q[3], ln[3];
+#pragma unroll
+        for (int a = 0; a < D; a++) {
+          const int hi = tl[a] >= kBlock;
+          q[a] = lb[a] + hi;
+          ln[a] = tl[a] - kBlock * hi;
+        }
+        const int gb = encode_local<D>(q, P);
+        const int node = D == 3 ? ln[0] + 4 * (ln[1] + 4 * ln[2]) : ln[0] + 4 * ln[1];
+        const float4 g = grid[(int64_t)gb * NPB + node];
+        tile_x[i] = g.x;
+        tile_y[i] = g.y;
+        tile_z[i] = g.z;
+      }
     }
     lds_barrier();
     int b[3];
@@ -1295,13 +1364,20 @@ __global__ __launch_bounds__(kThreads) void k_fill_u32(unsigned* __restrict__ p,
 // launchers
 // ---------------------------------------------------------------------------
 static inline int div_up(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
-// Workgroups of the grid operators (lanes per node x source block): enough
-// that a large window needs few grid-stride iterations per lane, while the
-// idle workgroups of a sparse window stay cheap.
-constexpr int kGridOpGroups = 16384;
-
 static inline int clamp_groups(int64_t g, int cap) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(g, cap));
+}
+// the same, a multiple of the eight XCDs (XcdItems)
+static inline int xcd_groups(int64_t g, int cap) {
+  return (int)std::min<int64_t>((std::max<int64_t>(g, 1) + 7) & ~7, cap & ~7);
+}
+
+// Workgroups of the grid operators: a lane per node of the active blocks (at
+// most the window's, and 2^D per particle), as many as are resident at once.
+template <int D>
+static int grid_op_groups(const SubstepBuffers& B) {
+  const int64_t blocks = std::min<int64_t>(B.total_blocks, (int64_t)B.n * (D == 3 ? 8 : 4));
+  return xcd_groups(div_up(blocks * Geo<D>::kNodesPerBlock, kThreads), 2048);
 }
 
 struct TimerScope {
@@ -1327,12 +1403,10 @@ static PrevBinning prev_binning(const SubstepBuffers& B) {
 }
 
 // Whether the transfer walks the direction lists itself (mpm_binning.h says
-// what each way costs): with about one chunk per workgroup, which a scene of
-// this many particles has unless they are spread very thinly.  A substep
-// that moves the particles takes the given order.
-constexpr int kListsInTransfer = 160 * 1024;
+// what each way costs).  A substep that moves the particles takes the given
+// order.
 static bool order_in_transfer(const SubstepBuffers& B) {
-  return !B.full_sort && !B.move && B.n <= kListsInTransfer;
+  return !B.full_sort && !B.move && B.n <= kOneRound;
 }
 
 // binning of one substep: block counts, the dense-window scan (chunks,
@@ -1425,7 +1499,7 @@ static void launch_g2p2g(const Params* P, const int* slab, SubstepBuffers& B, in
     if (order_in_transfer(B))
       kern = B.quant ? k_g2p2g<D, true, kOrderLists> : k_g2p2g<D, false, kOrderLists>;
     if (B.move) kern = B.quant ? k_g2p2g<D, true, kOrderMove> : k_g2p2g<D, false, kOrderMove>;
-    kern<<<clamp_groups(chunk_bound, G), kThreads, 0, st>>>(
+    kern<<<xcd_groups(chunk_bound, G), kThreads, 0, st>>>(
         P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.grid_in, B.tiles, B.n_final,
         B.maxv, B.step, B.persistent_groups, B.members, B.dseg, B.count_next, B.err,
         prev_binning(B), B.pstart, B.move ? B.pf_alt : B.pf, B.move ? B.pi_alt : nullptr, n, B.nw);
@@ -1433,9 +1507,7 @@ static void launch_g2p2g(const Params* P, const int* slab, SubstepBuffers& B, in
   }
   {
     TimerScope ts(tm, "k_grid_op", st);
-    const int64_t node_bound = (int64_t)B.total_blocks * Geo<D>::kNodesPerBlock;
-    k_grid_op_g2p2g<D><<<clamp_groups(div_up(node_bound * (D == 3 ? 8 : 4), kThreads), kGridOpGroups), kThreads,
-                         0, st>>>(
+    k_grid_op_g2p2g<D><<<grid_op_groups<D>(B), kThreads, 0, st>>>(
         P, slab, B.active, B.totals, B.pchunk_begin, B.pchunk_cnt, B.tiles, B.grid);
   }
   std::swap(B.count, B.count_next);
@@ -1455,16 +1527,15 @@ void launch_transfer(const Params* P, const int* slab, SubstepBuffers& B, int ra
     if (order_in_transfer(B))
       kern = B.quant ? k_p2g<D, 0, true, kOrderLists> : k_p2g<D, 0, false, kOrderLists>;
     if (B.move) kern = B.quant ? k_p2g<D, 0, true, kOrderMove> : k_p2g<D, 0, false, kOrderMove>;
-    kern<<<clamp_groups(chunk_bound, G), kThreads, 0, st>>>(
+    kern<<<xcd_groups(chunk_bound, G), kThreads, 0, st>>>(
         P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.tiles, nullptr,
         B.move ? B.pf_alt : B.pf_out, prev_binning(B), B.pstart, B.move ? B.pi_alt : nullptr, n,
         B.nw, B.err);
     if (B.move) take_moved(B);
   }
-  {
+  if (!B.grid_in_g2p) {
     TimerScope ts(tm, "k_grid_op", st);
-    const int64_t node_bound = (int64_t)B.total_blocks * Geo<D>::kNodesPerBlock;
-    k_grid_op<D, 0><<<clamp_groups(div_up(node_bound * (D == 3 ? 8 : 4), kThreads), kGridOpGroups), kThreads, 0, st>>>(
+    k_grid_op<D, 0><<<grid_op_groups<D>(B), kThreads, 0, st>>>(
         P, slab, B.active, B.totals, B.pchunk_begin, B.pchunk_cnt, B.tiles, B.grid, raw, nullptr,
         B.raw_out);
   }
@@ -1483,10 +1554,13 @@ void launch_g2p(const Params* P, const int* slab, SubstepBuffers& B, int s_index
     TimerScope ts(tm, "k_g2p", st);
     auto kern = B.g2p_waves >= 6 ? (B.quant ? k_g2p<D, true, 6> : k_g2p<D, false, 6>)
                                  : (B.quant ? k_g2p<D, true, 1> : k_g2p<D, false, 1>);
-    kern<<<clamp_groups(chunk_bound, G), kThreads, 0, st>>>(
+    if (B.grid_in_g2p)
+      kern = B.g2p_waves >= 6 ? (B.quant ? k_g2p<D, true, 6, true> : k_g2p<D, false, 6, true>)
+                              : (B.quant ? k_g2p<D, true, 1, true> : k_g2p<D, false, 1, true>);
+    kern<<<xcd_groups(chunk_bound, G), kThreads, 0, st>>>(
         P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.grid,
         B.maxv, B.step, B.persistent_groups, B.members, B.dseg, B.count_next, B.err,
-        B.pf_out, n);
+        B.pf_out, n, B.pchunk_begin, B.pchunk_cnt, B.tiles);
   }
   std::swap(B.count, B.count_next);
 }
@@ -1522,7 +1596,7 @@ void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const f
   const int n = B.n;
   const int G = B.persistent_groups;
   const int chunk_bound = n > 0 ? std::min(B.total_blocks, n) + div_up(n, B.chunk) : 1;
-  const int groups = clamp_groups(chunk_bound, G);
+  const int groups = xcd_groups(chunk_bound, G);
   const int pgroups = clamp_groups(div_up(n, kThreads), G);
   if (n > 0) {
     {
@@ -1538,8 +1612,7 @@ void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const f
     }
     {
       TimerScope ts(tm, "k_grid_op_adj", st);
-      const int64_t node_bound = (int64_t)B.total_blocks * Geo<D>::kNodesPerBlock;
-      k_grid_op<D, 1><<<clamp_groups(div_up(node_bound * (D == 3 ? 8 : 4), kThreads), kGridOpGroups), kThreads, 0, st>>>(
+      k_grid_op<D, 1><<<grid_op_groups<D>(B), kThreads, 0, st>>>(
           P, slab, B.active, B.totals, B.pchunk_begin, B.pchunk_cnt, B.tiles, B.grid, 0, gbar,
           nullptr);
     }

@@ -424,6 +424,9 @@ int alloc_chunk_buffers(mpm_solver* s) {
   return MPM_OK;
 }
 
+// The kernels look a block's scene up in the slab table; one scene needs none.
+const int* slab_table(const mpm_solver* s) { return s->scenes.size() > 1 ? s->d_slab : nullptr; }
+
 void fill_buffers(mpm_solver* s, SubstepBuffers& B) {
   B.pf = s->pf;
   B.pf_out = s->pf;
@@ -468,6 +471,7 @@ void fill_buffers(mpm_solver* s, SubstepBuffers& B) {
   B.tiles = s->tiles;
   B.grid = s->g2p2g ? s->grid_alt : s->grid;
   B.raw_out = nullptr;
+  B.grid_in_g2p = false;
   B.err = s->err;
   B.maxv = s->maxv;
   B.step = s->d_step;
@@ -513,14 +517,18 @@ void end_buffers(mpm_solver* s, const SubstepBuffers& B) {
   s->since_reorder++;
 }
 
-// One substep launched kernel by kernel (also what a graph captures).
-int eager_substep(mpm_solver* s, int k, Timer* tm) {
+// One substep launched kernel by kernel (also what a graph captures).  last:
+// the last substep of a call, which leaves the grid for its readers
+// (mpm_read_grid, mpm_max_grid_velocity); the others need no grid in memory
+// and run the grid operator inside g2p where that is faster (k_g2p's TILES).
+int eager_substep(mpm_solver* s, int k, bool last, Timer* tm) {
   SubstepBuffers B;
   begin_buffers(s, B);
+  B.grid_in_g2p = !last && !s->g2p2g && !(s->debug & 1) && s->n <= kOneRound && s->D == 2;
   if (s->D == 3)
-    launch_substep<3>(s->d_params, s->d_slab, B, k, s->debug & 1, s->stream, tm);
+    launch_substep<3>(s->d_params, slab_table(s), B, k, s->debug & 1, s->stream, tm);
   else
-    launch_substep<2>(s->d_params, s->d_slab, B, k, s->debug & 1, s->stream, tm);
+    launch_substep<2>(s->d_params, slab_table(s), B, k, s->debug & 1, s->stream, tm);
   end_buffers(s, B);
   return MPM_OK;
 }
@@ -568,8 +576,8 @@ int run_graph_pair(mpm_solver* s) {
   }
   hipGraph_t graph = nullptr;
   HIP_TRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-  int r = eager_substep(s, 0, nullptr);
-  if (r == MPM_OK) r = eager_substep(s, 1, nullptr);
+  int r = eager_substep(s, 0, false, nullptr);
+  if (r == MPM_OK) r = eager_substep(s, 1, false, nullptr);
   hipError_t e = hipStreamEndCapture(s->stream, &graph);
   if (r != MPM_OK) {
     if (graph) hipGraphDestroy(graph);
@@ -1199,12 +1207,13 @@ static int substeps_impl(mpm_solver* s, int32_t nsub, const float* dts, bool bat
       TRY(follow_particles(s, next_check - k));
     }
     const int left = s->unbounded ? next_check - k : nsub - k;
-    if (steady_pair(s, left, tm)) {
+    // (the call's last substep stays out of the graphs: it writes the grid)
+    if (steady_pair(s, std::min(left, nsub - 1 - k), tm)) {
       TRY(run_graph_pair(s));
       k += 2;
       continue;
     }
-    TRY(eager_substep(s, k, tm));
+    TRY(eager_substep(s, k, k == nsub - 1, tm));
     k++;
   }
   HIP_TRY(hipGetLastError());
@@ -1235,9 +1244,9 @@ int mpm_substep_begin(mpm_solver* s, float dt) {
     SubstepBuffers& B = s->half_B;
     begin_buffers(s, B);
     if (s->D == 3)
-      launch_substep_half<3>(s->d_params, s->d_slab, B, 0, 0, s->stream, tm);
+      launch_substep_half<3>(s->d_params, slab_table(s), B, 0, 0, s->stream, tm);
     else
-      launch_substep_half<2>(s->d_params, s->d_slab, B, 0, 0, s->stream, tm);
+      launch_substep_half<2>(s->d_params, slab_table(s), B, 0, 0, s->stream, tm);
     HIP_TRY(hipGetLastError());
   }
   s->half_pending = true;
@@ -1305,9 +1314,9 @@ int mpm_substep_end(mpm_solver* s) {
   Timer* tm = s->timing ? &s->timer : nullptr;
   SubstepBuffers& B = s->half_B;
   if (s->D == 3)
-    launch_substep_half<3>(s->d_params, s->d_slab, B, 0, 1, s->stream, tm);
+    launch_substep_half<3>(s->d_params, slab_table(s), B, 0, 1, s->stream, tm);
   else
-    launch_substep_half<2>(s->d_params, s->d_slab, B, 0, 1, s->stream, tm);
+    launch_substep_half<2>(s->d_params, slab_table(s), B, 0, 1, s->stream, tm);
   end_buffers(s, B);
   HIP_TRY(hipGetLastError());
   return MPM_OK;
@@ -1968,9 +1977,9 @@ int mpm_diff_substep(mpm_solver* s, float dt, const float* state_in, float* stat
   B.pf_out = state_out;  // p2g / g2p write the new state out of place
   if (binning) B.raw_out = (float4*)((char*)binning + bin_layout(s).grid);
   if (s->D == 3)
-    launch_substep<3>(s->d_params, s->d_slab, B, 0, 0, st, nullptr);
+    launch_substep<3>(s->d_params, slab_table(s), B, 0, 0, st, nullptr);
   else
-    launch_substep<2>(s->d_params, s->d_slab, B, 0, 0, st, nullptr);
+    launch_substep<2>(s->d_params, slab_table(s), B, 0, 0, st, nullptr);
   if (binning) {
     const BinLayout L = bin_layout(s);
     char* b = (char*)binning;
@@ -2031,9 +2040,9 @@ int mpm_diff_substep_noalloc(mpm_solver* s, float dt, const float* state_in, flo
   launch_fill_u32((unsigned*)B.lb_status_radix, 0u, 2 * kRadixBins * rtiles, st);
   launch_fill_u32((unsigned*)B.lbs, 0u, sizeof(LBState) / 4, st);
   if (s->D == 3)
-    launch_substep<3>(s->d_params, s->d_slab, B, 0, 0, st, nullptr);
+    launch_substep<3>(s->d_params, slab_table(s), B, 0, 0, st, nullptr);
   else
-    launch_substep<2>(s->d_params, s->d_slab, B, 0, 0, st, nullptr);
+    launch_substep<2>(s->d_params, slab_table(s), B, 0, 0, st, nullptr);
   HIP_TRY(hipGetLastError());
   return MPM_OK;
 }
@@ -2066,15 +2075,15 @@ int mpm_diff_substep_backward(mpm_solver* s, float dt, const float* state_in,
     B.grid = (float4*)(b + L.grid);
   } else {
     if (s->D == 3)
-      launch_front<3>(s->d_params, s->d_slab, B, 1, st, nullptr);
+      launch_front<3>(s->d_params, slab_table(s), B, 1, st, nullptr);
     else
-      launch_front<2>(s->d_params, s->d_slab, B, 1, st, nullptr);
+      launch_front<2>(s->d_params, slab_table(s), B, 1, st, nullptr);
   }
   if (s->D == 3)
-    launch_adjoint<3>(s->d_params, s->d_slab, B, state_in, grad_out, grad_in, grad_youngs,
+    launch_adjoint<3>(s->d_params, slab_table(s), B, state_in, grad_out, grad_in, grad_youngs,
                       s->diff_gbar, s->diff_abuf, s->diff_nu_part, grad_nu, st, nullptr);
   else
-    launch_adjoint<2>(s->d_params, s->d_slab, B, state_in, grad_out, grad_in, grad_youngs,
+    launch_adjoint<2>(s->d_params, slab_table(s), B, state_in, grad_out, grad_in, grad_youngs,
                       s->diff_gbar, s->diff_abuf, s->diff_nu_part, grad_nu, st, nullptr);
   if (!binning) {  // the block scan ran: keep the substep-parity bookkeeping
     take_buffers(s, B);
