@@ -38,8 +38,9 @@ __global__ __launch_bounds__(kThreads) void k_g2p2g(
     unsigned* __restrict__ maxv, const int* __restrict__ step, int stride,
     int* members, int* dseg, int* __restrict__ count_next, int* __restrict__ err,
     PrevBinning prev, const int* __restrict__ pstart, float* pf_out, int* __restrict__ pi_out,
-    int n, int nw) {
+    int n, int nw, ScanStatus scan) {
   using L = Layout<D>;
+  scan.clear();
   constexpr int NPB = Geo<D>::kNodesPerBlock, TN = Geo<D>::kTileNodes;
   constexpr int E8 = G2P2GGeo<D>::kEdge, TN8 = G2P2GGeo<D>::kNodes;
   constexpr int CELLS = NPB;

@@ -18,12 +18,13 @@ constexpr int kChunkMax = 1024;  // particles per transfer work item (max), kBat
 constexpr int kOneRound = 160 * 1024;
 constexpr int kScanItems = 2;                       // per thread in the block scan
 constexpr int kScanTile = kThreads * kScanItems;    // 512 blocks per workgroup
+constexpr int kScanTilesOnePass = 512;  // the single-pass scan's most tiles, all resident at once
 constexpr int kRadixItems = 16;
 constexpr int kRadixTile = kThreads * kRadixItems;  // 2048 keys per workgroup
 constexpr int kRadixBins = 256;
 constexpr int kMaxRadixPasses = 3;                  // block keys up to 24 bits
 
-// Ticket / epoch state shared by the single-pass (look-back) scans.
+// Ticket / epoch state of the radix passes' look-back scans.
 struct LBState {
   unsigned long long tile_ctr;
   unsigned long long done_ctr;
@@ -33,6 +34,17 @@ struct LBState {
 
 // Totals written on the device by the block scan (read by persistent kernels).
 enum Total : int { kTotValid = 0, kTotChunks = 1, kTotActive = 2, kTotPBlocks = 3, kTotCount = 4 };
+
+// The block scan's published tile sums, which the transfer that follows clears
+// for the next scan.
+struct ScanStatus {
+  unsigned long long* words;
+  int n;
+  __device__ __forceinline__ void clear() const {
+    if (blockIdx.x == 0)
+      for (int i = threadIdx.x; i < n; i += kThreads) words[i] = 0ull;
+  }
+};
 
 // Source of a transfer's particle order (k_p2g, k_g2p2g).
 enum Order : int { kOrderGiven = 0, kOrderLists = 1, kOrderMove = 2 };
@@ -57,10 +69,9 @@ struct SubstepBuffers {
   int* pchunk_cnt;
   int4* chunks;     // (block, begin, end, 0)
   int* active;      // active grid blocks
-  int4* partials;   // block-scan partial sums
   int* totals;      // kTot*
   int* ghist;       // radix digit histograms, 2 x [kMaxRadixPasses][256] (substep parity)
-  unsigned long long* lb_status_scan;   // look-back status of k_bscan  [4 * tiles]
+  unsigned long long* scan_status;      // published tile sums of k_bscan [4 * tiles], zero between scans
   unsigned long long* lb_status_radix;  // look-back status of k_onesweep [256 * tiles]
   LBState* lbs;
   float4* tiles;    // p2g per-chunk node tiles (momentum xyz, mass)
@@ -87,7 +98,7 @@ struct SubstepBuffers {
   const int* dseg_prev;
   int* members;     // [cap] slots, grouped by direction (null: g2p leaves no lists)
   int* dseg;        // [chunk_cap][27] count | start << 16
-  int4* tile_prefix;  // two-level block scan
+  int4* tile_sums;  // tile sums of the two-level block scan
   // use_g2p2g mode: the fused transfer reads grid_in and writes grid;
   // particles with an insertion index >= n_final skip the G2P
   bool g2p2g;

@@ -122,31 +122,38 @@ __global__ __launch_bounds__(kThreads) void k_keys(const Params* __restrict__ sc
 template <int D>
 __device__ __forceinline__ int4 block_values(int bid, const int* __restrict__ count,
                                              const Params& P, int chunk) {
-  const int c = count[bid];
   int lb[3];
   decode_local<D>(bid, P, lb);
-  bool act = false;
+  const int c = count[bid];
   // p2g reaches blocks b + {0, 1}^d of a particle block b; the fused g2p2g
-  // transfer (new positions up to one cell away) b + {-1, 0, 1}^d
-  const int lo = P.g2p2g ? -1 : 0;
+  // transfer (new positions up to one cell away) b + {-1, 0, 1}^d.  The loads
+  // are unconditional (past the window's edge: the block's own count), so
+  // that all of them are in flight at once.
+  const int sx = 1, sy = P.bn[0], sz = P.bn[0] * P.bn[1];
+  int any = 0;
+  if (!P.g2p2g) {
 #pragma unroll
-  for (int dz = (D == 3 ? -1 : 0); dz < (D == 3 ? 2 : 1); dz++)
+    for (int k = 0; k < (D == 3 ? 8 : 4); k++) {
+      const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
+      const bool in = lb[0] >= dx && lb[1] >= dy && lb[2] >= dz;
+      any |= count[in ? bid - dx * sx - dy * sy - dz * sz : bid];
+    }
+  } else {
 #pragma unroll
-    for (int dy = -1; dy < 2; dy++)
-#pragma unroll
-      for (int dx = -1; dx < 2; dx++) {
-        if (dx < lo || dy < lo || (D == 3 && dz < lo)) continue;
-        int q[3] = {lb[0] - dx, lb[1] - dy, lb[2] - dz};
-        if (q[0] < 0 || q[1] < 0 || q[2] < 0 || q[0] >= P.bn[0] || q[1] >= P.bn[1] ||
-            (D == 3 && q[2] >= P.bn[2]))
-          continue;
-        act |= count[encode_local<D>(q, P)] > 0;
-      }
+    for (int k = 0; k < (D == 3 ? 27 : 9); k++) {
+      const int dx = k % 3 - 1, dy = (k / 3) % 3 - 1, dz = D == 3 ? k / 9 - 1 : 0;
+      const int q[3] = {lb[0] - dx, lb[1] - dy, lb[2] - dz};
+      const bool in = q[0] >= 0 && q[1] >= 0 && q[2] >= 0 && q[0] < P.bn[0] && q[1] < P.bn[1] &&
+                      (D == 2 || q[2] < P.bn[2]);
+      any |= count[in ? bid - dx * sx - dy * sy - dz * sz : bid];
+    }
+  }
+  const bool act = any != 0;  // counts are not negative
   return make_int4(c, (c + chunk - 1) / chunk, act ? 1 : 0, c > 0 ? 1 : 0);
 }
 
 // ---------------------------------------------------------------------------
-// single-pass scans with decoupled look-back (Merrill & Garland 2016)
+// the radix passes' scans with decoupled look-back (Merrill & Garland 2016)
 //
 // Status word: value in bits 0-31, flag in bits 32-33 (1 = tile aggregate,
 // 2 = inclusive prefix), launch epoch in bits 34-63.  Words left by earlier
@@ -194,43 +201,6 @@ __device__ __forceinline__ unsigned lb_lookback(const unsigned long long* status
   return excl;
 }
 
-// The same prefix, looked back by a whole wave: lane j reads the status of
-// tile - 1 - j (64 predecessors per round trip instead of one); the nearest
-// inclusive prefix in the window ends the sum.  Every lane returns the sum.
-__device__ __forceinline__ unsigned lb_lookback_wave(const unsigned long long* status, int stride,
-                                                     int tile, int chan, unsigned epoch,
-                                                     int* err) {
-  const unsigned long long ep = lb_epoch_bits(epoch);
-  const int lane = threadIdx.x & 63;
-  unsigned excl = 0;
-  for (int top = tile - 1; top >= 0; top -= 64) {
-    const int t = top - lane;
-    unsigned long long w = 0;
-    if (t >= 0) {
-      int spins = 0;
-      for (;;) {
-        w = __hip_atomic_load(&status[(int64_t)t * stride + chan], __ATOMIC_RELAXED,
-                              __HIP_MEMORY_SCOPE_AGENT);
-        if ((w & ~0x3ffffffffull) == ep && (w & (kFlagAgg | kFlagPre))) break;
-        if (++spins > kSpinLimit) {
-          atomicOr(err, 2);
-          w = ep | kFlagPre;  // give up: count this tile as a zero prefix
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
-    }
-    const unsigned long long pre = __ballot(t >= 0 && (w & kFlagPre) != 0);
-    const int stop = pre ? __ffsll((unsigned long long)pre) - 1 : 63;
-    unsigned v = (t >= 0 && lane <= stop) ? (unsigned)w : 0u;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    excl += v;
-    if (pre) break;
-  }
-  return excl;
-}
-
 struct LBTicket {
   int tile;
   unsigned epoch;
@@ -261,34 +231,75 @@ __device__ __forceinline__ void lb_release(LBState* st, int ntiles, unsigned epo
 // active grid blocks, and the radix digit histograms of the block keys
 // weighted by the particle counts (count[total_blocks] holds the particles
 // outside the window, whose key is total_blocks).
+//
+// Bound by its chain of dependent round trips to memory: the counts, then the
+// other tiles' sums.  Up to kScanTilesOnePass tiles, all of them resident at
+// once, every tile publishes its four sums and adds up those of all tiles
+// before it (one wave per sum, eight words per lane): nobody waits for
+// somebody else's prefix.  status[tile][channel] holds kScanReady | sum and is
+// cleared by the substep's first transfer, so there is no ticket, no epoch
+// and no release.  With tickets, a look-back over prefixes and each
+// neighbour's count loaded behind a branch: 1M particles (99 tiles) 11.8 ->
+// 7.0 us, 2D 20k 6.1 -> 4.6, unbounded 50k 16.4 -> 7.8, use_g2p2g 300k 13.9 ->
+// 8.1.  Larger windows take the tile sums from k_bscan_reduce, every tile
+// adding up those before it (no kernel between the two): 16M, 512^3 58 ->
+// 41 us, a batch of 16 scenes 23 -> 14.
 // ---------------------------------------------------------------------------
+constexpr unsigned long long kScanReady = 1ull << 32;
+
+// Sum of channel c of the tiles before `tile`, by one wave.  Tiles that are
+// not running yet (other work holds the device) start as that work ends, so
+// the wait is long but bounded: past kScanSpinLimit polls (seconds) it flags
+// err bit 1 and counts what it has.
+constexpr int kScanSpinLimit = 1 << 22;
+__device__ __forceinline__ unsigned scan_before(const unsigned long long* status, int tile, int c,
+                                                int* err) {
+  constexpr int W = kScanTilesOnePass / 64;
+  const int lane = threadIdx.x & 63;
+  unsigned long long w[W];
+#pragma unroll
+  for (int j = 0; j < W; j++) w[j] = lane + 64 * j < tile ? 0ull : kScanReady;
+  for (int spins = 0;; spins++) {
+    bool ready = true;
+#pragma unroll
+    for (int j = 0; j < W; j++) {
+      if (!(w[j] & kScanReady))
+        w[j] = __hip_atomic_load(&status[(int64_t)(lane + 64 * j) * 4 + c], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+      ready &= (w[j] & kScanReady) != 0;
+    }
+    if (__all(ready)) break;
+    if (spins > kScanSpinLimit) {
+      atomicOr(err, 2);
+      break;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  unsigned v = 0;
+#pragma unroll
+  for (int j = 0; j < W; j++) v += (unsigned)w[j];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  return v;
+}
+
 template <int D>
 __global__ __launch_bounds__(kThreads) void k_bscan(
     const Params* __restrict__ scenes, const int* __restrict__ count, int* __restrict__ count_next, int total_blocks,
     int chunk, int ntiles, int passes, int* __restrict__ pstart, int* __restrict__ pchunk_begin,
     int* __restrict__ pchunk_cnt, int4* __restrict__ chunks, int* __restrict__ active,
     int* __restrict__ totals, int* __restrict__ ghist, int* __restrict__ ghist_next,
-    unsigned long long* __restrict__ status, LBState* __restrict__ lbs,
-    const int4* __restrict__ tile_prefix, int* __restrict__ err, int* __restrict__ step) {
-  __shared__ LBTicket tk_sh;
+    unsigned long long* __restrict__ status, const int4* __restrict__ tile_sums,
+    int* __restrict__ err, int* __restrict__ step) {
   // one launch per substep: the substep counter of the max-velocity slots
   if (step && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(step, 1);
   __shared__ int4 wsum[kThreads / 64];
   __shared__ unsigned excl_sh[4];
   __shared__ int lh[kMaxRadixPasses][kRadixBins];
   const Params& P = scenes[0];  // the combined window extents
-  // tile_prefix != nullptr: exclusive tile prefixes were computed by
-  // k_bscan_reduce + k_bscan_top (large windows, where a look-back chain over
-  // thousands of tiles is slower than two extra launches)
-  LBTicket tk;
-  if (tile_prefix) {
-    tk.tile = blockIdx.x;
-    tk.epoch = 0;
-  } else {
-    tk = lb_acquire(lbs, &tk_sh);
-  }
-  const int tile = tk.tile;
-  for (int i = threadIdx.x; i < kMaxRadixPasses * kRadixBins; i += kThreads) (&lh[0][0])[i] = 0;
+  const int tile = blockIdx.x;
+  if (passes > 0)
+    for (int i = threadIdx.x; i < kMaxRadixPasses * kRadixBins; i += kThreads) (&lh[0][0])[i] = 0;
 
   const int first = tile * kScanTile + threadIdx.x * kScanItems;
   int4 vals[kScanItems];
@@ -317,24 +328,23 @@ __global__ __launch_bounds__(kThreads) void k_bscan(
   }
 
   static_assert(kThreads == 256, "one wave per scanned channel");
-  if (tile_prefix) {
+  if (tile_sums) {
+    int4 before = make_int4(0, 0, 0, 0), all;
+#pragma unroll 4
+    for (int i = threadIdx.x; i < tile; i += kThreads) before = add4(before, tile_sums[i]);
+    block_exscan4(before, &all, wsum);
     if (threadIdx.x < 4) {
-      const int4 tp = tile_prefix[tile];
       const int c = threadIdx.x;
-      excl_sh[c] = (unsigned)(c == 0 ? tp.x : c == 1 ? tp.y : c == 2 ? tp.z : tp.w);
+      excl_sh[c] = (unsigned)(c == 0 ? all.x : c == 1 ? all.y : c == 2 ? all.z : all.w);
     }
   } else {
-    // wave c looks back channel c
+    // wave c takes channel c
     const int c = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const unsigned agg = (unsigned)(c == 0 ? tot.x : c == 1 ? tot.y : c == 2 ? tot.z : tot.w);
-    unsigned excl = 0;
-    if (tile == 0) {
-      if (lane == 0) lb_publish(&status[c], kFlagPre, tk.epoch, agg);
-    } else {
-      if (lane == 0) lb_publish(&status[(int64_t)tile * 4 + c], kFlagAgg, tk.epoch, agg);
-      excl = lb_lookback_wave(status, 4, tile, c, tk.epoch, err);
-      if (lane == 0) lb_publish(&status[(int64_t)tile * 4 + c], kFlagPre, tk.epoch, excl + agg);
-    }
+    if (lane == 0)
+      __hip_atomic_store(&status[(int64_t)tile * 4 + c], kScanReady | (unsigned long long)agg,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned excl = scan_before(status, tile, c, err);
     if (lane == 0) excl_sh[c] = excl;
   }
   __syncthreads();
@@ -370,17 +380,14 @@ __global__ __launch_bounds__(kThreads) void k_bscan(
   }
   if (tile == 0)
     for (int i = threadIdx.x; i < kMaxRadixPasses * kRadixBins; i += kThreads) ghist_next[i] = 0;
-  __syncthreads();
-  if (!tile_prefix) lb_release(lbs, ntiles, tk.epoch);
 }
 
-// Two-level mode of the block-window scan: per-tile sums, then one workgroup
-// turns them into exclusive tile prefixes.
+// Tile sums of a window too large for the single pass.
 template <int D>
 __global__ __launch_bounds__(kThreads) void k_bscan_reduce(const Params* __restrict__ scenes,
                                                            const int* __restrict__ count,
                                                            int total_blocks, int chunk,
-                                                           int4* __restrict__ partials) {
+                                                           int4* __restrict__ tile_sums) {
   __shared__ int4 wsum[kThreads / 64];
   const Params& P = scenes[0];  // the combined window extents
   int4 acc = make_int4(0, 0, 0, 0);
@@ -390,27 +397,7 @@ __global__ __launch_bounds__(kThreads) void k_bscan_reduce(const Params* __restr
     if (first + k < total_blocks) acc = add4(acc, block_values<D>(first + k, count, P, chunk));
   int4 tot;
   block_exscan4(acc, &tot, wsum);
-  if (threadIdx.x == 0) partials[blockIdx.x] = tot;
-}
-
-// Each thread owns a contiguous run of the tile sums: one pass of
-// independent loads, one workgroup scan of the run totals, then the run's
-// exclusive prefixes (one dependent round instead of one per 256 tiles).
-__global__ __launch_bounds__(kThreads) void k_bscan_top(int4* __restrict__ partials, int nparts) {
-  __shared__ int4 wsum[kThreads / 64];
-  const int per = (nparts + kThreads - 1) / kThreads;
-  const int i0 = min(nparts, (int)threadIdx.x * per), i1 = min(nparts, i0 + per);
-  int4 acc = make_int4(0, 0, 0, 0);
-#pragma unroll 8
-  for (int i = i0; i < i1; i++) acc = add4(acc, partials[i]);
-  int4 tot;
-  int4 run = block_exscan4(acc, &tot, wsum);
-#pragma unroll 8
-  for (int i = i0; i < i1; i++) {
-    const int4 v = partials[i];
-    partials[i] = run;
-    run = add4(run, v);
-  }
+  if (threadIdx.x == 0) tile_sums[blockIdx.x] = tot;
 }
 
 // ---------------------------------------------------------------------------
@@ -549,8 +536,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const int4* __restrict__ chunks, const int* __restrict__ totals, float4* __restrict__ tiles,
     const float* __restrict__ gf, float* __restrict__ pf_out, PrevBinning prev,
     const int* __restrict__ pstart, int* __restrict__ pi_out, int n, int nw,
-    int* __restrict__ err) {
+    int* __restrict__ err, ScanStatus scan) {
   using L = Layout<D>;
+  if (MODE == 0) scan.clear();
   constexpr int TN = Geo<D>::kTileNodes;
   constexpr int CELLS = Geo<D>::kNodesPerBlock;  // cells of a block (64 / 16)
   constexpr int GROUPS = 64 / CELLS;             // lane groups per wave
@@ -1433,16 +1421,15 @@ static void launch_binning(const Params* P, SubstepBuffers& B, hipStream_t st, T
   }
   {
     TimerScope ts(tm, "k_bscan", st);
-    const bool two_level = nparts > 256;
+    const bool two_level = nparts > kScanTilesOnePass;
     if (two_level) {
       k_bscan_reduce<D><<<nparts, kThreads, 0, st>>>(P, B.count, B.total_blocks, B.chunk,
-                                                     B.tile_prefix);
-      k_bscan_top<<<1, kThreads, 0, st>>>(B.tile_prefix, nparts);
+                                                     B.tile_sums);
     }
     k_bscan<D><<<nparts, kThreads, 0, st>>>(
         P, B.count, B.count_next, B.total_blocks, B.chunk, nparts, B.full_sort ? passes : 0,
         B.pstart, B.pchunk_begin, B.pchunk_cnt, B.chunks, B.active, B.totals, ghist, ghist_next,
-        B.lb_status_scan, B.lbs, two_level ? B.tile_prefix : nullptr, B.err, B.step);
+        B.scan_status, two_level ? B.tile_sums : nullptr, B.err, B.step);
   }
   if (B.full_sort) {
     TimerScope ts(tm, "k_radix", st);
@@ -1465,6 +1452,13 @@ static void launch_binning(const Params* P, SubstepBuffers& B, hipStream_t st, T
     k_members<D><<<clamp_groups(div_up(chunk_bound, kThreads / 64), 4096), kThreads, 0, st>>>(
         P, B.chunks, B.totals, B.pstart, prev_binning(B), B.perm, B.err);
   }
+}
+
+// The block scan's status words (single-pass scans only), for the transfer
+// after it to clear.
+static ScanStatus scan_status(const SubstepBuffers& B) {
+  const int tiles = div_up(B.total_blocks, kScanTile);
+  return {B.scan_status, tiles <= kScanTilesOnePass ? 4 * tiles : 0};
 }
 
 // The slots were rewritten in sorted order by the transfer just launched.
@@ -1502,7 +1496,8 @@ static void launch_g2p2g(const Params* P, const int* slab, SubstepBuffers& B, in
     kern<<<xcd_groups(chunk_bound, G), kThreads, 0, st>>>(
         P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.grid_in, B.tiles, B.n_final,
         B.maxv, B.step, B.persistent_groups, B.members, B.dseg, B.count_next, B.err,
-        prev_binning(B), B.pstart, B.move ? B.pf_alt : B.pf, B.move ? B.pi_alt : nullptr, n, B.nw);
+        prev_binning(B), B.pstart, B.move ? B.pf_alt : B.pf, B.move ? B.pi_alt : nullptr, n, B.nw,
+        scan_status(B));
     if (B.move) take_moved(B);
   }
   {
@@ -1530,7 +1525,7 @@ void launch_transfer(const Params* P, const int* slab, SubstepBuffers& B, int ra
     kern<<<xcd_groups(chunk_bound, G), kThreads, 0, st>>>(
         P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.tiles, nullptr,
         B.move ? B.pf_alt : B.pf_out, prev_binning(B), B.pstart, B.move ? B.pi_alt : nullptr, n,
-        B.nw, B.err);
+        B.nw, B.err, scan_status(B));
     if (B.move) take_moved(B);
   }
   if (!B.grid_in_g2p) {
@@ -1608,7 +1603,7 @@ void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const f
       TimerScope ts(tm, "k_g2p_adj_scatter", st);
       k_p2g<D, 1><<<groups, kThreads, 0, st>>>(P, slab, pf_in, B.pi, B.cap, B.perm, B.chunks,
                                                B.totals, B.tiles, gout, nullptr, PrevBinning{},
-                                               nullptr, nullptr, n, 0, nullptr);
+                                               nullptr, nullptr, n, 0, nullptr, ScanStatus{});
     }
     {
       TimerScope ts(tm, "k_grid_op_adj", st);

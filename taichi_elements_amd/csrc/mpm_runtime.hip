@@ -142,9 +142,9 @@ struct mpm_solver {
   int* pstart = nullptr;
   int* pchunk_begin = nullptr;  // 2 x total_blocks (substep parity)
   int* pchunk_cnt = nullptr;    // 2 x total_blocks
-  int4* tile_prefix = nullptr;
+  int4* tile_sums = nullptr;
   int* active = nullptr;
-  unsigned long long* lb_status_scan = nullptr;
+  unsigned long long* scan_status = nullptr;
   LBState* lbs = nullptr;
   int* ghist = nullptr;
   float4* grid = nullptr;
@@ -455,7 +455,7 @@ void fill_buffers(mpm_solver* s, SubstepBuffers& B) {
   B.members_prev = s->members + prev * s->cap;
   B.dseg = s->dseg + cur * 27 * s->chunk_cap;
   B.dseg_prev = s->dseg + prev * 27 * s->chunk_cap;
-  B.tile_prefix = s->tile_prefix;
+  B.tile_sums = s->tile_sums;
   B.full_sort = !s->have_perm;
   B.g2p2g = s->g2p2g != 0;
   B.quant = s->quant != 0;
@@ -463,7 +463,7 @@ void fill_buffers(mpm_solver* s, SubstepBuffers& B) {
   B.grid_in = s->g2p2g ? s->grid : nullptr;
   B.n_final = (int)s->n_final;
   B.active = s->active;
-  B.lb_status_scan = s->lb_status_scan;
+  B.scan_status = s->scan_status;
   B.lb_status_radix = s->lb_status_radix;
   B.lbs = s->lbs;
   B.ghist = s->ghist;
@@ -725,10 +725,10 @@ void carve_diff_workspace(const mpm_solver* s, Carve& c, SubstepBuffers& B) {
   B.pchunk_cnt = B.pchunk_cnt_prev = c.take<int>(tb);
   B.chunks = B.chunks_prev = c.take<int4>(chunk_cap);
   B.active = c.take<int>(tb);
-  B.tile_prefix = c.take<int4>(nparts);
+  B.tile_sums = c.take<int4>(nparts);
   B.totals = c.take<int>(16);
   B.ghist = c.take<int>(2 * kMaxRadixPasses * kRadixBins);
-  B.lb_status_scan = c.take<unsigned long long>(4 * nparts);
+  B.scan_status = c.take<unsigned long long>(4 * nparts);
   B.lb_status_radix = c.take<unsigned long long>(kRadixBins * rtiles);
   B.lbs = c.take<LBState>(1);
   B.members = nullptr;  // steady-state binning only
@@ -753,12 +753,12 @@ int alloc_window_buffers(mpm_solver* s) {
   const int64_t nparts = (tb + kScanTile - 1) / kScanTile;
   TRY(dalloc(&s->count, tb + 1));
   TRY(dalloc(&s->count_next, tb + 1));
-  TRY(dalloc(&s->lb_status_scan, 4 * nparts));
+  TRY(dalloc(&s->scan_status, 4 * nparts));
   TRY(dalloc(&s->pstart, tb));
   TRY(dalloc(&s->pchunk_begin, 2 * tb));
   TRY(dalloc(&s->pchunk_cnt, 2 * tb));
   TRY(dalloc(&s->active, tb));
-  TRY(dalloc(&s->tile_prefix, nparts));
+  TRY(dalloc(&s->tile_sums, nparts));
   TRY(dalloc(&s->grid, tb * NPB));
   if (s->g2p2g) TRY(dalloc(&s->grid_alt, tb * NPB));
   TRY(dalloc(&s->d_slab, s->bn[D - 1]));
@@ -769,7 +769,7 @@ int alloc_window_buffers(mpm_solver* s) {
                          s->stream));
   HIP_TRY(hipMemsetAsync(s->count, 0, sizeof(int) * (tb + 1), s->stream));
   HIP_TRY(hipMemsetAsync(s->count_next, 0, sizeof(int) * (tb + 1), s->stream));
-  HIP_TRY(hipMemsetAsync(s->lb_status_scan, 0, sizeof(unsigned long long) * 4 * nparts,
+  HIP_TRY(hipMemsetAsync(s->scan_status, 0, sizeof(unsigned long long) * 4 * nparts,
                          s->stream));
   HIP_TRY(hipMemsetAsync(s->grid, 0, sizeof(float4) * tb * NPB, s->stream));
   if (s->grid_alt) HIP_TRY(hipMemsetAsync(s->grid_alt, 0, sizeof(float4) * tb * NPB, s->stream));
@@ -780,12 +780,12 @@ int alloc_window_buffers(mpm_solver* s) {
 void free_window_buffers(mpm_solver* s) {
   dfree(s->count);
   dfree(s->count_next);
-  dfree(s->lb_status_scan);
+  dfree(s->scan_status);
   dfree(s->pstart);
   dfree(s->pchunk_begin);
   dfree(s->pchunk_cnt);
   dfree(s->active);
-  dfree(s->tile_prefix);
+  dfree(s->tile_sums);
   dfree(s->grid);
   dfree(s->grid_alt);
   dfree(s->d_slab);
@@ -1015,9 +1015,9 @@ int mpm_destroy(mpm_solver* s) {
   dfree(s->pstart);
   dfree(s->pchunk_begin);
   dfree(s->pchunk_cnt);
-  dfree(s->tile_prefix);
+  dfree(s->tile_sums);
   dfree(s->active);
-  dfree(s->lb_status_scan);
+  dfree(s->scan_status);
   dfree(s->lbs);
   dfree(s->ghist);
   for (auto& g : s->graphs) hipGraphExecDestroy(g.exec);
@@ -2036,7 +2036,7 @@ int mpm_diff_substep_noalloc(mpm_solver* s, float dt, const float* state_in, flo
   const int64_t nparts = (tb + kScanTile - 1) / kScanTile;
   const int64_t rtiles = (s->diff_n + kRadixTile - 1) / kRadixTile;
   launch_fill_u32((unsigned*)B.ghist, 0u, 2 * kMaxRadixPasses * kRadixBins, st);
-  launch_fill_u32((unsigned*)B.lb_status_scan, 0u, 2 * 4 * nparts, st);
+  launch_fill_u32((unsigned*)B.scan_status, 0u, 2 * 4 * nparts, st);
   launch_fill_u32((unsigned*)B.lb_status_radix, 0u, 2 * kRadixBins * rtiles, st);
   launch_fill_u32((unsigned*)B.lbs, 0u, sizeof(LBState) / 4, st);
   if (s->D == 3)
