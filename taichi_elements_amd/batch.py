@@ -62,10 +62,18 @@ class BatchScene(MPMSolver):
         self._ids = np.concatenate([self._ids, np.arange(n0, n1, dtype=np.int64)])
         return added
 
+    def _rows(self):
+        """This scene's rows of the batch's insertion order: a slice (so a
+        view, not a copy) where they are one run, as after one seeding call."""
+        ids = self._ids
+        if len(ids) and ids[-1] - ids[0] + 1 == len(ids):  # ascending, so one run
+            return slice(int(ids[0]), int(ids[-1]) + 1)
+        return ids
+
     # readout: the library returns the whole batch in insertion order
     def particle_info(self):
         full = self._batch._particle_info_all()
-        out = {k: v[self._ids] for k, v in full.items()}
+        out = {k: v[self._rows()] for k, v in full.items()}
         if self.use_emitter_id:
             out['emitter_ids'] = self._emitter_ids.copy()
         return out
@@ -256,7 +264,7 @@ class MPMSolverBatch:
     def particle_info(self):
         """``particle_info()`` of every scene from one readback."""
         full = self._particle_info_all()
-        return [{k: v[s._ids] for k, v in full.items()} for s in self.scenes]
+        return [{k: v[s._rows()] for k, v in full.items()} for s in self.scenes]
 
     def _get_state_all(self):
         n = self._total_particles()

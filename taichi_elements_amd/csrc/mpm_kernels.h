@@ -171,6 +171,12 @@ void launch_scatter_f(const float* src, int64_t cap, int ncomp, const int* orig,
                       float* dst, hipStream_t st);
 void launch_scatter_i(const int* src, int64_t cap, int ncomp, const int* orig, int n, int* dst,
                       hipStream_t st);
+// x, v (n, D) and material in insertion order (null: not wanted).
+void launch_particle_info(int D, bool quant, bool g2p2g, const float* pf, const int* pi,
+                          int64_t cap, int n, float* x, float* v, int* mat, hipStream_t st);
+// out[r] = max of part[r * stride .. + stride), r < rows; out[rows] = *err.
+void launch_max_rows(const unsigned* part, int rows, int stride, const int* err, unsigned* out,
+                     hipStream_t st);
 void launch_fill_u32(unsigned* p, unsigned v, int64_t n, hipStream_t st);
 // svd3 / svd2 on n row-major dim x dim matrices (tests of the device SVD).
 void launch_svd_batch(int dim, const float* A, float* U, float* sig, float* V, int64_t n,

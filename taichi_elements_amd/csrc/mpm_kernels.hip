@@ -1334,6 +1334,58 @@ __global__ __launch_bounds__(kThreads) void k_scatter(const T* __restrict__ src,
   }
 }
 
+// particle_info (mpm_solver.py:1172-1191): x, v (n, D) and material in
+// insertion order, from either layout (null: not wanted).
+template <int D, bool Q, bool G>
+__global__ __launch_bounds__(kThreads) void k_particle_info(const float* __restrict__ pf,
+                                                            const int* __restrict__ pi,
+                                                            int64_t cap, int n,
+                                                            float* __restrict__ x,
+                                                            float* __restrict__ v,
+                                                            int* __restrict__ mat) {
+  using L = Layout<D>;
+  using PS = Particles<D, Q, G>;
+  for (int j = blockIdx.x * kThreads + threadIdx.x; j < n; j += gridDim.x * kThreads) {
+    const int64_t o = pi[(int64_t)L::ORIG * cap + j];
+    float a[3];
+    if (x) {
+      PS::load_x(pf, cap, j, a);
+#pragma unroll
+      for (int c = 0; c < D; c++) x[o * D + c] = a[c];
+    }
+    if (v) {
+      PS::load_v(pf, cap, j, a);
+#pragma unroll
+      for (int c = 0; c < D; c++) v[o * D + c] = a[c];
+    }
+    if (mat) mat[o] = pi[(int64_t)L::MAT * cap + j];
+  }
+}
+
+// Largest |v| of each substep (one workgroup) from its per-workgroup maxima
+// (float bits); the last workgroup copies the error bits behind them.  out is
+// pinned host memory.
+__global__ __launch_bounds__(kThreads) void k_max_rows(const unsigned* __restrict__ part,
+                                                       int stride, const int* __restrict__ err,
+                                                       unsigned* __restrict__ out) {
+  if (blockIdx.x == gridDim.x - 1) {
+    if (threadIdx.x == 0) out[blockIdx.x] = (unsigned)*err;
+    return;
+  }
+  __shared__ unsigned red[kThreads / 64];
+  unsigned m = 0;
+  for (int i = threadIdx.x; i < stride; i += kThreads)
+    m = max(m, part[(int64_t)blockIdx.x * stride + i]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kThreads / 64; w++) m = max(m, red[w]);
+    out[blockIdx.x] = m;
+  }
+}
+
 __global__ __launch_bounds__(kThreads) void k_copy_segments(CopySegments S) {
   for (int s = 0; s < S.count; s++)
     for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < S.n[s];
@@ -1695,6 +1747,19 @@ void launch_scatter_i(const int* src, int64_t cap, int ncomp, const int* orig, i
   if (n > 0)
     k_scatter<int><<<clamp_groups(div_up(n, kThreads), 8192), kThreads, 0, st>>>(src, cap, ncomp,
                                                                               orig, n, dst);
+}
+void launch_particle_info(int D, bool quant, bool g2p2g, const float* pf, const int* pi,
+                          int64_t cap, int n, float* x, float* v, int* mat, hipStream_t st) {
+  if (n <= 0) return;
+  auto kern = D == 3 ? (quant ? (g2p2g ? k_particle_info<3, true, true> : k_particle_info<3, true, false>)
+                              : k_particle_info<3, false, false>)
+                     : (quant ? (g2p2g ? k_particle_info<2, true, true> : k_particle_info<2, true, false>)
+                              : k_particle_info<2, false, false>);
+  kern<<<clamp_groups(div_up(n, kThreads), 8192), kThreads, 0, st>>>(pf, pi, cap, n, x, v, mat);
+}
+void launch_max_rows(const unsigned* part, int rows, int stride, const int* err, unsigned* out,
+                     hipStream_t st) {
+  k_max_rows<<<rows + 1, kThreads, 0, st>>>(part, stride, err, out);
 }
 void launch_copy_segments(const CopySegments& S, hipStream_t st) {
   int64_t most = 0;

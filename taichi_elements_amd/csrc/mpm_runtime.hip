@@ -20,6 +20,7 @@
 
 #include "../../include/mpm_abi.h"
 #include "mpm_kernels.h"
+#include "mpm_readback.h"
 
 using namespace mpm;
 
@@ -154,6 +155,17 @@ struct mpm_solver {
   unsigned* maxv = nullptr;
   int maxv_cap = 0;
   int last_batch = 0;
+  // pinned: per-substep max |v| and the error bits, written by a kernel
+  // (behind the scene table, or own_words for calls of many substeps)
+  unsigned* host_words = nullptr;
+  unsigned* own_words = nullptr;
+  int host_words_cap = 0;
+  // read access to the particles: device staging in insertion order and the
+  // copies to the caller's memory; read_mu: readers of one handle take turns
+  std::mutex read_mu;
+  char* stage = nullptr;
+  size_t stage_cap = 0;
+  Readback readback;
 
   bool have_perm = false;  // perm of the previous substep matches the slots
   int since_reorder = 1 << 30;  // reorder at the first opportunity
@@ -267,12 +279,9 @@ int no_half_pending(const mpm_solver* s) {
   return MPM_OK;
 }
 
-int check_device_errors(mpm_solver* s) {
-  HIP_TRY(hipSetDevice(s->device));
-  HIP_TRY(hipStreamSynchronize(s->stream));
+// The error bits e of the kernels so far, as an error code; clears them.
+int report_errors(mpm_solver* s, int e) {
   if (s->timing) s->timer.collect();
-  int e = 0;
-  HIP_TRY(hipMemcpy(&e, s->err, sizeof(int), hipMemcpyDeviceToHost));
   if (e) {
     int z = 0;
     HIP_TRY(hipMemcpy(s->err, &z, sizeof(int), hipMemcpyHostToDevice));
@@ -288,6 +297,32 @@ int check_device_errors(mpm_solver* s) {
                               std::to_string(e) + ")");
   }
   return MPM_OK;
+}
+
+int check_device_errors(mpm_solver* s) {
+  HIP_TRY(hipSetDevice(s->device));
+  HIP_TRY(hipStreamSynchronize(s->stream));
+  int e = 0;
+  HIP_TRY(hipMemcpy(&e, s->err, sizeof(int), hipMemcpyDeviceToHost));
+  return report_errors(s, e);
+}
+
+// Device staging of at least `bytes`, kept by the handle.
+int stage_reserve(mpm_solver* s, size_t bytes) {
+  if (bytes <= s->stage_cap) return MPM_OK;
+  dfree(s->stage);
+  s->stage_cap = 0;
+  TRY(dalloc(&s->stage, (int64_t)bytes));
+  s->stage_cap = bytes;
+  return MPM_OK;
+}
+
+// The segments and the error bits to the host, after the stream's work so far.
+int read_back(mpm_solver* s, std::vector<Readback::Segment> segments) {
+  int e = 0;
+  segments.push_back({s->err, &e, sizeof(int), false});
+  HIP_TRY(s->readback.copy(segments, s->stream));
+  return report_errors(s, e);
 }
 
 void fill_params(Params& P, const mpm_solver* s, const SceneHost& sc, float dt, int skip) {
@@ -973,11 +1008,14 @@ static int create_impl(const mpm_config* cfgs, int nscenes, mpm_solver** out) {
     return r;
   }
   s->maxv_cap = 16 * s->persistent_groups;
-  if (hipHostMalloc((void**)&s->h_params, sizeof(Params) * nscenes) != hipSuccess) {
+  s->host_words_cap = 256;
+  if (hipHostMalloc((void**)&s->h_params,
+                    sizeof(Params) * nscenes + sizeof(unsigned) * s->host_words_cap) != hipSuccess) {
     s->h_params = nullptr;
     mpm_destroy(s);
     return fail(MPM_ENOMEM, "pinned host allocation failed");
   }
+  s->host_words = (unsigned*)(s->h_params + nscenes);
   if (hipMemsetAsync(s->lbs, 0, sizeof(LBState), s->stream) != hipSuccess ||
       hipMemsetAsync(s->ghist, 0, sizeof(int) * 2 * kMaxRadixPasses * kRadixBins, s->stream) !=
           hipSuccess ||
@@ -1041,6 +1079,9 @@ int mpm_destroy(mpm_solver* s) {
   dfree(s->diff_abuf);
   dfree(s->diff_nu_part);
   if (s->h_params) hipHostFree(s->h_params);
+  if (s->own_words) hipHostFree(s->own_words);
+  dfree(s->stage);
+  s->readback.release();
   if (s->stream) hipStreamDestroy(s->stream);
   delete s;
   return MPM_OK;
@@ -1325,18 +1366,22 @@ int mpm_substep_end(mpm_solver* s) {
 int mpm_read_max_velocity(mpm_solver* s, int32_t nsub, float* out) {
   if (!s || (!out && nsub > 0)) return fail(MPM_EINVAL, "null argument");
   if (nsub > s->last_batch) return fail(MPM_EINVAL, "more entries than substeps run");
-  int r = check_device_errors(s);
-  if (nsub > 0) {
-    const int G = s->persistent_groups;
-    std::vector<float> part((size_t)nsub * G);
-    HIP_TRY(hipMemcpy(part.data(), s->maxv, sizeof(float) * part.size(), hipMemcpyDeviceToHost));
-    for (int k = 0; k < nsub; k++) {
-      float m = 0.0f;
-      for (int g = 0; g < G; g++) m = std::max(m, part[(size_t)k * G + g]);
-      out[k] = m;
-    }
+  HIP_TRY(hipSetDevice(s->device));
+  std::lock_guard<std::mutex> lock(s->read_mu);
+  // reduced on the device, straight into pinned host memory with the error bits
+  if (s->host_words_cap < nsub + 1) {
+    unsigned* more = nullptr;
+    if (hipHostMalloc((void**)&more, sizeof(unsigned) * (nsub + 1)) != hipSuccess)
+      return fail(MPM_ENOMEM, "pinned host allocation failed");
+    if (s->own_words) hipHostFree(s->own_words);
+    s->host_words = s->own_words = more;
+    s->host_words_cap = nsub + 1;
   }
-  return r;
+  launch_max_rows(s->maxv, nsub, s->persistent_groups, s->err, s->host_words, s->stream);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(s->stream));
+  if (nsub > 0) std::memcpy(out, s->host_words, sizeof(float) * nsub);
+  return report_errors(s, (int)s->host_words[nsub]);
 }
 
 int mpm_sync(mpm_solver* s) {
@@ -1377,20 +1422,18 @@ int mpm_get_state(mpm_solver* s, int32_t field, void* host) {
     TRY(unpacked(s, flt));
     src = flt.p;
   }
-  void* tmp = nullptr;
-  HIP_TRY(hipMalloc(&tmp, sizeof(float) * s->n * nc));
+  const size_t bytes = sizeof(float) * s->n * nc;
+  std::lock_guard<std::mutex> lock(s->read_mu);
+  TRY(stage_reserve(s, bytes));
   const int* orig = s->pi + s->cap;  // Layout ORIG == 1
   if (is_int)
-    launch_gather_i(s->pi + (int64_t)c0 * s->cap, s->cap, nc, orig, (int)s->n, (int*)tmp,
+    launch_gather_i(s->pi + (int64_t)c0 * s->cap, s->cap, nc, orig, (int)s->n, (int*)s->stage,
                     s->stream);
   else
-    launch_gather_f(src + (int64_t)c0 * s->cap, s->cap, nc, orig, (int)s->n, (float*)tmp,
+    launch_gather_f(src + (int64_t)c0 * s->cap, s->cap, nc, orig, (int)s->n, (float*)s->stage,
                     s->stream);
-  int r = check_device_errors(s);
-  hipError_t e = hipMemcpy(host, tmp, sizeof(float) * s->n * nc, hipMemcpyDeviceToHost);
-  hipFree(tmp);
-  if (e != hipSuccess) return fail(MPM_EHIP, std::string("hipMemcpy: ") + hipGetErrorString(e));
-  return r;
+  HIP_TRY(hipGetLastError());
+  return read_back(s, {{s->stage, host, bytes, false}});
 }
 
 int mpm_set_state(mpm_solver* s, int32_t field, const void* host) {
@@ -1444,11 +1487,23 @@ int mpm_set_state(mpm_solver* s, int32_t field, const void* host) {
 int mpm_particle_info(mpm_solver* s, float* x, float* v, int32_t* material, int32_t* color) {
   if (!s) return fail(MPM_EINVAL, "null argument");
   TRY(no_half_pending(s));
-  if (x) TRY(mpm_get_state(s, MPM_FIELD_X, x));
-  if (v) TRY(mpm_get_state(s, MPM_FIELD_V, v));
-  if (material) TRY(mpm_get_state(s, MPM_FIELD_MATERIAL, material));
-  if (color) TRY(mpm_get_state(s, MPM_FIELD_COLOR, color));
-  return MPM_OK;
+  HIP_TRY(hipSetDevice(s->device));
+  if (s->n == 0) return MPM_OK;
+  // x, v and material gathered together, then one pass of copies for all
+  std::lock_guard<std::mutex> lock(s->read_mu);
+  const size_t nx = x ? sizeof(float) * s->n * s->D : 0, nv = v ? sizeof(float) * s->n * s->D : 0;
+  const size_t nm = material ? sizeof(int32_t) * s->n : 0;
+  TRY(stage_reserve(s, std::max<size_t>(nx + nv + nm, 1)));
+  char *dx = s->stage, *dv = dx + nx, *dm = dv + nv;
+  if (nx + nv + nm > 0)
+    launch_particle_info(s->D, s->quant != 0, s->g2p2g != 0, s->pf, s->pi, s->cap, (int)s->n,
+                         x ? (float*)dx : nullptr, v ? (float*)dv : nullptr,
+                         material ? (int*)dm : nullptr, s->stream);
+  HIP_TRY(hipGetLastError());
+  return read_back(s, {{dx, x, nx, false},
+                       {dv, v, nv, false},
+                       {dm, material, nm, false},
+                       {s->color.data(), color, color ? sizeof(int32_t) * s->n : 0, true}});
 }
 
 int mpm_read_grid(mpm_solver* s, const int32_t* lo, const int32_t* nn, float* m, float* v) {
