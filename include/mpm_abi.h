@@ -308,6 +308,10 @@ int mpm_last_counts(mpm_solver* s, int64_t* out4);
  *   grad_in = dL/d state_in, grad_youngs = dL/dE (may be NULL) and
  *   grad_nu[0] = dL/dnu (device).  The grid is recomputed from state_in, on
  *   the forward's binning record when given (else the binning is redone).
+ * mpm_diff_reorder: dst[r * n + i] = src[r * row_stride + index[i] *
+ *   col_stride] for r < rows and i < n, the particle count of mpm_diff_setup
+ *   (strides in floats, >= 0; index: device, a permutation of 0 .. n - 1 or
+ *   any in-range columns of src; dst must not overlap src).
  * mpm_diff_sync: waits for stream and reports domain / CFL errors. */
 int mpm_diff_setup(mpm_solver* s, int64_t n, const int32_t* material);
 int mpm_diff_binning_bytes(mpm_solver* s, int64_t* bytes);
@@ -317,6 +321,8 @@ int mpm_diff_substep_backward(mpm_solver* s, float dt, const float* state_in,
                               const float* youngs, double nu, const void* binning,
                               const float* grad_out, float* grad_in, float* grad_youngs,
                               float* grad_nu, void* stream);
+int mpm_diff_reorder(mpm_solver* s, const float* src, int64_t row_stride, int64_t col_stride,
+                     const int64_t* index, float* dst, int32_t rows, void* stream);
 int mpm_diff_sync(mpm_solver* s, void* stream);
 /* Allocation-free form of mpm_diff_substep (no counterpart in the reference:
  * it is for callers that cannot allocate device memory -- code under HIP

@@ -81,6 +81,8 @@ SIGNATURES = [
                                         _P]),
     ("mpm_diff_substep_backward", ctypes.c_int, [_P, ctypes.c_float, _P, _P, ctypes.c_double, _P,
                                                  _P, _P, _P, _P, _P]),
+    ("mpm_diff_reorder", ctypes.c_int, [_P, _P, ctypes.c_int64, ctypes.c_int64, _P, _P,
+                                        ctypes.c_int32, _P]),
     ("mpm_diff_sync", ctypes.c_int, [_P, _P]),
     ("mpm_diff_substep_noalloc", ctypes.c_int, [_P, ctypes.c_float, _P, _P, _P,
                                                 ctypes.c_double, _P]),

@@ -218,6 +218,8 @@ struct CopySegments {
   int count;
 };
 void launch_copy_segments(const CopySegments& S, hipStream_t st);
+void launch_take_columns(const float* src, int64_t row_stride, int64_t col_stride,
+                         const int64_t* index, float* dst, int rows, int64_t n, hipStream_t st);
 
 // Quantised particle output (mpm_io.hip).  Components 0..D-1 are x, D..2D-1 v.
 struct QuantRanges {

@@ -2148,6 +2148,19 @@ int mpm_diff_substep_backward(mpm_solver* s, float dt, const float* state_in,
   return MPM_OK;
 }
 
+int mpm_diff_reorder(mpm_solver* s, const float* src, int64_t row_stride, int64_t col_stride,
+                     const int64_t* index, float* dst, int32_t rows, void* stream) {
+  if (!s || !index || (rows != 0 && (!src || !dst))) return fail(MPM_EINVAL, "null argument");
+  if (s->diff_n == 0) return fail(MPM_EINVAL, "mpm_diff_setup first");
+  if (rows < 0 || row_stride < 0 || col_stride < 0)
+    return fail(MPM_EINVAL, "rows and strides must be >= 0");
+  HIP_TRY(hipSetDevice(s->device));
+  launch_take_columns(src, row_stride, col_stride, index, dst, rows, s->diff_n,
+                      (hipStream_t)stream);
+  HIP_TRY(hipGetLastError());
+  return MPM_OK;
+}
+
 int mpm_diff_sync(mpm_solver* s, void* stream) {
   if (!s) return fail(MPM_EINVAL, "null argument");
   HIP_TRY(hipSetDevice(s->device));

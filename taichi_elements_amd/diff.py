@@ -51,14 +51,16 @@ def _stream():
 class _Substep(torch.autograd.Function):
 
     @staticmethod
-    def forward(ctx, state, youngs, nu, solver, nu_value, dt):
+    def forward(ctx, state, youngs, nu, solver, nu_value, dt, keep):
         # the kernels read the state as dense (NF, n) rows and E as n floats
         if not (state.is_contiguous() and youngs.is_contiguous()):
             raise ValueError("state and youngs must be contiguous tensors")
         out = torch.empty_like(state)
         # the substep's record (binning and grid sums), kept for the backward
-        # pass, which then runs only the adjoint kernels
-        binning = torch.empty(solver._binning_bytes, dtype=torch.uint8, device=state.device)
+        # pass, which then runs only the adjoint kernels; without gradients
+        # (keep) there is none to keep
+        binning = torch.empty(solver._binning_bytes if keep else 0, dtype=torch.uint8,
+                              device=state.device)
         check(_lib.lib().mpm_diff_substep(solver._handle, float(dt), _ptr(state), _ptr(out),
                                           _ptr(youngs), float(nu_value), _ptr(binning),
                                           _stream()))
@@ -83,7 +85,26 @@ class _Substep(torch.autograd.Function):
             _ptr(binning), _ptr(grad_out), _ptr(grad_in), _ptr(grad_e), _ptr(grad_nu),
             _stream()))
         return (grad_in, grad_e, grad_nu.reshape(ctx.nu_shape).to(ctx.nu_dtype), None, None,
-                None)
+                None, None)
+
+
+class _Reorder(torch.autograd.Function):
+    """Particles (the last axis of a 1-D or 2-D float32 tensor) taken in the
+    order of the permutation ``index``, whose inverse takes the gradient back
+    (the backward of ``t[:, index]`` sorts the indices first)."""
+
+    @staticmethod
+    def forward(ctx, t, solver, index, inverse):
+        ctx.solver, ctx.index, ctx.inverse = solver, index, inverse
+        out = torch.empty(t.shape, dtype=t.dtype, device=t.device)
+        rows, row_stride = (t.shape[0], t.stride(0)) if t.dim() == 2 else (1, 0)
+        check(_lib.lib().mpm_diff_reorder(solver._handle, _ptr(t), row_stride, t.stride(-1),
+                                          _ptr(index), _ptr(out), rows, _stream()))
+        return out
+
+    @staticmethod
+    def backward(ctx, grad):
+        return _Reorder.apply(grad, ctx.solver, ctx.inverse, ctx.index), None, None, None
 
 
 class DiffMPMSolver:
@@ -179,7 +200,9 @@ class DiffMPMSolver:
 
     def _segment(self, state, youngs, nu, nu_value, dt, k):
         for _ in range(k):
-            state, _ = _Substep.apply(state, youngs, nu, self, nu_value, dt)
+            keep = torch.is_grad_enabled() and (state.requires_grad or youngs.requires_grad
+                                                or nu.requires_grad)
+            state, _ = _Substep.apply(state, youngs, nu, self, nu_value, dt, keep)
         return state
 
     # Device memory that run() may fill with the inputs of every substep
@@ -201,8 +224,8 @@ class DiffMPMSolver:
         if nu_value is None:
             nu_value = float(nu.detach()) if torch.is_tensor(nu) else float(nu)
         if self._order is not None:
-            state = state[:, self._order]
-            youngs = youngs[self._order]
+            state = self._reordered(state, 2, nsub, self._order, self._inverse)
+            youngs = self._reordered(youngs, 1, nsub, self._order, self._inverse)
         # a transposed or sliced tensor is copied into the (NF, n) row layout
         # the kernels read (the copy is part of the autograd graph)
         state = state.contiguous()
@@ -220,8 +243,17 @@ class DiffMPMSolver:
             else:
                 state = self._segment(state, youngs, nu, nu_value, dt, m)
         if self._inverse is not None:
-            state = state[:, self._inverse]
+            state = self._reordered(state, 2, nsub, self._inverse, self._order)
         return state
+
+    def _reordered(self, t, dims, nsub, index, inverse):
+        # The kernel reads n float32 columns on the solver's device.  Anything
+        # else, and a run of no substeps (which has all of indexing's
+        # transforms, where a substep has its backward alone), is indexed.
+        if (nsub > 0 and t.dim() == dims and t.shape[-1] == self.n and t.dtype == torch.float32
+                and t.device == index.device and t.layout == torch.strided):
+            return _Reorder.apply(t, self, index, inverse)
+        return t[:, index] if dims == 2 else t[index]
 
     def check(self):
         """Waits for the work queued so far; raises DomainError if particles
