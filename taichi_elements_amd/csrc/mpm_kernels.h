@@ -19,8 +19,17 @@ constexpr int kOneRound = 160 * 1024;
 constexpr int kScanItems = 2;                       // per thread in the block scan
 constexpr int kScanTile = kThreads * kScanItems;    // 512 blocks per workgroup
 constexpr int kScanTilesOnePass = 512;  // the single-pass scan's most tiles, all resident at once
-constexpr int kRadixItems = 16;
-constexpr int kRadixTile = kThreads * kRadixItems;  // 2048 keys per workgroup
+// Keys per workgroup of a sort pass: kRadixTile, or, while they make no more
+// than kRadixSmallTiles tiles, kRadixSmallTile (k_onesweep says why).
+constexpr int kRadixItems = 16, kRadixSmallItems = 8;
+constexpr int kRadixTile = kThreads * kRadixItems;
+constexpr int kRadixSmallTile = kThreads * kRadixSmallItems;
+constexpr int kRadixSmallTiles = 128;
+// Tiles whose status words a sort of n keys can make use of.
+constexpr int64_t radix_tiles(int64_t n) {
+  const int64_t small = (n + kRadixSmallTile - 1) / kRadixSmallTile;
+  return small <= kRadixSmallTiles ? small : (n + kRadixTile - 1) / kRadixTile;
+}
 constexpr int kRadixBins = 256;
 constexpr int kMaxRadixPasses = 3;                  // block keys up to 24 bits
 
@@ -72,7 +81,8 @@ struct SubstepBuffers {
   int* totals;      // kTot*
   int* ghist;       // radix digit histograms, 2 x [kMaxRadixPasses][256] (substep parity)
   unsigned long long* scan_status;      // published tile sums of k_bscan [4 * tiles], zero between scans
-  unsigned long long* lb_status_radix;  // look-back status of k_onesweep [256 * tiles]
+  unsigned long long* lb_status_radix;  // look-back status of k_onesweep [256 * radix_cap]
+  int64_t radix_cap;
   LBState* lbs;
   float4* tiles;    // p2g per-chunk node tiles (momentum xyz, mass)
   float4* grid;     // dense block-major grid [total_blocks][nodes] of (v, mass)
@@ -106,6 +116,7 @@ struct SubstepBuffers {
   int n_final;
   bool quant;         // packed particle layout (PackedLayout<D>)
   int nw;             // particle float-buffer words per slot
+  bool count_zeroed;  // count holds zeros (full_sort clears it otherwise)
   bool full_sort;     // radix-sort the slots (first substep / positions set by the host)
 };
 

@@ -180,23 +180,37 @@ __device__ __forceinline__ void lb_publish(unsigned long long* p, unsigned long 
 // A bounded wait: past kSpinLimit polls it flags err bit 1 and returns what it has.
 __device__ __forceinline__ unsigned lb_lookback(const unsigned long long* status, int stride,
                                                 int tile, int chan, unsigned epoch, int* err) {
+  constexpr int W = 8;  // predecessors read at once: one round trip, not eight in turn
   const unsigned long long ep = lb_epoch_bits(epoch);
   unsigned excl = 0;
-  for (int t = tile - 1; t >= 0; t--) {
-    unsigned long long w = 0;
-    int spins = 0;
-    for (;;) {
-      w = __hip_atomic_load(&status[(int64_t)t * stride + chan], __ATOMIC_RELAXED,
-                            __HIP_MEMORY_SCOPE_AGENT);
-      if ((w & ~0x3ffffffffull) == ep && (w & (kFlagAgg | kFlagPre))) break;
+  int spins = 0;
+  for (int t = tile - 1; t >= 0;) {
+    unsigned long long w[W];
+#pragma unroll
+    for (int j = 0; j < W; j++)
+      w[j] = t - j >= 0 ? __hip_atomic_load(&status[(int64_t)(t - j) * stride + chan],
+                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                        : (ep | kFlagPre);
+    bool ready = true, done = false;
+    int used = 0;
+#pragma unroll
+    for (int j = 0; j < W; j++) {
+      ready &= (w[j] & ~0x3ffffffffull) == ep && (w[j] & (kFlagAgg | kFlagPre));
+      if (ready && !done) {
+        excl += (unsigned)w[j];
+        done = (w[j] & kFlagPre) != 0;
+        used++;
+      }
+    }
+    if (done) break;
+    t -= used;
+    if (used < W) {
       if (++spins > kSpinLimit) {
         atomicOr(err, 2);
         return excl;
       }
       __builtin_amdgcn_s_sleep(1);
     }
-    excl += (unsigned)w;
-    if (w & kFlagPre) break;
   }
   return excl;
 }
@@ -206,7 +220,12 @@ struct LBTicket {
   unsigned epoch;
 };
 
-__device__ __forceinline__ LBTicket lb_acquire(LBState* st, LBTicket* sh) {
+// Tiles that are all resident at once need no ticket to be sure that their
+// predecessors run; the epoch changes only after every tile has read it.
+__device__ __forceinline__ LBTicket lb_acquire(LBState* st, LBTicket* sh, int ntiles) {
+  if (ntiles <= kScanTilesOnePass)
+    return {(int)blockIdx.x,
+            __hip_atomic_load(&st->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
   if (threadIdx.x == 0) {
     sh->tile = (int)atomicAdd(&st->tile_ctr, 1ull);
     sh->epoch = __hip_atomic_load(&st->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -407,23 +426,33 @@ __global__ __launch_bounds__(kThreads) void k_bscan_reduce(const Params* __restr
 // the four waves gives tile-local stable ranks; decoupled look-back over
 // tiles gives the per-digit tile offsets; the digit totals come from the
 // histogram k_bscan built.
+//
+// Up to a few hundred thousand keys a pass is one chain of latencies: the
+// keys, ITEMS rounds of ranking, the look-back, the stores.  Smaller tiles
+// halve the rounds but lengthen the look-back, whose status words come from
+// memory past the L2s: 200k keys, 16 items a thread with a ticket and one
+// predecessor at a time 13.0 us; eight predecessors at a time, no ticket and
+// 16 / 8 / 4 / 2 items 12.5 / 11.0 / 11.9 / 14.1 us; 32 predecessors at a time
+// 13.0 (8 items) and 14.6 (4).
 // ---------------------------------------------------------------------------
+template <int ITEMS>
 __global__ __launch_bounds__(kThreads) void k_onesweep(
     const int* __restrict__ keys_in, const int* __restrict__ vals_in, int* __restrict__ keys_out,
     int* __restrict__ vals_out, int n, int shift, int ntiles, const int* __restrict__ ghist,
     unsigned long long* __restrict__ status, LBState* __restrict__ lbs, int* __restrict__ err) {
   constexpr int WAVES = kThreads / 64;
-  constexpr int PER_WAVE = kRadixTile / WAVES;
+  constexpr int TILE = kThreads * ITEMS;
+  constexpr int PER_WAVE = TILE / WAVES;
   constexpr int ROUNDS = PER_WAVE / 64;
   __shared__ LBTicket tk_sh;
   __shared__ int wcnt[WAVES][kRadixBins];
   __shared__ int gbase[kRadixBins];
   __shared__ int4 wsum[WAVES];
-  const LBTicket tk = lb_acquire(lbs, &tk_sh);
+  const LBTicket tk = lb_acquire(lbs, &tk_sh, ntiles);
   const int tile = tk.tile;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  const int i0 = tile * kRadixTile + wave * PER_WAVE + lane;
+  const int i0 = tile * TILE + wave * PER_WAVE + lane;
 
   int key[ROUNDS], val[ROUNDS], lr[ROUNDS];
 #pragma unroll
@@ -1489,7 +1518,7 @@ static void launch_binning(const Params* P, SubstepBuffers& B, hipStream_t st, T
     // first substep (or positions changed from the host): block counts from
     // scratch, then a stable radix sort of the slots
     TimerScope ts(tm, "k_keys", st);
-    launch_fill_u32((unsigned*)B.count, 0u, B.total_blocks + 1, st);
+    if (!B.count_zeroed) launch_fill_u32((unsigned*)B.count, 0u, B.total_blocks + 1, st);
     if (B.quant)
       k_keys<D, true><<<clamp_groups(div_up(n, kThreads), 8192), kThreads, 0, st>>>(
           P, B.pf, B.pi, B.cap, n, B.total_blocks, B.keys, B.count, B.err);
@@ -1511,13 +1540,16 @@ static void launch_binning(const Params* P, SubstepBuffers& B, hipStream_t st, T
   }
   if (B.full_sort) {
     TimerScope ts(tm, "k_radix", st);
-    const int ntiles = div_up(n, kRadixTile);
+    const int small = div_up(n, kRadixSmallTile);
+    const bool use_small = small <= kRadixSmallTiles && small <= B.radix_cap;
+    const int ntiles = use_small ? small : div_up(n, kRadixTile);
+    auto kern = use_small ? k_onesweep<kRadixSmallItems> : k_onesweep<kRadixItems>;
     const int* kin = B.keys;
     const int* vin = nullptr;
     int* kbuf[2] = {B.keys_alt, B.keys_alt + B.cap};
     int* vbuf[2] = {B.perm, B.perm_alt};
     for (int pass = 0; pass < passes; pass++) {
-      k_onesweep<<<ntiles, kThreads, 0, st>>>(kin, vin, kbuf[pass & 1], vbuf[pass & 1], n,
+      kern<<<ntiles, kThreads, 0, st>>>(kin, vin, kbuf[pass & 1], vbuf[pass & 1], n,
                                                pass * 8, ntiles, ghist + pass * kRadixBins,
                                                B.lb_status_radix, B.lbs, B.err);
       kin = kbuf[pass & 1];

@@ -132,6 +132,7 @@ struct mpm_solver {
   int* perm = nullptr;
   int* perm_alt = nullptr;
   unsigned long long* lb_status_radix = nullptr;
+  int64_t radix_cap = 0;  // tiles it holds
   float4* tiles = nullptr;
   int4* chunks = nullptr;  // 2 x chunk_cap (substep parity)
   int64_t chunk_cap = 0;
@@ -139,6 +140,7 @@ struct mpm_solver {
   int* dseg = nullptr;     // 2 x 27 x chunk_cap (substep parity)
   // buffers sized by the block window
   int* count = nullptr;
+  bool count_zeroed = false;  // count holds zeros: the differentiable substep before cleared it
   int* count_next = nullptr;
   int* pstart = nullptr;
   int* pchunk_begin = nullptr;  // 2 x total_blocks (substep parity)
@@ -431,7 +433,11 @@ int grow(mpm_solver* s, int64_t need) {
   TRY(dalloc(&s->keys_alt, 2 * ncap));
   TRY(dalloc(&s->perm, ncap));
   TRY(dalloc(&s->perm_alt, ncap));
-  const int64_t ntiles = (ncap + kRadixTile - 1) / kRadixTile;
+  // any n <= ncap: radix_tiles() grows up to kRadixSmallTiles, then drops
+  const int64_t ntiles = std::max(radix_tiles(ncap),
+                                  radix_tiles(std::min<int64_t>(
+                                      ncap, (int64_t)kRadixSmallTiles * kRadixSmallTile)));
+  s->radix_cap = ntiles;
   TRY(dalloc(&s->lb_status_radix, kRadixBins * ntiles));
   HIP_TRY(hipMemsetAsync(s->lb_status_radix, 0, sizeof(unsigned long long) * kRadixBins * ntiles,
                          s->stream));
@@ -500,6 +506,8 @@ void fill_buffers(mpm_solver* s, SubstepBuffers& B) {
   B.active = s->active;
   B.scan_status = s->scan_status;
   B.lb_status_radix = s->lb_status_radix;
+  B.radix_cap = s->radix_cap;
+  B.count_zeroed = false;
   B.lbs = s->lbs;
   B.ghist = s->ghist;
   B.totals = s->totals + cur * 16;
@@ -528,6 +536,7 @@ void take_buffers(mpm_solver* s, const SubstepBuffers& B) {
   s->last_parity = B.parity;
   s->count = B.count;
   s->count_next = B.count_next;
+  s->count_zeroed = false;
 }
 
 // B for the next substep; the particles move into the sorted order with it
@@ -765,6 +774,7 @@ void carve_diff_workspace(const mpm_solver* s, Carve& c, SubstepBuffers& B) {
   B.ghist = c.take<int>(2 * kMaxRadixPasses * kRadixBins);
   B.scan_status = c.take<unsigned long long>(4 * nparts);
   B.lb_status_radix = c.take<unsigned long long>(kRadixBins * rtiles);
+  B.radix_cap = rtiles;
   B.lbs = c.take<LBState>(1);
   B.members = nullptr;  // steady-state binning only
   B.dseg = nullptr;
@@ -2031,6 +2041,15 @@ int mpm_diff_substep(mpm_solver* s, float dt, const float* state_in, float* stat
   diff_buffers(s, B, const_cast<float*>(state_in));
   B.pf_out = state_out;  // p2g / g2p write the new state out of place
   if (binning) B.raw_out = (float4*)((char*)binning + bin_layout(s).grid);
+  // A differentiable substep leaves the other count array cleared (its block
+  // scan does that, and its g2p counts nothing), so the next one needs no fill
+  // (3 us of 85).  Under capture there is always one: a replay may follow
+  // anything.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &cap));
+  const bool eager = cap == hipStreamCaptureStatusNone;
+  B.count_zeroed = eager && s->count_zeroed;
+  s->count_zeroed = false;
   if (s->D == 3)
     launch_substep<3>(s->d_params, slab_table(s), B, 0, 0, st, nullptr);
   else
@@ -2055,6 +2074,7 @@ int mpm_diff_substep(mpm_solver* s, float dt, const float* state_in, float* stat
   take_buffers(s, B);
   s->substep_counter++;
   HIP_TRY(hipGetLastError());
+  s->count_zeroed = eager;
   return MPM_OK;
 }
 
