@@ -120,10 +120,8 @@ __global__ __launch_bounds__(kThreads) void k_keys(const Params* __restrict__ sc
 // block, non-empty particle block).  A grid block is active when one of the
 // particle blocks b - {0,1}^d holds particles (their stencils reach it).
 template <int D>
-__device__ __forceinline__ int4 block_values(int bid, const int* __restrict__ count,
-                                             const Params& P, int chunk) {
-  int lb[3];
-  decode_local<D>(bid, P, lb);
+__device__ __forceinline__ int4 block_values(int bid, const int lb[3],
+                                             const int* __restrict__ count, const Params& P) {
   const int c = count[bid];
   // p2g reaches blocks b + {0, 1}^d of a particle block b; the fused g2p2g
   // transfer (new positions up to one cell away) b + {-1, 0, 1}^d.  The loads
@@ -149,7 +147,17 @@ __device__ __forceinline__ int4 block_values(int bid, const int* __restrict__ co
     }
   }
   const bool act = any != 0;  // counts are not negative
-  return make_int4(c, (c + chunk - 1) / chunk, act ? 1 : 0, c > 0 ? 1 : 0);
+  return make_int4(c, 0, act ? 1 : 0, c > 0 ? 1 : 0);
+}
+
+template <int D>
+__device__ __forceinline__ int4 block_values(int bid, const int* __restrict__ count,
+                                             const Params& P, int chunk) {
+  int lb[3];
+  decode_local<D>(bid, P, lb);
+  int4 v = block_values<D>(bid, lb, count, P);
+  v.y = (v.x + chunk - 1) / chunk;
+  return v;
 }
 
 // ---------------------------------------------------------------------------
@@ -526,6 +534,125 @@ __global__ __launch_bounds__(kThreads) void k_onesweep(
 }
 
 // ---------------------------------------------------------------------------
+// The block scan inside p2g.  Every workgroup scans the whole window itself
+// (kWindowItems blocks per thread) to find its chunks; the last one, which
+// seldom has a chunk, also writes k_bscan's results for the kernels after it.
+// Bound, like k_bscan, by round trips to memory, of which this is one instead
+// of a kernel's four: taken in 2D by steady-state substeps of windows of up to
+// kThreads kWindowItems blocks and up to kOneRound particles, where each
+// workgroup has about one chunk.  A kernel of 3.9 to 4.7 us and its launch
+// go, p2g takes 3 to 4 us longer: a substep of 5000 particles (400 blocks)
+// 19.8 -> 17.5 us, 60000 (1369 blocks) 24.1 -> 23.1, 160000 (2025 blocks) 28.5
+// -> 27.4.  With the counts read by each thread where it needs them, without
+// LDS, p2g took 12 us longer at 1369 blocks.  In 3D the registers spill.
+// ---------------------------------------------------------------------------
+struct WindowScan {
+  const int* count;
+  int* count_next;
+  int total_blocks, chunk;
+  unsigned chunk_inv;  // ceil(2^32 / chunk): x / chunk for x < 2^32 / chunk
+  int *pstart, *pchunk_begin, *pchunk_cnt;
+  int4* chunks;
+  int *active, *totals, *ghist_next, *step;
+};
+constexpr int kWindowItems = 9;
+constexpr int kWindowGroups = 1024;  // all resident at once
+
+template <int D>
+struct ScannedWindow {
+  static constexpr int K = kWindowItems;
+  int per;                   // blocks per thread: odd, so that its LDS reads conflict with none
+  int nchunks, pos, chunk0;  // position and chunk of the thread's first block
+  int n[K], nc[K];           // particles and chunks of its blocks
+
+  // lcount: kThreads K words of LDS, free again afterwards.
+  __device__ void scan(const WindowScan& A, const Params& P, int* lcount, int4* wsum) {
+    per = (A.total_blocks + kThreads - 1) / kThreads | 1;
+    int c[K];
+#pragma unroll
+    for (int k = 0; k < K; k++)
+      if (k < per) c[k] = A.count[min(k * kThreads + (int)threadIdx.x, A.total_blocks)];
+#pragma unroll
+    for (int k = 0; k < K; k++)
+      if (k < per) lcount[k * kThreads + threadIdx.x] = c[k];
+    lds_barrier();
+    const int first = threadIdx.x * per;
+    int lb[3] = {0, 0, 0};
+    if (first < A.total_blocks) decode_local<D>(first, P, lb);
+    int4 v[K], acc = make_int4(0, 0, 0, 0), tot;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      v[k] = make_int4(0, 0, 0, 0);
+      n[k] = nc[k] = 0;
+      if (k >= per) continue;
+      // past the window: block 0, read like the others, counts for nothing
+      const bool on = first + k < A.total_blocks;
+      const int l[3] = {on ? lb[0] : 0, on ? lb[1] : 0, on ? lb[2] : 0};
+      v[k] = block_values<D>(on ? first + k : 0, l, lcount, P);
+      v[k].y = (int)__umulhi((unsigned)(v[k].x + A.chunk - 1), A.chunk_inv);
+      if (!on) v[k] = make_int4(0, 0, 0, 0);
+      if (++lb[0] == P.bn[0]) {
+        lb[0] = 0;
+        if (++lb[1] == P.bn[1]) {
+          lb[1] = 0;
+          lb[2]++;
+        }
+      }
+      acc = add4(acc, v[k]);
+      n[k] = v[k].x;
+      nc[k] = v[k].y;
+    }
+    int4 pre = block_exscan4(acc, &tot, wsum);
+    nchunks = tot.y;
+    pos = pre.x;
+    chunk0 = pre.y;
+    if (blockIdx.x != gridDim.x - 1) return;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const int bid = first + k;
+      if (k >= per || bid >= A.total_blocks) break;
+      A.pstart[bid] = pre.x;
+      A.pchunk_begin[bid] = pre.y;
+      A.pchunk_cnt[bid] = v[k].y;
+      for (int c = 0; c < v[k].y; c++) {
+        const int b0 = pre.x + c * A.chunk;
+        A.chunks[pre.y + c] = make_int4(bid, b0, min(b0 + A.chunk, pre.x + v[k].x), 0);
+      }
+      if (v[k].z) A.active[pre.z] = bid;
+      A.count_next[bid] = 0;
+      pre = add4(pre, v[k]);
+    }
+    for (int i = threadIdx.x; i < kMaxRadixPasses * kRadixBins; i += kThreads) A.ghist_next[i] = 0;
+    if (threadIdx.x == 0) {
+      A.count_next[A.total_blocks] = 0;
+      A.totals[kTotValid] = tot.x;
+      A.totals[kTotChunks] = tot.y;
+      A.totals[kTotActive] = tot.z;
+      A.totals[kTotPBlocks] = tot.w;
+      if (A.step) atomicAdd(A.step, 1);  // the substep counter of the max-velocity slots
+    }
+  }
+
+  // Chunk c (block, begin, end, the block's first position), from the thread
+  // that holds its block; the whole workgroup calls it with a slot that no
+  // call without a barrier in between uses.
+  __device__ int4 find(int c, int chunk, int4* slot) const {
+    int p = pos, c0 = chunk0;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      if (c >= c0 && c < c0 + nc[k]) {
+        const int b0 = p + (c - c0) * chunk;
+        *slot = make_int4(threadIdx.x * per + k, b0, min(b0 + chunk, p + n[k]), p);
+      }
+      p += n[k];
+      c0 += nc[k];
+    }
+    lds_barrier();
+    return *slot;
+  }
+};
+
+// ---------------------------------------------------------------------------
 // P2G (mpm_solver.py:487-584)
 //
 // One workgroup per chunk (<= kChunkMax particles of one grid block), taken
@@ -558,16 +685,17 @@ __global__ __launch_bounds__(kThreads) void k_onesweep(
 // bound by the vector ALU and LDS, so the extra writes cost less than a pass
 // of their own (1M particles: 76 -> 98 us instead of 76 + 65; 16M: 1.15 ->
 // 2.24 ms instead of 1.15 + 1.64).
-template <int D, int MODE, bool Q = false, int ORDER = kOrderGiven>
+// SCAN (with kOrderLists): the block scan runs in here (WindowScan).
+template <int D, int MODE, bool Q = false, int ORDER = kOrderGiven, bool SCAN = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_p2g(
     const Params* __restrict__ scenes, const int* __restrict__ slab, const float* __restrict__ pf,
     const int* __restrict__ pi, int64_t cap, int* __restrict__ perm,
     const int4* __restrict__ chunks, const int* __restrict__ totals, float4* __restrict__ tiles,
     const float* __restrict__ gf, float* __restrict__ pf_out, PrevBinning prev,
     const int* __restrict__ pstart, int* __restrict__ pi_out, int n, int nw,
-    int* __restrict__ err, ScanStatus scan) {
+    int* __restrict__ err, ScanStatus scan, WindowScan window) {
   using L = Layout<D>;
-  if (MODE == 0) scan.clear();
+  if (MODE == 0 && !SCAN) scan.clear();
   constexpr int TN = Geo<D>::kTileNodes;
   constexpr int CELLS = Geo<D>::kNodesPerBlock;  // cells of a block (64 / 16)
   constexpr int GROUPS = 64 / CELLS;             // lane groups per wave
@@ -581,15 +709,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  for (XcdItems it(totals[kTotChunks], kSpreadChunks); it.valid(); it.next()) {
+  __shared__ int4 wsum[SCAN ? kThreads / 64 : 1], found[SCAN ? 2 : 1];
+  ScannedWindow<D> own;
+  if (SCAN) own.scan(window, scenes[0], reinterpret_cast<int*>(&ptile[0][0]), wsum);
+  static_assert(!SCAN || sizeof(ptile) >= sizeof(int) * kThreads * kWindowItems, "");
+  int turn = 0;
+  for (XcdItems it(SCAN ? own.nchunks : totals[kTotChunks], kSpreadChunks); it.valid(); it.next()) {
     const int c = it.c;
-    const int4 ck = chunks[c];
+    const int4 ck = SCAN ? own.find(c, window.chunk, &found[SCAN ? turn ^= 1 : 0]) : chunks[c];
     int lbc[3], b[3];
     decode_local<D>(ck.x, scenes[0], lbc);
     const Params& P = scenes[scene_of<D>(lbc, slab)];
     int ids[kChunkMax / kThreads];  // slots of this thread's particle of each batch
     if (ORDER == kOrderLists) {
-      const int first = pstart[ck.x];
+      const int first = SCAN ? ck.w : pstart[ck.x];
       wave_members<D, kChunkMax / kThreads>(lbc, ck.y - first + threadIdx.x, kThreads,
                                             ck.z - first, scenes[0], prev, ids);
 #pragma unroll
@@ -1504,6 +1637,13 @@ static bool order_in_transfer(const SubstepBuffers& B) {
   return !B.full_sort && !B.move && B.n <= kOneRound;
 }
 
+// Whether p2g scans the block window itself (WindowScan says why there).
+template <int D>
+static bool scan_in_p2g(const SubstepBuffers& B) {
+  return D == 2 && order_in_transfer(B) && !B.g2p2g &&
+         B.total_blocks <= kThreads * kWindowItems;
+}
+
 // binning of one substep: block counts, the dense-window scan (chunks,
 // active blocks) and the sorted order
 template <int D>
@@ -1526,7 +1666,7 @@ static void launch_binning(const Params* P, SubstepBuffers& B, hipStream_t st, T
       k_keys<D, false><<<clamp_groups(div_up(n, kThreads), 8192), kThreads, 0, st>>>(
           P, B.pf, B.pi, B.cap, n, B.total_blocks, B.keys, B.count, B.err);
   }
-  {
+  if (!scan_in_p2g<D>(B)) {
     TimerScope ts(tm, "k_bscan", st);
     const bool two_level = nparts > kScanTilesOnePass;
     if (two_level) {
@@ -1569,6 +1709,13 @@ static void launch_binning(const Params* P, SubstepBuffers& B, hipStream_t st, T
 static ScanStatus scan_status(const SubstepBuffers& B) {
   const int tiles = div_up(B.total_blocks, kScanTile);
   return {B.scan_status, tiles <= kScanTilesOnePass ? 4 * tiles : 0};
+}
+
+static WindowScan window_scan(const SubstepBuffers& B) {
+  const unsigned inv = (unsigned)(((1ull << 32) + B.chunk - 1) / B.chunk);
+  return {B.count, B.count_next, B.total_blocks, B.chunk, inv, B.pstart, B.pchunk_begin,
+          B.pchunk_cnt, B.chunks, B.active, B.totals,
+          B.ghist + ((B.parity & 1) ^ 1) * kMaxRadixPasses * kRadixBins, B.step};
 }
 
 // The slots were rewritten in sorted order by the transfer just launched.
@@ -1631,11 +1778,17 @@ void launch_transfer(const Params* P, const int* slab, SubstepBuffers& B, int ra
     auto kern = B.quant ? k_p2g<D, 0, true> : k_p2g<D, 0, false>;
     if (order_in_transfer(B))
       kern = B.quant ? k_p2g<D, 0, true, kOrderLists> : k_p2g<D, 0, false, kOrderLists>;
+    int groups = xcd_groups(chunk_bound, G);
+    if constexpr (D == 2)
+      if (scan_in_p2g<D>(B)) {
+        groups = std::min(groups, kWindowGroups);
+        kern = B.quant ? k_p2g<D, 0, true, kOrderLists, true> : k_p2g<D, 0, false, kOrderLists, true>;
+      }
     if (B.move) kern = B.quant ? k_p2g<D, 0, true, kOrderMove> : k_p2g<D, 0, false, kOrderMove>;
-    kern<<<xcd_groups(chunk_bound, G), kThreads, 0, st>>>(
+    kern<<<groups, kThreads, 0, st>>>(
         P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.tiles, nullptr,
         B.move ? B.pf_alt : B.pf_out, prev_binning(B), B.pstart, B.move ? B.pi_alt : nullptr, n,
-        B.nw, B.err, scan_status(B));
+        B.nw, B.err, scan_status(B), window_scan(B));
     if (B.move) take_moved(B);
   }
   if (!B.grid_in_g2p) {
@@ -1713,7 +1866,8 @@ void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const f
       TimerScope ts(tm, "k_g2p_adj_scatter", st);
       k_p2g<D, 1><<<groups, kThreads, 0, st>>>(P, slab, pf_in, B.pi, B.cap, B.perm, B.chunks,
                                                B.totals, B.tiles, gout, nullptr, PrevBinning{},
-                                               nullptr, nullptr, n, 0, nullptr, ScanStatus{});
+                                               nullptr, nullptr, n, 0, nullptr, ScanStatus{},
+                                               WindowScan{});
     }
     {
       TimerScope ts(tm, "k_grid_op_adj", st);
