@@ -1778,7 +1778,12 @@ void launch_transfer(const Params* P, const int* slab, SubstepBuffers& B, int ra
     auto kern = B.quant ? k_p2g<D, 0, true> : k_p2g<D, 0, false>;
     if (order_in_transfer(B))
       kern = B.quant ? k_p2g<D, 0, true, kOrderLists> : k_p2g<D, 0, false, kOrderLists>;
-    int groups = xcd_groups(chunk_bound, G);
+    // Past kOneRound particles four times the workgroups of the other transfer:
+    // with one or two chunks each, the hardware evens out chunks that differ by
+    // material and size, and p2g has little to set up per workgroup (2048 and
+    // 8192: 1M 74.6 and 72.5 us, 2D 400k 21.2 and 19.4, a batch of 1.1M 86.5
+    // and 82.4, 16M 1258 and 1219).
+    int groups = xcd_groups(chunk_bound, n > kOneRound ? 4 * G : G);
     if constexpr (D == 2)
       if (scan_in_p2g<D>(B)) {
         groups = std::min(groups, kWindowGroups);
