@@ -380,52 +380,228 @@ __device__ __forceinline__ void load_cf(const float* __restrict__ pf, int64_t ca
     }
 }
 
-// Step 1 (per particle): the affine matrix A of every binned particle, into
-// abuf (D*D rows of cap).
+// The affine matrix A of a particle.
 template <int D>
-__global__ __launch_bounds__(kThreads) void k_adj_affine(
-    const Params* __restrict__ scenes, const int* __restrict__ slab,
-    const float* __restrict__ pf, const int* __restrict__ pi, int64_t cap,
-    const int* __restrict__ perm, const int* __restrict__ totals, float* __restrict__ abuf) {
+__device__ __forceinline__ void affine_matrix(const Params& P, const float* __restrict__ pf,
+                                              int64_t cap, int p, int mat, float A[3][3]) {
   using L = Layout<D>;
-  const int nvalid = totals[kTotValid];
-  for (int j = blockIdx.x * kThreads + threadIdx.x; j < nvalid; j += gridDim.x * kThreads) {
-    const int p = perm[j];
-    const Params& P = scenes[pi[(int64_t)L::SCENE * cap + p]];
-    const int mat = pi[(int64_t)L::MAT * cap + p];
-    float C[3][3], F[3][3];
-    load_cf<D>(pf, cap, p, C, F);
-    if (mat == kSnow || mat == kSand) {  // the forward's own constitutive update
-      float Jc = pf[(int64_t)L::JP * cap + p], stress[3][3];
-      const float E = P.youngs ? P.youngs[p] : 0.0f;
-      constitutive<D>(mat, P, P.youngs ? E * P.kmu : P.mu_0, P.youngs ? E * P.kla : P.lambda_0, F,
-                      C, Jc, stress);
+  float C[3][3], F[3][3];
+  load_cf<D>(pf, cap, p, C, F);
+  const float E = P.youngs ? P.youngs[p] : 0.0f;
+  if (mat == kSnow || mat == kSand) {  // the forward's own constitutive update
+    float Jc = pf[(int64_t)L::JP * cap + p], stress[3][3];
+    constitutive<D>(mat, P, P.youngs ? E * P.kmu : P.mu_0, P.youngs ? E * P.kla : P.lambda_0, F, C,
+                    Jc, stress);
 #pragma unroll
-      for (int a = 0; a < D; a++)
+    for (int a = 0; a < D; a++)
 #pragma unroll
-        for (int e = 0; e < D; e++)
-          abuf[(int64_t)(a * D + e) * cap + p] = P.stress_scale * stress[a][e] + P.p_mass * C[a][e];
-      continue;
+      for (int e = 0; e < D; e++) A[a][e] = P.stress_scale * stress[a][e] + P.p_mass * C[a][e];
+    return;
+  }
+  Recompute<D> r;
+  recompute<D>(P, mat, C, F, pf[(int64_t)L::JP * cap + p], E, r);
+  const float iso = r.la * r.J * (r.J - 1.0f);
+#pragma unroll
+  for (int a = 0; a < D; a++)
+#pragma unroll
+    for (int e = 0; e < D; e++) {
+      float s = 0.0f;
+#pragma unroll
+      for (int k = 0; k < D; k++) s += (r.Fp[a][k] - r.R[a][k]) * r.Fp[e][k];
+      const float tau = 2.0f * r.mu * s + (a == e ? iso : 0.0f);
+      A[a][e] = P.stress_scale * tau + r.mass * C[a][e];
     }
-    Recompute<D> r;
-    recompute<D>(P, mat, C, F, pf[(int64_t)L::JP * cap + p], P.youngs ? P.youngs[p] : 0.0f, r);
-    const float iso = r.la * r.J * (r.J - 1.0f);
+}
+
+// The constitutive adjoint of a particle: from Ab = Abar, writes Cbar, Fbar,
+// Jpbar and Ebar and adds to the nu adjoint.
+template <int D>
+__device__ __forceinline__ void constitutive_adjoint(const Params& P, const float* __restrict__ pf,
+                                                     int64_t cap, int p, int mat,
+                                                     const float* __restrict__ gf,
+                                                     const float Ab[3][3],
+                                                     float* __restrict__ gin,
+                                                     float* __restrict__ gE, float& nu_acc) {
+  using L = Layout<D>;
+  float C[3][3], F[3][3];
+  load_cf<D>(pf, cap, p, C, F);
+  const float Jp = pf[(int64_t)L::JP * cap + p];
+  const float E = P.youngs ? P.youngs[p] : 0.0f;
+  if (mat == kSnow || mat == kSand) {
+    float K[3][3] = {{0.0f}}, Fp[3][3] = {{0.0f}}, G[3][3] = {{0.0f}}, Fbo[3][3] = {{0.0f}};
+    float Cb[3][3] = {{0.0f}};
+#pragma unroll
+    for (int a = 0; a < D; a++)
+#pragma unroll
+      for (int e = 0; e < D; e++) {
+        K[a][e] = (a == e ? 1.0f : 0.0f) + P.dt * C[a][e];
+        const float abar = Ab[a][e];
+        Cb[a][e] = P.p_mass * abar;
+        G[a][e] = P.stress_scale * abar;
+        Fbo[a][e] = gf[(int64_t)(L::F + a * D + e) * cap + p];
+      }
 #pragma unroll
     for (int a = 0; a < D; a++)
 #pragma unroll
       for (int e = 0; e < D; e++) {
         float s = 0.0f;
 #pragma unroll
-        for (int k = 0; k < D; k++) s += (r.Fp[a][k] - r.R[a][k]) * r.Fp[e][k];
-        const float tau = 2.0f * r.mu * s + (a == e ? iso : 0.0f);
-        abuf[(int64_t)(a * D + e) * cap + p] = P.stress_scale * tau + r.mass * C[a][e];
+        for (int k = 0; k < D; k++) s += K[a][k] * F[k][e];
+        Fp[a][e] = s;
       }
+    float Fpb[3][3], Jpbar, mu0b, la0b, cb;
+    plastic_adjoint<D>(P, mat, Fp, Jp, P.youngs ? E * P.kmu : P.mu_0,
+                       P.youngs ? E * P.kla : P.lambda_0, G, Fbo,
+                       gf[(int64_t)L::JP * cap + p], Fpb, Jpbar, mu0b, la0b, cb);
+    // F' = K F: Fbar = K^T F'bar, Cbar += dt F'bar F^T
+#pragma unroll
+    for (int a = 0; a < D; a++)
+#pragma unroll
+      for (int e = 0; e < D; e++) {
+        float fb = 0.0f, t = 0.0f;
+#pragma unroll
+        for (int k = 0; k < D; k++) {
+          fb += K[k][a] * Fpb[k][e];
+          t += Fpb[a][k] * F[e][k];
+        }
+        gin[(int64_t)(L::C + a * D + e) * cap + p] = Cb[a][e] + P.dt * t;
+        gin[(int64_t)(L::F + a * D + e) * cap + p] = fb;
+      }
+    gin[(int64_t)L::JP * cap + p] = Jpbar;
+    // mu_0 = E kmu, lambda_0 = E kla; sand's coefficient depends on nu
+    if (gE) gE[p] = P.kmu * mu0b + P.kla * la0b;
+    nu_acc += E * (P.dkmu * mu0b + P.dkla * la0b) + cb * P.dsand_coef * P.alpha;
+    return;
   }
+  Recompute<D> r;
+  recompute<D>(P, mat, C, F, Jp, E, r);
+  float Cbar[3][3] = {{0}}, G[3][3] = {{0}}, Fbo[3][3] = {{0}};
+#pragma unroll
+  for (int a = 0; a < D; a++)
+#pragma unroll
+    for (int e = 0; e < D; e++) {
+      const float abar = Ab[a][e];
+      Cbar[a][e] = r.mass * abar;
+      G[a][e] = P.stress_scale * abar;
+      Fbo[a][e] = gf[(int64_t)(L::F + a * D + e) * cap + p];
+    }
+  const float Jpbo = gf[(int64_t)L::JP * cap + p];
+  float trG = 0.0f;
+#pragma unroll
+  for (int a = 0; a < D; a++) trG += G[a][a];
+  const float J = r.J;
+  const float labar = trG * J * (J - 1.0f);
+  float Jbar = r.la * trG * (2.0f * J - 1.0f);
+  float Fbar[3][3] = {{0}}, Jpbar, mubar = 0.0f;
+  if (r.water) {
+    Jbar += Fbo[0][0] + Jpbo;
+    const float detK = det_d<D>(r.K);
+    float cK[3][3];
+    cofactor_d<D>(r.K, cK);
+    Jpbar = Jbar * detK;
+#pragma unroll
+    for (int a = 0; a < D; a++)
+#pragma unroll
+      for (int e = 0; e < D; e++) Cbar[a][e] += Jbar * Jp * P.dt * cK[a][e];
+  } else {
+    const float mu = r.mu;
+    float Fpb[3][3], Rb[3][3];
+    {
+      float cF[3][3];
+      cofactor_d<D>(r.Fp, cF);
+#pragma unroll
+      for (int a = 0; a < D; a++)
+#pragma unroll
+        for (int e = 0; e < D; e++) {
+          float gfp = 0.0f, gtt = 0.0f, tft = 0.0f;
+#pragma unroll
+          for (int k = 0; k < D; k++) {
+            gfp += G[a][k] * r.Fp[k][e];                          // (G F')_ae
+            gtt += G[k][a] * (r.Fp[k][e] - r.R[k][e]);            // (G^T (F' - R))_ae
+            tft += (r.Fp[a][k] - r.R[a][k]) * r.Fp[e][k];         // ((F' - R) F'^T)_ae
+          }
+          mubar += 2.0f * G[a][e] * tft;
+          Fpb[a][e] = Fbo[a][e] + 2.0f * mu * (gfp + gtt) + Jbar * cF[a][e];
+          Rb[a][e] = -2.0f * mu * gfp;
+        }
+    }
+    // polar adjoint: B = U^T Rb V, Mbar = skew(B) / (sig_i + sig_j), F'bar += U Mbar V^T
+    float Bm[3][3];
+#pragma unroll
+    for (int a = 0; a < D; a++)
+#pragma unroll
+      for (int e = 0; e < D; e++) {
+        float t[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int m2 = 0; m2 < D; m2++)
+#pragma unroll
+          for (int k = 0; k < D; k++) t[m2] += r.U[k][a] * Rb[k][m2];
+        float s = 0.0f;
+#pragma unroll
+        for (int m2 = 0; m2 < D; m2++) s += t[m2] * r.V[m2][e];
+        Bm[a][e] = s;
+      }
+    float Mb[3][3];
+#pragma unroll
+    for (int a = 0; a < D; a++)
+#pragma unroll
+      for (int e = 0; e < D; e++) {
+        if (a == e) {
+          Mb[a][e] = 0.0f;
+        } else {
+          float den = r.sig[a] + r.sig[e];
+          if (fabsf(den) < 1e-6f) den = den < 0.0f ? -1e-6f : 1e-6f;
+          Mb[a][e] = (Bm[a][e] - Bm[e][a]) / den;
+        }
+      }
+#pragma unroll
+    for (int a = 0; a < D; a++)
+#pragma unroll
+      for (int e = 0; e < D; e++) {
+        float s = 0.0f;
+#pragma unroll
+        for (int k = 0; k < D; k++)
+#pragma unroll
+          for (int m2 = 0; m2 < D; m2++) s += r.U[a][k] * Mb[k][m2] * r.V[e][m2];
+        Fpb[a][e] += s;
+      }
+    // F' = K F: Fbar = K^T F'bar, Cbar += dt F'bar F^T
+#pragma unroll
+    for (int a = 0; a < D; a++)
+#pragma unroll
+      for (int e = 0; e < D; e++) {
+        float s = 0.0f, t = 0.0f;
+#pragma unroll
+        for (int k = 0; k < D; k++) {
+          s += r.K[k][a] * Fpb[k][e];
+          t += Fpb[a][k] * F[e][k];
+        }
+        Fbar[a][e] = s;
+        Cbar[a][e] += P.dt * t;
+      }
+    Jpbar = Jpbo;
+  }
+  // mu = h E kmu, la = h E kla
+  if (gE) gE[p] = r.h * (P.kmu * mubar + P.kla * labar);
+  nu_acc += r.h * E * (P.dkmu * mubar + P.dkla * labar);
+#pragma unroll
+  for (int a = 0; a < D; a++)
+#pragma unroll
+    for (int e = 0; e < D; e++) {
+      gin[(int64_t)(L::C + a * D + e) * cap + p] = Cbar[a][e];
+      gin[(int64_t)(L::F + a * D + e) * cap + p] = Fbar[a][e];
+    }
+  gin[(int64_t)L::JP * cap + p] = Jpbar;
 }
 
-// Step 2 (per chunk, stencil): the g2p adjoint gather and the p2g adjoint
-// gathers.  Writes xbar and vbar into gin, and Abar = dx sum_i w_i pbar_i
-// d_i^T into gin's C rows (step 3 turns it into Cbar).
+// The adjoint of the particles (per chunk): A again, the g2p adjoint gather and
+// the p2g adjoint gathers (xbar, vbar and Abar = dx sum_i w_i pbar_i d_i^T),
+// and the constitutive adjoint, with per-workgroup nu partials.  One kernel:
+// bound by latency at the sizes that are differentiated; with A and the
+// constitutive adjoint in kernels of their own, each read the state again and
+// A and Abar went through memory
+// (150k: 10.4 + 16.5 + 12.4 us and two launches -> 34.0; 1.5M, four substeps
+// forward and backward 4.16 -> 4.11 ms).
 template <int D>
 __global__ __launch_bounds__(kThreads) void k_p2g_adj(
     const Params* __restrict__ scenes, const int* __restrict__ slab,
@@ -433,11 +609,13 @@ __global__ __launch_bounds__(kThreads) void k_p2g_adj(
     const int* __restrict__ perm, const int4* __restrict__ chunks,
     const int* __restrict__ totals, const float4* __restrict__ grid,
     const float4* __restrict__ gbar, const float* __restrict__ gf,
-    const float* __restrict__ abuf, float* __restrict__ gin, float* __restrict__ gE, int n) {
+    float* __restrict__ gin, float* __restrict__ gE, float* __restrict__ nu_part, int n) {
   using L = Layout<D>;
   constexpr int NPB = Geo<D>::kNodesPerBlock, TN = Geo<D>::kTileNodes;
   __shared__ float4 vt[TN];
   __shared__ float4 gt[TN];
+  __shared__ float red[kThreads / 64];
+  float nu_acc = 0.0f;
   for (XcdItems it(totals[kTotChunks], kSpreadChunks); it.valid(); it.next()) {
     const int4 ck = chunks[it.c];
     int lb[3], lbl[3];
@@ -476,6 +654,8 @@ __global__ __launch_bounds__(kThreads) void k_p2g_adj(
     for (int j = ck.y + threadIdx.x; j < ck.z; j += kThreads) {  // the chunk, kThreads at a time
       const int p = perm[j];
       const int mat = pi[(int64_t)L::MAT * cap + p];
+      float A[3][3] = {{0}};
+      affine_matrix<D>(P, pf, cap, p, mat, A);
       float mass = P.p_mass;
       if (mat == kWater) mass *= P.water_density;
       float xp[3] = {0, 0, 0}, vp[3] = {0, 0, 0}, av[3] = {0, 0, 0}, xbo[3] = {0, 0, 0};
@@ -505,11 +685,6 @@ __global__ __launch_bounds__(kThreads) void k_p2g_adj(
         bspline_grad(fx[a], dw[a]);
         l[a] = base - b[a];
       }
-      float A[3][3] = {{0}};
-#pragma unroll
-      for (int a = 0; a < D; a++)
-#pragma unroll
-        for (int e = 0; e < D; e++) A[a][e] = abuf[(int64_t)(a * D + e) * cap + p];
       float vnew[3] = {0, 0, 0}, xg[3] = {0, 0, 0}, S[3] = {0, 0, 0};
       float Ab[3][3] = {{0}};
 #pragma unroll 1  // keeps the LDS loads of one z-layer in flight, not all 27
@@ -572,7 +747,8 @@ __global__ __launch_bounds__(kThreads) void k_p2g_adj(
 #pragma unroll
       for (int a = 0; a < D; a++)
 #pragma unroll
-        for (int e = 0; e < D; e++) gin[(int64_t)(L::C + a * D + e) * cap + p] = P.dx * Ab[a][e];
+        for (int e = 0; e < D; e++) Ab[a][e] *= P.dx;
+      constitutive_adjoint<D>(P, pf, cap, p, mat, gf, Ab, gin, gE, nu_acc);
     }
     __syncthreads();
   }
@@ -583,194 +759,6 @@ __global__ __launch_bounds__(kThreads) void k_p2g_adj(
     const int p = perm[j];
     for (int c = 0; c < L::NF; c++) gin[(int64_t)c * cap + p] = 0.0f;
     if (gE) gE[p] = 0.0f;
-  }
-}
-
-// Step 3 (per particle): the constitutive adjoint.  Reads Abar from gin's C
-// rows and writes Cbar, Fbar, Jpbar, Ebar and per-workgroup nu partials.
-template <int D>
-__global__ __launch_bounds__(kThreads) void k_adj_constitutive(
-    const Params* __restrict__ scenes, const int* __restrict__ slab,
-    const float* __restrict__ pf, const int* __restrict__ pi, int64_t cap,
-    const int* __restrict__ perm, const int* __restrict__ totals, const float* __restrict__ gf,
-    float* __restrict__ gin, float* __restrict__ gE, float* __restrict__ nu_part) {
-  using L = Layout<D>;
-  __shared__ float red[kThreads / 64];
-  float nu_acc = 0.0f;
-  const int nvalid = totals[kTotValid];
-  for (int j = blockIdx.x * kThreads + threadIdx.x; j < nvalid; j += gridDim.x * kThreads) {
-    const int p = perm[j];
-    const Params& P = scenes[pi[(int64_t)L::SCENE * cap + p]];
-    const int mat = pi[(int64_t)L::MAT * cap + p];
-    float C[3][3], F[3][3];
-    load_cf<D>(pf, cap, p, C, F);
-    const float Jp = pf[(int64_t)L::JP * cap + p];
-    const float E = P.youngs ? P.youngs[p] : 0.0f;
-    if (mat == kSnow || mat == kSand) {
-      float K[3][3] = {{0.0f}}, Fp[3][3] = {{0.0f}}, G[3][3] = {{0.0f}}, Fbo[3][3] = {{0.0f}};
-      float Cb[3][3] = {{0.0f}};
-#pragma unroll
-      for (int a = 0; a < D; a++)
-#pragma unroll
-        for (int e = 0; e < D; e++) {
-          K[a][e] = (a == e ? 1.0f : 0.0f) + P.dt * C[a][e];
-          const float abar = gin[(int64_t)(L::C + a * D + e) * cap + p];
-          Cb[a][e] = P.p_mass * abar;
-          G[a][e] = P.stress_scale * abar;
-          Fbo[a][e] = gf[(int64_t)(L::F + a * D + e) * cap + p];
-        }
-#pragma unroll
-      for (int a = 0; a < D; a++)
-#pragma unroll
-        for (int e = 0; e < D; e++) {
-          float s = 0.0f;
-#pragma unroll
-          for (int k = 0; k < D; k++) s += K[a][k] * F[k][e];
-          Fp[a][e] = s;
-        }
-      float Fpb[3][3], Jpbar, mu0b, la0b, cb;
-      plastic_adjoint<D>(P, mat, Fp, Jp, P.youngs ? E * P.kmu : P.mu_0,
-                         P.youngs ? E * P.kla : P.lambda_0, G, Fbo,
-                         gf[(int64_t)L::JP * cap + p], Fpb, Jpbar, mu0b, la0b, cb);
-      // F' = K F: Fbar = K^T F'bar, Cbar += dt F'bar F^T
-#pragma unroll
-      for (int a = 0; a < D; a++)
-#pragma unroll
-        for (int e = 0; e < D; e++) {
-          float fb = 0.0f, t = 0.0f;
-#pragma unroll
-          for (int k = 0; k < D; k++) {
-            fb += K[k][a] * Fpb[k][e];
-            t += Fpb[a][k] * F[e][k];
-          }
-          gin[(int64_t)(L::C + a * D + e) * cap + p] = Cb[a][e] + P.dt * t;
-          gin[(int64_t)(L::F + a * D + e) * cap + p] = fb;
-        }
-      gin[(int64_t)L::JP * cap + p] = Jpbar;
-      // mu_0 = E kmu, lambda_0 = E kla; sand's coefficient depends on nu
-      if (gE) gE[p] = P.kmu * mu0b + P.kla * la0b;
-      nu_acc += E * (P.dkmu * mu0b + P.dkla * la0b) + cb * P.dsand_coef * P.alpha;
-      continue;
-    }
-    Recompute<D> r;
-    recompute<D>(P, mat, C, F, Jp, E, r);
-    float Cbar[3][3] = {{0}}, G[3][3] = {{0}}, Fbo[3][3] = {{0}};
-#pragma unroll
-    for (int a = 0; a < D; a++)
-#pragma unroll
-      for (int e = 0; e < D; e++) {
-        const float abar = gin[(int64_t)(L::C + a * D + e) * cap + p];
-        Cbar[a][e] = r.mass * abar;
-        G[a][e] = P.stress_scale * abar;
-        Fbo[a][e] = gf[(int64_t)(L::F + a * D + e) * cap + p];
-      }
-    const float Jpbo = gf[(int64_t)L::JP * cap + p];
-    float trG = 0.0f;
-#pragma unroll
-    for (int a = 0; a < D; a++) trG += G[a][a];
-    const float J = r.J;
-    const float labar = trG * J * (J - 1.0f);
-    float Jbar = r.la * trG * (2.0f * J - 1.0f);
-    float Fbar[3][3] = {{0}}, Jpbar, mubar = 0.0f;
-    if (r.water) {
-      Jbar += Fbo[0][0] + Jpbo;
-      const float detK = det_d<D>(r.K);
-      float cK[3][3];
-      cofactor_d<D>(r.K, cK);
-      Jpbar = Jbar * detK;
-#pragma unroll
-      for (int a = 0; a < D; a++)
-#pragma unroll
-        for (int e = 0; e < D; e++) Cbar[a][e] += Jbar * Jp * P.dt * cK[a][e];
-    } else {
-      const float mu = r.mu;
-      float Fpb[3][3], Rb[3][3];
-      {
-        float cF[3][3];
-        cofactor_d<D>(r.Fp, cF);
-#pragma unroll
-        for (int a = 0; a < D; a++)
-#pragma unroll
-          for (int e = 0; e < D; e++) {
-            float gfp = 0.0f, gtt = 0.0f, tft = 0.0f;
-#pragma unroll
-            for (int k = 0; k < D; k++) {
-              gfp += G[a][k] * r.Fp[k][e];                          // (G F')_ae
-              gtt += G[k][a] * (r.Fp[k][e] - r.R[k][e]);            // (G^T (F' - R))_ae
-              tft += (r.Fp[a][k] - r.R[a][k]) * r.Fp[e][k];         // ((F' - R) F'^T)_ae
-            }
-            mubar += 2.0f * G[a][e] * tft;
-            Fpb[a][e] = Fbo[a][e] + 2.0f * mu * (gfp + gtt) + Jbar * cF[a][e];
-            Rb[a][e] = -2.0f * mu * gfp;
-          }
-      }
-      // polar adjoint: B = U^T Rb V, Mbar = skew(B) / (sig_i + sig_j), F'bar += U Mbar V^T
-      float Bm[3][3];
-#pragma unroll
-      for (int a = 0; a < D; a++)
-#pragma unroll
-        for (int e = 0; e < D; e++) {
-          float t[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll
-          for (int m2 = 0; m2 < D; m2++)
-#pragma unroll
-            for (int k = 0; k < D; k++) t[m2] += r.U[k][a] * Rb[k][m2];
-          float s = 0.0f;
-#pragma unroll
-          for (int m2 = 0; m2 < D; m2++) s += t[m2] * r.V[m2][e];
-          Bm[a][e] = s;
-        }
-      float Mb[3][3];
-#pragma unroll
-      for (int a = 0; a < D; a++)
-#pragma unroll
-        for (int e = 0; e < D; e++) {
-          if (a == e) {
-            Mb[a][e] = 0.0f;
-          } else {
-            float den = r.sig[a] + r.sig[e];
-            if (fabsf(den) < 1e-6f) den = den < 0.0f ? -1e-6f : 1e-6f;
-            Mb[a][e] = (Bm[a][e] - Bm[e][a]) / den;
-          }
-        }
-#pragma unroll
-      for (int a = 0; a < D; a++)
-#pragma unroll
-        for (int e = 0; e < D; e++) {
-          float s = 0.0f;
-#pragma unroll
-          for (int k = 0; k < D; k++)
-#pragma unroll
-            for (int m2 = 0; m2 < D; m2++) s += r.U[a][k] * Mb[k][m2] * r.V[e][m2];
-          Fpb[a][e] += s;
-        }
-      // F' = K F: Fbar = K^T F'bar, Cbar += dt F'bar F^T
-#pragma unroll
-      for (int a = 0; a < D; a++)
-#pragma unroll
-        for (int e = 0; e < D; e++) {
-          float s = 0.0f, t = 0.0f;
-#pragma unroll
-          for (int k = 0; k < D; k++) {
-            s += r.K[k][a] * Fpb[k][e];
-            t += Fpb[a][k] * F[e][k];
-          }
-          Fbar[a][e] = s;
-          Cbar[a][e] += P.dt * t;
-        }
-      Jpbar = Jpbo;
-    }
-    // mu = h E kmu, la = h E kla
-    if (gE) gE[p] = r.h * (P.kmu * mubar + P.kla * labar);
-    nu_acc += r.h * E * (P.dkmu * mubar + P.dkla * labar);
-#pragma unroll
-    for (int a = 0; a < D; a++)
-#pragma unroll
-      for (int e = 0; e < D; e++) {
-        gin[(int64_t)(L::C + a * D + e) * cap + p] = Cbar[a][e];
-        gin[(int64_t)(L::F + a * D + e) * cap + p] = Fbar[a][e];
-      }
-    gin[(int64_t)L::JP * cap + p] = Jpbar;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) nu_acc += __shfl_xor(nu_acc, off);

@@ -154,7 +154,7 @@ void launch_front(const Params* P, const int* slab, SubstepBuffers& B, int raw_g
 // persistent_groups floats.
 template <int D>
 void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const float* pf_in,
-                    const float* gout, float* gin, float* gE, float4* gbar, float* abuf,
+                    const float* gout, float* gin, float* gE, float4* gbar,
                     float* nu_part, float* gnu, hipStream_t st, Timer* timer);
 
 // Block keys in sorted order (of the binning whose chunks and totals are given).

@@ -1854,19 +1854,13 @@ void launch_substep_half(const Params* P, const int* slab, SubstepBuffers& B, in
 
 template <int D>
 void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const float* pf_in,
-                    const float* gout, float* gin, float* gE, float4* gbar, float* abuf,
+                    const float* gout, float* gin, float* gE, float4* gbar,
                     float* nu_part, float* gnu, hipStream_t st, Timer* tm) {
   const int n = B.n;
   const int G = B.persistent_groups;
   const int chunk_bound = n > 0 ? std::min(B.total_blocks, n) + div_up(n, B.chunk) : 1;
   const int groups = xcd_groups(chunk_bound, G);
-  const int pgroups = clamp_groups(div_up(n, kThreads), G);
   if (n > 0) {
-    {
-      TimerScope ts(tm, "k_adj_affine", st);
-      k_adj_affine<D><<<pgroups, kThreads, 0, st>>>(P, slab, pf_in, B.pi, B.cap, B.perm,
-                                                    B.totals, abuf);
-    }
     {
       TimerScope ts(tm, "k_g2p_adj_scatter", st);
       k_p2g<D, 1><<<groups, kThreads, 0, st>>>(P, slab, pf_in, B.pi, B.cap, B.perm, B.chunks,
@@ -1883,17 +1877,12 @@ void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const f
     {
       TimerScope ts(tm, "k_p2g_adj", st);
       k_p2g_adj<D><<<groups, kThreads, 0, st>>>(P, slab, pf_in, B.pi, B.cap, B.perm, B.chunks,
-                                                B.totals, B.grid, gbar, gout, abuf, gin, gE, n);
-    }
-    {
-      TimerScope ts(tm, "k_adj_constitutive", st);
-      k_adj_constitutive<D><<<pgroups, kThreads, 0, st>>>(P, slab, pf_in, B.pi, B.cap, B.perm,
-                                                          B.totals, gout, gin, gE, nu_part);
+                                                B.totals, B.grid, gbar, gout, gin, gE, nu_part, n);
     }
   } else {
-    launch_fill_u32((unsigned*)nu_part, 0u, pgroups, st);
+    launch_fill_u32((unsigned*)nu_part, 0u, groups, st);
   }
-  k_sum_partials<<<1, kThreads, 0, st>>>(nu_part, pgroups, gnu);
+  k_sum_partials<<<1, kThreads, 0, st>>>(nu_part, groups, gnu);
 }
 
 void launch_sorted_keys(const int4* chunks, const int* totals, int n, int total_blocks, int* keys,
@@ -2214,11 +2203,11 @@ template void launch_front<2>(const Params*, const int*, SubstepBuffers&, int, h
 template void launch_front<3>(const Params*, const int*, SubstepBuffers&, int, hipStream_t,
                               Timer*);
 template void launch_adjoint<2>(const Params*, const int*, SubstepBuffers&, const float*,
-                                const float*, float*, float*, float4*, float*, float*, float*,
-                                hipStream_t, Timer*);
+                                const float*, float*, float*, float4*, float*, float*, hipStream_t,
+                                Timer*);
 template void launch_adjoint<3>(const Params*, const int*, SubstepBuffers&, const float*,
-                                const float*, float*, float*, float4*, float*, float*, float*,
-                                hipStream_t, Timer*);
+                                const float*, float*, float*, float4*, float*, float*, hipStream_t,
+                                Timer*);
 template void launch_substep<2>(const Params*, const int*, SubstepBuffers&, int, int, hipStream_t,
                                 Timer*);
 template void launch_substep<3>(const Params*, const int*, SubstepBuffers&, int, int, hipStream_t,

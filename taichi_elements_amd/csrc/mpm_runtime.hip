@@ -211,7 +211,6 @@ struct mpm_solver {
   int* diff_pi = nullptr;          // 3 x diff_n: material, insertion index, scene 0
   float* diff_scratch = nullptr;   // NF x diff_n: the state p2g rewrites in backward
   float4* diff_gbar = nullptr;     // grid adjoint
-  float* diff_abuf = nullptr;      // D*D x diff_n: affine matrices of the backward
   float* diff_nu_part = nullptr;   // per-workgroup nu adjoints
   bool diff_params_valid = false;  // the device scene table holds these values:
   float diff_dt = 0.0f;
@@ -1086,7 +1085,6 @@ int mpm_destroy(mpm_solver* s) {
   dfree(s->diff_pi);
   dfree(s->diff_scratch);
   dfree(s->diff_gbar);
-  dfree(s->diff_abuf);
   dfree(s->diff_nu_part);
   if (s->h_params) hipHostFree(s->h_params);
   if (s->own_words) hipHostFree(s->own_words);
@@ -1703,14 +1701,12 @@ int mpm_diff_setup(mpm_solver* s, int64_t n, const int32_t* material) {
   dfree(s->diff_pi);
   dfree(s->diff_scratch);
   dfree(s->diff_gbar);
-  dfree(s->diff_abuf);
   dfree(s->diff_nu_part);
   const int NPB = s->D == 3 ? Geo<3>::kNodesPerBlock : Geo<2>::kNodesPerBlock;
   TRY(dalloc(&s->diff_pi, 3 * n));
   TRY(dalloc(&s->diff_scratch, (int64_t)s->nf() * n));
   TRY(dalloc(&s->diff_gbar, (int64_t)s->total_blocks * NPB));
   TRY(dalloc(&s->diff_nu_part, s->persistent_groups));
-  TRY(dalloc(&s->diff_abuf, (int64_t)s->D * s->D * n));
   std::vector<int32_t> host(3 * n);
   for (int64_t i = 0; i < n; i++) {
     host[i] = material[i];
@@ -2156,10 +2152,10 @@ int mpm_diff_substep_backward(mpm_solver* s, float dt, const float* state_in,
   }
   if (s->D == 3)
     launch_adjoint<3>(s->d_params, slab_table(s), B, state_in, grad_out, grad_in, grad_youngs,
-                      s->diff_gbar, s->diff_abuf, s->diff_nu_part, grad_nu, st, nullptr);
+                      s->diff_gbar, s->diff_nu_part, grad_nu, st, nullptr);
   else
     launch_adjoint<2>(s->d_params, slab_table(s), B, state_in, grad_out, grad_in, grad_youngs,
-                      s->diff_gbar, s->diff_abuf, s->diff_nu_part, grad_nu, st, nullptr);
+                      s->diff_gbar, s->diff_nu_part, grad_nu, st, nullptr);
   if (!binning) {  // the block scan ran: keep the substep-parity bookkeeping
     take_buffers(s, B);
     s->substep_counter++;
