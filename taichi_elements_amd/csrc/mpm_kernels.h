@@ -16,6 +16,7 @@ constexpr int kChunkMax = 1024;  // particles per transfer work item (max), kBat
 // they are spread very thinly): work that each chunk adds to a transfer then
 // costs its latency once, less than a kernel of its own.
 constexpr int kOneRound = 160 * 1024;
+constexpr int kFewChunks = 2560;  // chunks up to which g2p runs the grid operator (k_g2p)
 constexpr int kScanItems = 2;                       // per thread in the block scan
 constexpr int kScanTile = kThreads * kScanItems;    // 512 blocks per workgroup
 constexpr int kScanTilesOnePass = 512;  // the single-pass scan's most tiles, all resident at once
@@ -186,8 +187,8 @@ void launch_scatter_i(const int* src, int64_t cap, int ncomp, const int* orig, i
 void launch_particle_info(int D, bool quant, bool g2p2g, const float* pf, const int* pi,
                           int64_t cap, int n, float* x, float* v, int* mat, hipStream_t st);
 // out[r] = max of part[r * stride .. + stride), r < rows; out[rows] = *err.
-void launch_max_rows(const unsigned* part, int rows, int stride, const int* err, unsigned* out,
-                     hipStream_t st);
+void launch_max_rows(const unsigned* part, int rows, int stride, const int* err,
+                     const int* totals, unsigned* out, hipStream_t st);
 void launch_fill_u32(unsigned* p, unsigned v, int64_t n, hipStream_t st);
 // svd3 / svd2 on n row-major dim x dim matrices (tests of the device SVD).
 void launch_svd_batch(int dim, const float* A, float* U, float* sig, float* V, int64_t n,

@@ -1068,10 +1068,14 @@ __global__ __launch_bounds__(kThreads) void k_grid_op(const Params* __restrict__
 // TILES: the grid operator runs in here.  The workgroup sums the p2g tiles
 // that reach its (4+2)^d nodes itself, in k_grid_op's order (bitwise the same
 // velocities), instead of reading them from the grid: every node is summed by
-// up to 2^d workgroups, out of L2, and a kernel and the grid's round trip
-// through memory go.  Taken in 2D up to kOneRound particles: 20k, g2p 4.8 +
-// grid operator 4.3 -> 6.6 us; at 400k in 2D 22.6 -> 24.6, in 3D 15.4 -> 14.4
-// (50k, no gain over the present grid operator), 51 -> 84 us (1M).
+// up to 2^d workgroups, out of L2, and a kernel, its launch and the grid's
+// round trip through memory go.  Taken up to kOneRound particles in up to
+// kFewChunks chunks, that is while the workgroups run at once; substeps with
+// the grid operator apart and inside: 2D 20k (143 chunks) 21.5 -> 19.0 us; 3D
+// 2000 particles 33.6 -> 31.6, 30k 37.7 -> 34.8, 100k (593 chunks) 43.9 ->
+// 41.4, 160k (855) 48.7 -> 45.8, 100k in 1872 chunks 52.4 -> 51.9, but 250k
+// 64.2 -> 66.8, and spread thinly 50k in 2975 chunks 60.2 -> 61.5, 100k in 8687
+// 138 -> 153, in 2D 20k in 10289 chunks 87.6 -> 94.2.
 template <int D, bool Q = false, int W = 1, bool TILES = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) void k_g2p(const Params* __restrict__ scenes,
                                                   const int* __restrict__ slab,
@@ -1525,13 +1529,17 @@ __global__ __launch_bounds__(kThreads) void k_particle_info(const float* __restr
 }
 
 // Largest |v| of each substep (one workgroup) from its per-workgroup maxima
-// (float bits); the last workgroup copies the error bits behind them.  out is
-// pinned host memory.
+// (float bits); the last workgroup copies the error bits and the number of
+// chunks behind them.  out is pinned host memory.
 __global__ __launch_bounds__(kThreads) void k_max_rows(const unsigned* __restrict__ part,
                                                        int stride, const int* __restrict__ err,
+                                                       const int* __restrict__ totals,
                                                        unsigned* __restrict__ out) {
   if (blockIdx.x == gridDim.x - 1) {
-    if (threadIdx.x == 0) out[blockIdx.x] = (unsigned)*err;
+    if (threadIdx.x == 0) {
+      out[blockIdx.x] = (unsigned)*err;
+      out[blockIdx.x + 1] = (unsigned)totals[kTotChunks];
+    }
     return;
   }
   __shared__ unsigned red[kThreads / 64];
@@ -1963,9 +1971,9 @@ void launch_particle_info(int D, bool quant, bool g2p2g, const float* pf, const 
                               : k_particle_info<2, false, false>);
   kern<<<clamp_groups(div_up(n, kThreads), 8192), kThreads, 0, st>>>(pf, pi, cap, n, x, v, mat);
 }
-void launch_max_rows(const unsigned* part, int rows, int stride, const int* err, unsigned* out,
-                     hipStream_t st) {
-  k_max_rows<<<rows + 1, kThreads, 0, st>>>(part, stride, err, out);
+void launch_max_rows(const unsigned* part, int rows, int stride, const int* err,
+                     const int* totals, unsigned* out, hipStream_t st) {
+  k_max_rows<<<rows + 1, kThreads, 0, st>>>(part, stride, err, totals, out);
 }
 void launch_copy_segments(const CopySegments& S, hipStream_t st) {
   int64_t most = 0;

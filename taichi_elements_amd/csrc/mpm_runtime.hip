@@ -9,6 +9,7 @@
 // Colors never take part in a substep and stay on the host in insertion
 // order.
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -162,6 +163,9 @@ struct mpm_solver {
   unsigned* host_words = nullptr;
   unsigned* own_words = nullptr;
   int host_words_cap = 0;
+  // chunks of the last substep whose maxima were read (0: none yet): which of
+  // two equal ways the grid operator goes, never what it gives
+  std::atomic<int> chunks_seen{0};
   // read access to the particles: device staging in insertion order and the
   // copies to the caller's memory; read_mu: readers of one handle take turns
   std::mutex read_mu;
@@ -567,7 +571,8 @@ void end_buffers(mpm_solver* s, const SubstepBuffers& B) {
 int eager_substep(mpm_solver* s, int k, bool last, Timer* tm) {
   SubstepBuffers B;
   begin_buffers(s, B);
-  B.grid_in_g2p = !last && !s->g2p2g && !(s->debug & 1) && s->n <= kOneRound && s->D == 2;
+  B.grid_in_g2p = !last && !s->g2p2g && !(s->debug & 1) && s->n <= kOneRound &&
+                  s->chunks_seen <= kFewChunks;
   if (s->D == 3)
     launch_substep<3>(s->d_params, slab_table(s), B, k, s->debug & 1, s->stream, tm);
   else
@@ -1377,18 +1382,20 @@ int mpm_read_max_velocity(mpm_solver* s, int32_t nsub, float* out) {
   HIP_TRY(hipSetDevice(s->device));
   std::lock_guard<std::mutex> lock(s->read_mu);
   // reduced on the device, straight into pinned host memory with the error bits
-  if (s->host_words_cap < nsub + 1) {
+  if (s->host_words_cap < nsub + 2) {
     unsigned* more = nullptr;
-    if (hipHostMalloc((void**)&more, sizeof(unsigned) * (nsub + 1)) != hipSuccess)
+    if (hipHostMalloc((void**)&more, sizeof(unsigned) * (nsub + 2)) != hipSuccess)
       return fail(MPM_ENOMEM, "pinned host allocation failed");
     if (s->own_words) hipHostFree(s->own_words);
     s->host_words = s->own_words = more;
-    s->host_words_cap = nsub + 1;
+    s->host_words_cap = nsub + 2;
   }
-  launch_max_rows(s->maxv, nsub, s->persistent_groups, s->err, s->host_words, s->stream);
+  launch_max_rows(s->maxv, nsub, s->persistent_groups, s->err, s->totals + s->last_parity * 16,
+                  s->host_words, s->stream);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(s->stream));
   if (nsub > 0) std::memcpy(out, s->host_words, sizeof(float) * nsub);
+  s->chunks_seen = (int)s->host_words[nsub + 1];
   return report_errors(s, (int)s->host_words[nsub]);
 }
 

@@ -1,4 +1,4 @@
-"""The grid operator inside g2p (small 2D scenes, every substep of a call but
+"""The grid operator inside g2p (small scenes, every substep of a call but
 the last) against the grid operator kernel (a call of one substep): the sums
 take the same order, so state and grid are bitwise the same."""
 import numpy as np
@@ -35,11 +35,18 @@ def _scene(dim, res, n, chunk, **options):
     (2, 48, 20000, 1024, dict(quant=True)),
     (2, 128, LINE, 256, {}),
     (2, 128, LINE + 1, 256, {}),
+    (3, 16, 1, 256, {}),
     (3, 24, 20000, 64, {}),
+    (3, 32, 9001, 1024, dict(quant=True)),
+    (3, 96, LINE, 256, {}),
+    (3, 96, LINE + 1, 256, {}),
+    # more chunks than it is taken for, known after the first call
+    (2, 128, 60000, 16, {}),
+    (3, 48, 60000, 16, {}),
 ])
 def test_call_of_many_substeps_is_bitwise_single_substeps(dim, res, n, chunk, options):
     a, b = (_scene(dim, res, n, chunk, **options) for _ in range(2))
-    for count in (1, 5, 2):
+    for count in (5, 1, 3):
         a._run_substeps(count, a.default_dt)
         for _ in range(count):
             b._run_substeps(1, b.default_dt)
@@ -51,19 +58,20 @@ def test_call_of_many_substeps_is_bitwise_single_substeps(dim, res, n, chunk, op
             assert np.array_equal(p, q)
 
 
-def test_scenes_that_sit_out():
-    """A batch of 2D scenes, one of which sits the call out: it keeps its
+@pytest.mark.parametrize("dim", [2, 3])
+def test_scenes_that_sit_out(dim):
+    """A batch of scenes, one of which sits the call out: it keeps its
     state, the others advance as alone."""
     from taichi_elements_amd import MPMSolver, MPMSolverBatch
     rng = np.random.default_rng(5)
     parts = []
     for k in range(3):
         n = 1500 + 700 * k
-        parts.append((cube_particles(rng, n, [0.2, 0.2], [0.4, 0.3], 2),
-                      rng.uniform(-1, 1, (n, 2)).astype(np.float32),
+        parts.append((cube_particles(rng, n, [0.2] * dim, [0.4, 0.3, 0.4][:dim], dim),
+                      rng.uniform(-1, 1, (n, dim)).astype(np.float32),
                       rng.integers(0, 4, n).astype(np.int32)))
-    b = MPMSolverBatch([dict(res=(24 + 8 * k, ) * 2) for k in range(3)])
-    solos = [MPMSolver(res=(24 + 8 * k, ) * 2) for k in range(3)]
+    b = MPMSolverBatch([dict(res=(24 + 8 * k, ) * dim) for k in range(3)])
+    solos = [MPMSolver(res=(24 + 8 * k, ) * dim) for k in range(3)]
     for s, t, (x, v, m) in zip(b, solos, parts):
         for u in (s, t):
             u.read_restart(len(x), x, v, m, np.zeros(len(x), np.int32))
