@@ -230,6 +230,8 @@ struct CopySegments {
   int count;
 };
 void launch_copy_segments(const CopySegments& S, hipStream_t st);
+void launch_begin_call(const Params* host_table, Params* table, int scenes, unsigned* maxv,
+                       int64_t n, int* step, hipStream_t st);
 void launch_take_columns(const float* src, int64_t row_stride, int64_t col_stride,
                          const int64_t* index, float* dst, int rows, int64_t n, hipStream_t st);
 

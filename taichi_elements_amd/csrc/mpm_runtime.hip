@@ -1231,16 +1231,18 @@ static int prepare_substeps(mpm_solver* s, int32_t nsub, const float* dts, bool 
     TRY(dalloc(&s->maxv, (int64_t)nsub * s->persistent_groups));
     s->maxv_cap = nsub * s->persistent_groups;
   }
-  launch_fill_u32(s->maxv, 0u, (int64_t)std::max(nsub, 1) * s->persistent_groups, s->stream);
   s->last_batch = nsub;
-  if (s->n == 0) return MPM_OK;
+  const int64_t slots = (int64_t)std::max(nsub, 1) * s->persistent_groups;
+  if (s->n == 0) {
+    launch_fill_u32(s->maxv, 0u, slots, s->stream);
+    return MPM_OK;
+  }
   // scene table: the staging buffer is reused only once the last upload is done
   HIP_TRY(hipStreamSynchronize(s->stream));
   for (size_t k = 0; k < s->scenes.size(); k++)
     fill_params(s->h_params[k], s, s->scenes[k], dts[k], batch && dts[k] == 0.0f);
-  HIP_TRY(hipMemcpyAsync(s->d_params, s->h_params, sizeof(Params) * s->scenes.size(),
-                         hipMemcpyHostToDevice, s->stream));
-  launch_fill_u32((unsigned*)s->d_step, 0xFFFFFFFFu, 1, s->stream);  // slot k for substep k
+  launch_begin_call(s->h_params, s->d_params, (int)s->scenes.size(), s->maxv, slots, s->d_step,
+                    s->stream);
   return MPM_OK;
 }
 
