@@ -23,7 +23,14 @@
 // particles).  It takes the place of an offsets kernel over the blocks and a
 // scatter over the particles (6.4 + 6.5, 4.9 + 5.3 and 65 + 125 us), with the
 // key and code arrays between them; a workgroup per chunk instead of a wave
-// took 13.2, 10.6 and 151 us.
+// took 13.2, 10.6 and 151 us.  The line lies at kListsInTransfer particles
+// (kOneRound for the fused transfer) in kFewChunks chunks, as far as the
+// number is known: substeps with the lists walked by k_members and inside p2g
+// take 56.2 and 54.6 us at 200k particles in 1117 chunks (3D), 63.9 and 62.3 at
+// 250k in 1390, 84.3 and 84.9 at 500k in 2686; 38.1 and 37.0 at 250k in 2116
+// (2D), 51.7 and 55.1 at 400k in 4225; spread thinly 59.6 and 60.5 at 50k in
+// 2975 chunks, 129 and 138 at 100k in 8687, in 2D 38.0 and 42.2 at 60k in 3385,
+// 285 and 354 at 100k in 45096.
 #pragma once
 
 #include "mpm_device.h"

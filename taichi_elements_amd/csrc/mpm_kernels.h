@@ -12,11 +12,12 @@ namespace mpm {
 constexpr int kThreads = 256;
 constexpr int kBatch = kThreads;  // particles a transfer workgroup holds at a time
 constexpr int kChunkMax = 1024;  // particles per transfer work item (max), kBatch at a time
-// Up to this many particles a scene has about one chunk per workgroup (unless
-// they are spread very thinly): work that each chunk adds to a transfer then
-// costs its latency once, less than a kernel of its own.
-constexpr int kOneRound = 160 * 1024;
-constexpr int kFewChunks = 2560;  // chunks up to which g2p runs the grid operator (k_g2p)
+// Up to this many particles and chunks a scene has about one chunk per
+// workgroup: work that each chunk adds to a transfer then costs its latency
+// once, less than a kernel of its own.
+constexpr int kOneRound = 160 * 1024;         // the grid operator inside g2p (k_g2p)
+constexpr int kListsInTransfer = 256 * 1024;  // the walk of the direction lists (mpm_binning.h)
+constexpr int kFewChunks = 2560;              // both
 constexpr int kScanItems = 2;                       // per thread in the block scan
 constexpr int kScanTile = kThreads * kScanItems;    // 512 blocks per workgroup
 constexpr int kScanTilesOnePass = 512;  // the single-pass scan's most tiles, all resident at once
@@ -117,6 +118,7 @@ struct SubstepBuffers {
   int n_final;
   bool quant;         // packed particle layout (PackedLayout<D>)
   int nw;             // particle float-buffer words per slot
+  bool few_chunks;    // as far as is known there are at most kFewChunks
   bool count_zeroed;  // count holds zeros (full_sort clears it otherwise)
   bool full_sort;     // radix-sort the slots (first substep / positions set by the host)
 };

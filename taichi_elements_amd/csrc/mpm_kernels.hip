@@ -539,8 +539,8 @@ __global__ __launch_bounds__(kThreads) void k_onesweep(
 // seldom has a chunk, also writes k_bscan's results for the kernels after it.
 // Bound, like k_bscan, by round trips to memory, of which this is one instead
 // of a kernel's four: taken in 2D by steady-state substeps of windows of up to
-// kThreads kWindowItems blocks and up to kOneRound particles, where each
-// workgroup has about one chunk.  A kernel of 3.9 to 4.7 us and its launch
+// kThreads kWindowItems blocks whose transfer walks the direction lists, where
+// each workgroup has about one chunk.  A kernel of 3.9 to 4.7 us and its launch
 // go, p2g takes 3 to 4 us longer: a substep of 5000 particles (400 blocks)
 // 19.8 -> 17.5 us, 60000 (1369 blocks) 24.1 -> 23.1, 160000 (2025 blocks) 28.5
 // -> 27.4.  With the counts read by each thread where it needs them, without
@@ -1656,7 +1656,8 @@ static PrevBinning prev_binning(const SubstepBuffers& B) {
 // what each way costs).  A substep that moves the particles takes the given
 // order.
 static bool order_in_transfer(const SubstepBuffers& B) {
-  return !B.full_sort && !B.move && B.n <= kOneRound;
+  return !B.full_sort && !B.move && B.few_chunks &&
+         B.n <= (B.g2p2g ? kOneRound : kListsInTransfer);
 }
 
 // Whether p2g scans the block window itself (WindowScan says why there).

@@ -513,6 +513,7 @@ void fill_buffers(mpm_solver* s, SubstepBuffers& B) {
   B.lb_status_radix = s->lb_status_radix;
   B.radix_cap = s->radix_cap;
   B.count_zeroed = false;
+  B.few_chunks = s->chunks_seen <= kFewChunks;
   B.lbs = s->lbs;
   B.ghist = s->ghist;
   B.totals = s->totals + cur * 16;
@@ -574,7 +575,7 @@ int eager_substep(mpm_solver* s, int k, bool last, Timer* tm) {
   SubstepBuffers B;
   begin_buffers(s, B);
   B.grid_in_g2p = !last && !s->g2p2g && !(s->debug & 1) && s->n <= kOneRound &&
-                  s->chunks_seen <= kFewChunks;
+                  B.few_chunks;
   if (s->D == 3)
     launch_substep<3>(s->d_params, slab_table(s), B, k, s->debug & 1, s->stream, tm);
   else

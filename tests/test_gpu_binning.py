@@ -11,7 +11,8 @@ from tests.helpers import cube_particles
 
 pytestmark = pytest.mark.gpu
 
-LINE = 160 * 1024  # particles up to which the transfer walks the lists
+# particles up to which the transfer walks the lists (use_g2p2g, p2g)
+LINE, P2G_LINE = 160 * 1024, 256 * 1024
 
 
 @pytest.fixture(autouse=True)
@@ -31,6 +32,9 @@ CASES = [
     (3, 48, LINE, 0.4, 256, -1, {}),
     (3, 48, LINE + 1, 0.4, 256, -1, {}),
     (3, 48, LINE + 1, 0.2, 1000, 2, {}),
+    (3, 48, P2G_LINE, 0.5, 256, -1, {}),
+    (3, 48, P2G_LINE + 1, 0.5, 256, -1, {}),
+    (3, 48, 60000, 0.6, 16, -1, {}),  # more chunks than the transfer walks the lists for
     (3, 32, 9001, 0.3, 64, 2, dict(use_g2p2g=True)),
     (3, 48, LINE + 1, 0.4, 256, -1, dict(use_g2p2g=True)),
     (3, 32, 9001, 0.3, 64, 2, dict(quant=True)),

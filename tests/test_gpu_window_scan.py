@@ -11,7 +11,7 @@ from tests.helpers import cube_particles
 
 pytestmark = pytest.mark.gpu
 
-LINE = 160 * 1024  # particles up to which p2g walks the lists
+LINE = 256 * 1024  # particles up to which p2g walks the lists
 
 
 @pytest.fixture(autouse=True)
@@ -30,6 +30,7 @@ def _quiet():
     ((184, 184), 20000, 0.8, 256, {}),          # past the range
     ((160, 160), LINE, 0.8, 1024, {}),
     ((160, 160), LINE + 1, 0.8, 1000, {}),
+    ((128, 128), LINE, 0.9, 16, {}),            # more chunks than the lists are walked for
 ])
 def test_order_and_results(oracle, res, n, side, chunk, options):
     from taichi_elements_amd import MPMSolver
