@@ -17,6 +17,8 @@
 //                     normalisation, gravity, post-process              (mpm:586-692)
 //   k_g2p             per chunk: LDS tile of grid velocity, gather,
 //                     advection, max |v|, next binning's lists          (g2p, mpm:694-735)
+// Small scenes run the grid operator inside k_g2p, in 2D also the scan inside
+// k_p2g.
 // use_g2p2g replaces p2g / grid op / g2p with k_g2p2g + k_grid_op_g2p2g
 // (mpm_g2p2g.h); the differentiable backward runs the adjoints of
 // mpm_adjoint.h.  Particles are read and written through Particles<D, Q>
