@@ -1775,7 +1775,12 @@ static void launch_g2p2g(const Params* P, const int* slab, SubstepBuffers& B, in
     if (order_in_transfer(B))
       kern = B.quant ? k_g2p2g<D, true, kOrderLists> : k_g2p2g<D, false, kOrderLists>;
     if (B.move) kern = B.quant ? k_g2p2g<D, true, kOrderMove> : k_g2p2g<D, false, kOrderMove>;
-    kern<<<xcd_groups(chunk_bound, G), kThreads, 0, st>>>(
+    // In 3D no more workgroups than are resident at once (three per CU, by LDS)
+    // while each takes a few chunks: the rest would start in a second, uneven
+    // round (2048 and 768: 300k 68.4 and 66.3 us a substep, 600k thinly spread
+    // 101.8 and 98.7, 1M 132.3 and 132.6, with 4096 asked for 134 and 137).
+    const int resident = D == 3 && n <= 768 * 1024 ? std::min(G, 768) : G;
+    kern<<<xcd_groups(chunk_bound, resident), kThreads, 0, st>>>(
         P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.grid_in, B.tiles, B.n_final,
         B.maxv, B.step, B.persistent_groups, B.members, B.dseg, B.count_next, B.err,
         prev_binning(B), B.pstart, B.move ? B.pf_alt : B.pf, B.move ? B.pi_alt : nullptr, n, B.nw,

@@ -2051,7 +2051,10 @@ int mpm_diff_substep(mpm_solver* s, float dt, const float* state_in, float* stat
   // (3 us of 85).  Under capture there is always one: a replay may follow
   // anything.
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(st, &cap));
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess) {  // not for it to refuse the call
+    (void)hipGetLastError();
+    cap = hipStreamCaptureStatusActive;
+  }
   const bool eager = cap == hipStreamCaptureStatusNone;
   B.count_zeroed = eager && s->count_zeroed;
   s->count_zeroed = false;
