@@ -24,6 +24,10 @@
 // mpm_adjoint.h.  Particles are read and written through Particles<D, Q>
 // (mpm_particles.h), instantiated for the float and the packed layout.
 #include "mpm_kernels.h"
+
+#include <map>
+#include <mutex>
+
 #include "mpm_binning.h"
 #include "mpm_adjoint.h"
 #include "mpm_g2p2g.h"
@@ -1624,6 +1628,24 @@ static inline int xcd_groups(int64_t g, int cap) {
   return (int)std::min<int64_t>((std::max<int64_t>(g, 1) + 7) & ~7, cap & ~7);
 }
 
+// Workgroups of a kernel that the device holds at once.
+static int resident_groups(const void* kern) {
+  static std::mutex mu;
+  static std::map<const void*, int> known;
+  std::lock_guard<std::mutex> lock(mu);
+  const auto it = known.find(kern);
+  if (it != known.end()) return it->second;
+  int dev = 0, cus = 0, per_cu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kThreads, 0) != hipSuccess ||
+      cus * per_cu < 8) {
+    (void)hipGetLastError();
+    return 1024;
+  }
+  return known[kern] = cus * per_cu;
+}
+
 // Workgroups of the grid operators: a lane per node of the active blocks (at
 // most the window's, and 2^D per particle), as many as are resident at once.
 template <int D>
@@ -1850,7 +1872,15 @@ void launch_g2p(const Params* P, const int* slab, SubstepBuffers& B, int s_index
     if (B.grid_in_g2p)
       kern = B.g2p_waves >= 6 ? (B.quant ? k_g2p<D, true, 6, true> : k_g2p<D, false, 6, true>)
                               : (B.quant ? k_g2p<D, true, 1, true> : k_g2p<D, false, 1, true>);
-    kern<<<xcd_groups(chunk_bound, G), kThreads, 0, st>>>(
+    // In 3D no more workgroups than are resident at once (1280): with more, the
+    // ones that start in a second round leave the device uneven (2048 and 1280:
+    // substeps of 300k 66.6 and 65.0 us, 1M 117.5 and 116.3, 4M 419 and 405; 16M
+    // g2p 645 and 568).  No gain in 2D (60.8 and 61.8 us at 400k) and packed (1M
+    // 120.2 and 119.2; a frame of 778k 8.5 and 8.8 ms).
+    const int resident = D == 2 || B.quant || B.grid_in_g2p
+                             ? G
+                             : std::min(G, resident_groups((const void*)kern));
+    kern<<<xcd_groups(chunk_bound, resident), kThreads, 0, st>>>(
         P, slab, B.pf, B.pi, B.cap, B.perm, B.chunks, B.totals, B.grid,
         B.maxv, B.step, B.persistent_groups, B.members, B.dseg, B.count_next, B.err,
         B.pf_out, n, B.pchunk_begin, B.pchunk_cnt, B.tiles);
