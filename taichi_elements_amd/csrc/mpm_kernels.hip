@@ -556,7 +556,7 @@ struct WindowScan {
   const int* count;
   int* count_next;
   int total_blocks, chunk;
-  unsigned chunk_inv;  // ceil(2^32 / chunk): x / chunk for x < 2^32 / chunk
+  unsigned chunk_inv;  // ceil(2^32 / chunk): x / chunk for x < 2^32 / chunk, chunk > 1
   int *pstart, *pchunk_begin, *pchunk_cnt;
   int4* chunks;
   int *active, *totals, *ghist_next, *step;
@@ -1684,10 +1684,12 @@ static bool order_in_transfer(const SubstepBuffers& B) {
          B.n <= (B.g2p2g ? kOneRound : kListsInTransfer);
 }
 
-// Whether p2g scans the block window itself (WindowScan says why there).
+// Whether p2g scans the block window itself (WindowScan says why there).  Its
+// division by the chunk size is a multiplication by ceil(2^32 / chunk), which
+// for chunks of one particle does not fit 32 bits: those take k_bscan.
 template <int D>
 static bool scan_in_p2g(const SubstepBuffers& B) {
-  return D == 2 && order_in_transfer(B) && !B.g2p2g &&
+  return D == 2 && order_in_transfer(B) && !B.g2p2g && B.chunk > 1 &&
          B.total_blocks <= kThreads * kWindowItems;
 }
 
