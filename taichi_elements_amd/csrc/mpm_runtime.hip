@@ -144,6 +144,7 @@ struct mpm_solver {
   // buffers sized by the block window
   int* count = nullptr;
   bool count_zeroed = false;  // count holds zeros: the differentiable substep before cleared it
+  bool diff_captured = false; // a graph outside the handle's sight may write count (note_capture)
   int* count_next = nullptr;
   int* pstart = nullptr;
   int* pchunk_begin = nullptr;  // 2 x total_blocks (substep parity)
@@ -1800,6 +1801,19 @@ void diff_buffers(mpm_solver* s, SubstepBuffers& B, float* pf) {
   B.members = nullptr;
 }
 
+// A call that bins was captured into a graph: the handle does not see the
+// replays, which may come between any two of its calls and count in the arrays
+// that the graph holds.  So from then on every call clears its counts first,
+// as the captured one does.
+void note_capture(mpm_solver* s, hipStream_t st) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess) {  // not for it to refuse the call
+    (void)hipGetLastError();
+    cap = hipStreamCaptureStatusActive;
+  }
+  if (cap != hipStreamCaptureStatusNone) s->diff_captured = true;
+}
+
 }  // namespace
 
 int mpm_set_g2p2g(mpm_solver* s, int32_t enabled, double allowed_cfl, int32_t clamp) {
@@ -2048,15 +2062,9 @@ int mpm_diff_substep(mpm_solver* s, float dt, const float* state_in, float* stat
   if (binning) B.raw_out = (float4*)((char*)binning + bin_layout(s).grid);
   // A differentiable substep leaves the other count array cleared (its block
   // scan does that, and its g2p counts nothing), so the next one needs no fill
-  // (3 us of 85).  Under capture there is always one: a replay may follow
-  // anything.
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cap) != hipSuccess) {  // not for it to refuse the call
-    (void)hipGetLastError();
-    cap = hipStreamCaptureStatusActive;
-  }
-  const bool eager = cap == hipStreamCaptureStatusNone;
-  B.count_zeroed = eager && s->count_zeroed;
+  // (3 us of 85).
+  note_capture(s, st);
+  B.count_zeroed = s->count_zeroed && !s->diff_captured;
   s->count_zeroed = false;
   if (s->D == 3)
     launch_substep<3>(s->d_params, slab_table(s), B, 0, 0, st, nullptr);
@@ -2082,7 +2090,7 @@ int mpm_diff_substep(mpm_solver* s, float dt, const float* state_in, float* stat
   take_buffers(s, B);
   s->substep_counter++;
   HIP_TRY(hipGetLastError());
-  s->count_zeroed = eager;
+  s->count_zeroed = true;
   return MPM_OK;
 }
 
@@ -2157,6 +2165,7 @@ int mpm_diff_substep_backward(mpm_solver* s, float dt, const float* state_in,
     B.totals = (int*)(b + L.totals);
     B.grid = (float4*)(b + L.grid);
   } else {
+    note_capture(s, st);
     if (s->D == 3)
       launch_front<3>(s->d_params, slab_table(s), B, 1, st, nullptr);
     else
