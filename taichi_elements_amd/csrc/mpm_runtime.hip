@@ -1382,6 +1382,7 @@ int mpm_substep_end(mpm_solver* s) {
 int mpm_read_max_velocity(mpm_solver* s, int32_t nsub, float* out) {
   if (!s || (!out && nsub > 0)) return fail(MPM_EINVAL, "null argument");
   if (nsub > s->last_batch) return fail(MPM_EINVAL, "more entries than substeps run");
+  nsub = std::max(nsub, 0);  // none wanted: the wait and the error bits alone
   HIP_TRY(hipSetDevice(s->device));
   std::lock_guard<std::mutex> lock(s->read_mu);
   // reduced on the device, straight into pinned host memory with the error bits
