@@ -96,6 +96,7 @@ class _Reorder(torch.autograd.Function):
     @staticmethod
     def forward(ctx, t, solver, index, inverse):
         ctx.solver, ctx.index, ctx.inverse = solver, index, inverse
+        t = t.resolve_neg()  # a lazily negated view: the kernel reads its memory as it is
         out = torch.empty(t.shape, dtype=t.dtype, device=t.device)
         rows, row_stride = (t.shape[0], t.stride(0)) if t.dim() == 2 else (1, 0)
         check(_lib.lib().mpm_diff_reorder(solver._handle, _ptr(t), row_stride, t.stride(-1),
