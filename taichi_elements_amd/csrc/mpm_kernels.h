@@ -20,9 +20,15 @@ constexpr int kListsInTransfer = 256 * 1024;  // the walk of the direction lists
 constexpr int kFewChunks = 2560;              // both
 constexpr int kScanItems = 2;                       // per thread in the block scan
 constexpr int kScanTile = kThreads * kScanItems;    // 512 blocks per workgroup
-constexpr int kScanTilesOnePass = 512;  // the single-pass scan's most tiles, all resident at once
+// The single-pass scan's most tiles.  A tile waits for those before it, which
+// the hardware may start later on another XCD, so scans of other streams must
+// not be able to fill an XCD with waiting tiles: three of them (a process has
+// four hardware queues) leave 24 of an XCD's 192 places free.
+constexpr int kScanTilesOnePass = 448;
 // Keys per workgroup of a sort pass: kRadixTile, or, while they make no more
-// than kRadixSmallTiles tiles, kRadixSmallTile (k_onesweep says why).
+// than kRadixSmallTiles tiles, kRadixSmallTile (k_onesweep says why).  The
+// small tiles wait for each other as the scan's do, 16 on each XCD with places
+// for 128; the others are numbered as they start (lb_acquire).
 constexpr int kRadixItems = 16, kRadixSmallItems = 8;
 constexpr int kRadixTile = kThreads * kRadixItems;
 constexpr int kRadixSmallTile = kThreads * kRadixSmallItems;

@@ -172,13 +172,17 @@ __device__ __forceinline__ int4 block_values(int bid, const int* __restrict__ co
 // Status word: value in bits 0-31, flag in bits 32-33 (1 = tile aggregate,
 // 2 = inclusive prefix), launch epoch in bits 34-63.  Words left by earlier
 // launches carry an older epoch and read as "not ready", so the status
-// arrays are never cleared.  Tiles are numbered in the order workgroups start
-// (an atomic ticket), so a tile only waits on tiles that are already running;
-// the last workgroup to finish resets the ticket and advances the epoch,
-// which keeps the kernels free of host-side per-launch state.
+// arrays are never cleared.  Past kRadixSmallTiles tiles they are numbered in
+// the order workgroups start (an atomic ticket), so a tile only waits on tiles
+// that are already running; the last workgroup to finish resets the ticket and
+// advances the epoch, which keeps the kernels free of host-side per-launch
+// state.
 // ---------------------------------------------------------------------------
 constexpr unsigned long long kFlagAgg = 1ull << 32, kFlagPre = 2ull << 32;
-constexpr int kSpinLimit = 1 << 18;
+// Polls (of a microsecond or more) after which a wait for another tile gives
+// up: seconds, because a tile that is not running yet starts only when other
+// work on the device makes room for it.
+constexpr int kWaitLimit = 1 << 22;
 
 __device__ __forceinline__ unsigned long long lb_epoch_bits(unsigned epoch) {
   return (unsigned long long)(epoch & 0x3fffffffu) << 34;
@@ -191,7 +195,7 @@ __device__ __forceinline__ void lb_publish(unsigned long long* p, unsigned long 
 }
 
 // Exclusive prefix of channel `chan` for tile `tile` (status[t * stride + chan]).
-// A bounded wait: past kSpinLimit polls it flags err bit 1 and returns what it has.
+// A bounded wait: past kWaitLimit polls it flags err bit 1 and returns what it has.
 __device__ __forceinline__ unsigned lb_lookback(const unsigned long long* status, int stride,
                                                 int tile, int chan, unsigned epoch, int* err) {
   constexpr int W = 8;  // predecessors read at once: one round trip, not eight in turn
@@ -219,7 +223,7 @@ __device__ __forceinline__ unsigned lb_lookback(const unsigned long long* status
     if (done) break;
     t -= used;
     if (used < W) {
-      if (++spins > kSpinLimit) {
+      if (++spins > kWaitLimit) {
         atomicOr(err, 2);
         return excl;
       }
@@ -234,10 +238,11 @@ struct LBTicket {
   unsigned epoch;
 };
 
-// Tiles that are all resident at once need no ticket to be sure that their
-// predecessors run; the epoch changes only after every tile has read it.
+// A few tiles find room on the device whatever else runs there and take no
+// ticket (a round trip more: 200k keys 12.5 us a pass, 11.0 without); the epoch
+// changes only after every tile has read it.
 __device__ __forceinline__ LBTicket lb_acquire(LBState* st, LBTicket* sh, int ntiles) {
-  if (ntiles <= kScanTilesOnePass)
+  if (ntiles <= kRadixSmallTiles)
     return {(int)blockIdx.x,
             __hip_atomic_load(&st->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
   if (threadIdx.x == 0) {
@@ -266,12 +271,11 @@ __device__ __forceinline__ void lb_release(LBState* st, int ntiles, unsigned epo
 // outside the window, whose key is total_blocks).
 //
 // Bound by its chain of dependent round trips to memory: the counts, then the
-// other tiles' sums.  Up to kScanTilesOnePass tiles, all of them resident at
-// once, every tile publishes its four sums and adds up those of all tiles
-// before it (one wave per sum, eight words per lane): nobody waits for
-// somebody else's prefix.  status[tile][channel] holds kScanReady | sum and is
-// cleared by the substep's first transfer, so there is no ticket, no epoch
-// and no release.  With tickets, a look-back over prefixes and each
+// other tiles' sums.  Up to kScanTilesOnePass tiles every tile publishes its
+// four sums and adds up those of all tiles before it (one wave per sum, seven
+// words per lane): nobody waits for somebody else's prefix.
+// status[tile][channel] holds kScanReady | sum and is cleared by the substep's
+// first transfer, so there is no ticket, no epoch and no release.  With tickets, a look-back over prefixes and each
 // neighbour's count loaded behind a branch: 1M particles (99 tiles) 11.8 ->
 // 7.0 us, 2D 20k 6.1 -> 4.6, unbounded 50k 16.4 -> 7.8, use_g2p2g 300k 13.9 ->
 // 8.1.  Larger windows take the tile sums from k_bscan_reduce, every tile
@@ -282,9 +286,8 @@ constexpr unsigned long long kScanReady = 1ull << 32;
 
 // Sum of channel c of the tiles before `tile`, by one wave.  Tiles that are
 // not running yet (other work holds the device) start as that work ends, so
-// the wait is long but bounded: past kScanSpinLimit polls (seconds) it flags
-// err bit 1 and counts what it has.
-constexpr int kScanSpinLimit = 1 << 22;
+// the wait is long but bounded: past kWaitLimit polls it flags err bit 1 and
+// counts what it has.
 __device__ __forceinline__ unsigned scan_before(const unsigned long long* status, int tile, int c,
                                                 int* err) {
   constexpr int W = kScanTilesOnePass / 64;
@@ -302,7 +305,7 @@ __device__ __forceinline__ unsigned scan_before(const unsigned long long* status
       ready &= (w[j] & kScanReady) != 0;
     }
     if (__all(ready)) break;
-    if (spins > kScanSpinLimit) {
+    if (spins > kWaitLimit) {
       atomicOr(err, 2);
       break;
     }
