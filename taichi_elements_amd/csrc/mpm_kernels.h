@@ -145,6 +145,11 @@ template <int D>
 void launch_substep_half(const Params* P, const int* slab, SubstepBuffers& B, int substep_index,
                          int half, hipStream_t st, Timer* timer);
 
+// grid operator on the binning and the p2g tiles already in B
+template <int D>
+void launch_grid_op(const Params* P, const int* slab, const SubstepBuffers& B, int raw_grid,
+                    hipStream_t st, Timer* timer);
+
 // p2g + grid operator on the binning already in B
 template <int D>
 void launch_transfer(const Params* P, const int* slab, SubstepBuffers& B, int raw_grid,

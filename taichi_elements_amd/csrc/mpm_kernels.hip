@@ -1822,6 +1822,15 @@ static void launch_g2p2g(const Params* P, const int* slab, SubstepBuffers& B, in
   std::swap(B.count, B.count_next);
 }
 
+template <int D>
+void launch_grid_op(const Params* P, const int* slab, const SubstepBuffers& B, int raw,
+                    hipStream_t st, Timer* tm) {
+  TimerScope ts(tm, "k_grid_op", st);
+  k_grid_op<D, 0><<<grid_op_groups<D>(B), kThreads, 0, st>>>(
+      P, slab, B.active, B.totals, B.pchunk_begin, B.pchunk_cnt, B.tiles, B.grid, raw, nullptr,
+      B.raw_out);
+}
+
 // p2g and the grid operator on an existing binning
 template <int D>
 void launch_transfer(const Params* P, const int* slab, SubstepBuffers& B, int raw, hipStream_t st,
@@ -1853,12 +1862,7 @@ void launch_transfer(const Params* P, const int* slab, SubstepBuffers& B, int ra
         B.nw, B.err, scan_status(B), window_scan(B));
     if (B.move) take_moved(B);
   }
-  if (!B.grid_in_g2p) {
-    TimerScope ts(tm, "k_grid_op", st);
-    k_grid_op<D, 0><<<grid_op_groups<D>(B), kThreads, 0, st>>>(
-        P, slab, B.active, B.totals, B.pchunk_begin, B.pchunk_cnt, B.tiles, B.grid, raw, nullptr,
-        B.raw_out);
-  }
+  if (!B.grid_in_g2p) launch_grid_op<D>(P, slab, B, raw, st, tm);
 }
 
 // g2p of one substep (after launch_front); the max-velocity slot is the
@@ -2271,6 +2275,10 @@ template void launch_transfer<2>(const Params*, const int*, SubstepBuffers&, int
                                  Timer*);
 template void launch_transfer<3>(const Params*, const int*, SubstepBuffers&, int, hipStream_t,
                                  Timer*);
+template void launch_grid_op<2>(const Params*, const int*, const SubstepBuffers&, int, hipStream_t,
+                                Timer*);
+template void launch_grid_op<3>(const Params*, const int*, const SubstepBuffers&, int, hipStream_t,
+                                Timer*);
 template void launch_front<2>(const Params*, const int*, SubstepBuffers&, int, hipStream_t,
                               Timer*);
 template void launch_front<3>(const Params*, const int*, SubstepBuffers&, int, hipStream_t,

@@ -571,7 +571,8 @@ void end_buffers(mpm_solver* s, const SubstepBuffers& B) {
 // One substep launched kernel by kernel (also what a graph captures).  last:
 // the last substep of a call, which leaves the grid for its readers
 // (mpm_read_grid, mpm_max_grid_velocity); the others need no grid in memory
-// and run the grid operator inside g2p where that is faster (k_g2p's TILES).
+// and run the grid operator inside g2p where that is faster (k_g2p's TILES;
+// finish_grid where a call stops before its last substep).
 int eager_substep(mpm_solver* s, int k, bool last, Timer* tm) {
   SubstepBuffers B;
   begin_buffers(s, B);
@@ -583,6 +584,21 @@ int eager_substep(mpm_solver* s, int k, bool last, Timer* tm) {
     launch_substep<2>(s->d_params, slab_table(s), B, k, s->debug & 1, s->stream, tm);
   end_buffers(s, B);
   return MPM_OK;
+}
+
+// The grid of the last substep from its binning and tiles, where a call ends
+// early: its substeps so far may have kept the grid inside g2p.
+void finish_grid(mpm_solver* s) {
+  if (s->g2p2g || s->n == 0) return;
+  SubstepBuffers B;
+  fill_buffers(s, B);
+  B.pchunk_begin = B.pchunk_begin_prev;
+  B.pchunk_cnt = B.pchunk_cnt_prev;
+  B.totals = s->totals + s->last_parity * 16;
+  if (s->D == 3)
+    launch_grid_op<3>(s->d_params, slab_table(s), B, s->debug & 1, s->stream, nullptr);
+  else
+    launch_grid_op<2>(s->d_params, slab_table(s), B, s->debug & 1, s->stream, nullptr);
 }
 
 // The next two substeps can run as one HIP graph: binning by the
@@ -1261,7 +1277,10 @@ static int substeps_impl(mpm_solver* s, int32_t nsub, const float* dts, bool bat
   for (int k = 0; k < nsub;) {
     if (s->unbounded && k == next_check) {
       next_check = std::min(k + kSegment, nsub);
-      TRY(follow_particles(s, next_check - k));
+      const int r = follow_particles(s, next_check - k);
+      // refused before anything changed: the call's last substep was the one before
+      if (r == MPM_EDOMAIN && k > 0) finish_grid(s);
+      if (r != MPM_OK) return r;
     }
     const int left = s->unbounded ? next_check - k : nsub - k;
     // (the call's last substep stays out of the graphs: it writes the grid)
