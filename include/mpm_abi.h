@@ -259,7 +259,8 @@ int mpm_get_tuning(mpm_solver* s, int32_t* chunk, int32_t* groups);
 /* g2p's occupancy (no reference counterpart): waves = 0 lets the compiler
  * allocate registers freely (5 waves per SIMD), 6 holds g2p to six waves
  * per SIMD (more grid-tile gathers in flight, which pays in sparse scenes
- * whose blocks hold few particles).  Results are bitwise the same either
+ * whose blocks hold few particles).  Small scenes, where g2p also runs the
+ * grid operator, keep the compiler's.  Results are bitwise the same either
  * way; MPMSolver.autotune() times both at the chosen launch shape. */
 int mpm_set_g2p_waves(mpm_solver* s, int32_t waves);
 int mpm_get_g2p_waves(mpm_solver* s, int32_t* waves);

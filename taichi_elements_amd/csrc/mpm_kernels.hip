@@ -55,6 +55,12 @@ __device__ __forceinline__ int4 wave_inclusive_scan4(int4 v) {
   return v;
 }
 
+// Set bits of mask below this lane.
+__device__ __forceinline__ int lanes_before(unsigned long long mask) {
+  return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                   __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
+}
+
 // Exclusive scan of one int4 per thread over a kThreads workgroup.
 __device__ __forceinline__ int4 block_exscan4(int4 v, int4* total, int4* wsum) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -1117,8 +1123,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
   __shared__ int2 nbr[TILES ? 27 : 1];  // chunk ranges of the neighbouring blocks
   // the particles of the earlier batches: direction | rank << 8, slot
   __shared__ int lcode[kChunkMax - kBatch], lid[kChunkMax - kBatch];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  // Packed, and at six waves, registers decide the occupancy: there the thread's
+  // index after the particle part is kept out of the compiler's sight, so that
+  // what is computed from it is not held through that part (packed 98 -> 90
+  // registers, five waves per SIMD instead of four; 3 to 5 spilled at six -> none;
+  // substeps of 778k packed, with the resident workgroups that go with it, 111.5
+  // -> 106.9 us, 300k 70.1 -> 67.7, 2M 220.3 -> 215.3).  Computing it again
+  // costs the others 1 to 2% (2D 400k 51.4 and 52.5, 3D 1M 129.1 and 130.5).
+  constexpr bool TIGHT = D == 3 && (Q || W >= 6);
+  const int wave0 = threadIdx.x >> 6, lane0 = threadIdx.x & 63;
+  const unsigned long long lt0 = lane0 == 0 ? 0ull : (~0ull >> (64 - lane0));
   float vmax = 0.0f;
   for (XcdItems it(totals[kTotChunks], kSpreadChunks); it.valid(); it.next()) {
     const int c = it.c;
@@ -1327,6 +1341,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
         }
       }
       if (!members) continue;  // no binning follows from this substep
+      int tid = threadIdx.x;
+      if (TIGHT) __asm__ volatile("" : "+v"(tid));
+      const int wave = TIGHT ? tid >> 6 : wave0, lane = TIGHT ? tid & 63 : lane0;
       // stable rank of the particle among the chunk's particles with the same
       // direction
       if (lane < 32) dwcnt[wave][lane] = 0;  // the wave's own row, in program order
@@ -1337,11 +1354,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
         const unsigned long long bal = __ballot(on);
         peers &= on ? bal : ~bal;
       }
-      const int rank = (int)__popcll(peers & lt);
+      const int rank = TIGHT ? lanes_before(peers) : (int)__popcll(peers & lt0);
       if (live && rank == 0) dwcnt[wave][dir] = (int)__popcll(peers);
       lds_barrier();
       const bool last = b0 + kBatch >= ck.z;
-      if (threadIdx.x < 64) {
+      if (tid < 64) {
         int run = 0;
         if (lane < 27) {
           run = dbase[lane];
@@ -1361,12 +1378,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W))) v
         if (last) {
           members[ck.y + dstart[dir] + r] = p;
         } else {
-          lcode[j - ck.y] = dir | (r << 8);
-          lid[j - ck.y] = p;
+          const int i = TIGHT ? b0 - ck.y + tid : j - ck.y;
+          lcode[i] = dir | (r << 8);
+          lid[i] = p;
         }
       }
       if (last)  // the earlier batches' particles (this thread's own entries)
-        for (int i = threadIdx.x; i < b0 - ck.y; i += kThreads)
+        for (int i = tid; i < b0 - ck.y; i += kThreads)
           members[ck.y + dstart[lcode[i] & 255] + (lcode[i] >> 8)] = lid[i];
       lds_barrier();
     }  // batches of the chunk
@@ -1878,15 +1896,13 @@ void launch_g2p(const Params* P, const int* slab, SubstepBuffers& B, int s_index
     TimerScope ts(tm, "k_g2p", st);
     auto kern = B.g2p_waves >= 6 ? (B.quant ? k_g2p<D, true, 6> : k_g2p<D, false, 6>)
                                  : (B.quant ? k_g2p<D, true, 1> : k_g2p<D, false, 1>);
-    if (B.grid_in_g2p)
-      kern = B.g2p_waves >= 6 ? (B.quant ? k_g2p<D, true, 6, true> : k_g2p<D, false, 6, true>)
-                              : (B.quant ? k_g2p<D, true, 1, true> : k_g2p<D, false, 1, true>);
+    if (B.grid_in_g2p) kern = B.quant ? k_g2p<D, true, 1, true> : k_g2p<D, false, 1, true>;
     // In 3D no more workgroups than are resident at once (1280): with more, the
     // ones that start in a second round leave the device uneven (2048 and 1280:
     // substeps of 300k 66.6 and 65.0 us, 1M 117.5 and 116.3, 4M 419 and 405; 16M
-    // g2p 645 and 568).  No gain in 2D (60.8 and 61.8 us at 400k) and packed (1M
-    // 120.2 and 119.2; a frame of 778k 8.5 and 8.8 ms).
-    const int resident = D == 2 || B.quant || B.grid_in_g2p
+    // g2p 645 and 568; packed 778k 109.9 and 106.9).  No gain in 2D (60.8 and 61.8
+    // us at 400k).
+    const int resident = D == 2 || B.grid_in_g2p
                              ? G
                              : std::min(G, resident_groups((const void*)kern));
     kern<<<xcd_groups(chunk_bound, resident), kThreads, 0, st>>>(
