@@ -25,6 +25,7 @@ constexpr int kScanTile = kThreads * kScanItems;    // 512 blocks per workgroup
 // not be able to fill an XCD with waiting tiles: three of them (a process has
 // four hardware queues) leave 24 of an XCD's 192 places free.
 constexpr int kScanTilesOnePass = 448;
+constexpr int kScanGroup = 128;  // tiles whose sums a larger window adds up together
 // Keys per workgroup of a sort pass: kRadixTile, or, while they make no more
 // than kRadixSmallTiles tiles, kRadixSmallTile (k_onesweep says why).  The
 // small tiles wait for each other as the scan's do, 16 on each XCD with places
@@ -52,8 +53,8 @@ struct LBState {
 // Totals written on the device by the block scan (read by persistent kernels).
 enum Total : int { kTotValid = 0, kTotChunks = 1, kTotActive = 2, kTotPBlocks = 3, kTotCount = 4 };
 
-// The block scan's published tile sums, which the transfer that follows clears
-// for the next scan.
+// The block scan's published tile or group sums, which the transfer that
+// follows clears for the next scan.
 struct ScanStatus {
   unsigned long long* words;
   int n;
@@ -88,7 +89,7 @@ struct SubstepBuffers {
   int* active;      // active grid blocks
   int* totals;      // kTot*
   int* ghist;       // radix digit histograms, 2 x [kMaxRadixPasses][256] (substep parity)
-  unsigned long long* scan_status;      // published tile sums of k_bscan [4 * tiles], zero between scans
+  unsigned long long* scan_status;      // tile or group sums of k_bscan [4 * tiles], zero between scans
   unsigned long long* lb_status_radix;  // look-back status of k_onesweep [256 * radix_cap]
   int64_t radix_cap;
   LBState* lbs;

@@ -284,9 +284,14 @@ __device__ __forceinline__ void lb_release(LBState* st, int ntiles, unsigned epo
 // first transfer, so there is no ticket, no epoch and no release.  With tickets, a look-back over prefixes and each
 // neighbour's count loaded behind a branch: 1M particles (99 tiles) 11.8 ->
 // 7.0 us, 2D 20k 6.1 -> 4.6, unbounded 50k 16.4 -> 7.8, use_g2p2g 300k 13.9 ->
-// 8.1.  Larger windows take the tile sums from k_bscan_reduce, every tile
-// adding up those before it (no kernel between the two): 16M, 512^3 58 ->
-// 41 us, a batch of 16 scenes 23 -> 14.
+// 8.1.  Larger windows take the tile sums from k_bscan_reduce, which also adds
+// them up by groups of kScanGroup tiles: every tile adds up the groups before
+// its own and the tiles of its own before it, a round of loads each up to the
+// largest window (2^24 blocks, 256 groups), and there is no kernel between the
+// two.  Substeps of 1M particles with a kernel between that scans the tile sums,
+// with every tile adding up all tiles before it, and with groups: 512^3 (4.6k
+// tiles) 212, 160 and 156 us, 800^3 (16.8k) 338, 287 and 232, 1000^3 (32.4k)
+// 493, 537 and 330 (the first with the other kernels of its time, ~45 us more).
 // ---------------------------------------------------------------------------
 constexpr unsigned long long kScanReady = 1ull << 32;
 
@@ -332,7 +337,7 @@ __global__ __launch_bounds__(kThreads) void k_bscan(
     int* __restrict__ pchunk_cnt, int4* __restrict__ chunks, int* __restrict__ active,
     int* __restrict__ totals, int* __restrict__ ghist, int* __restrict__ ghist_next,
     unsigned long long* __restrict__ status, const int4* __restrict__ tile_sums,
-    int* __restrict__ err, int* __restrict__ step) {
+    const int4* __restrict__ group_sums, int* __restrict__ err, int* __restrict__ step) {
   // one launch per substep: the substep counter of the max-velocity slots
   if (step && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(step, 1);
   __shared__ int4 wsum[kThreads / 64];
@@ -372,8 +377,10 @@ __global__ __launch_bounds__(kThreads) void k_bscan(
   static_assert(kThreads == 256, "one wave per scanned channel");
   if (tile_sums) {
     int4 before = make_int4(0, 0, 0, 0), all;
-#pragma unroll 4
-    for (int i = threadIdx.x; i < tile; i += kThreads) before = add4(before, tile_sums[i]);
+    const int group = tile / kScanGroup;
+    for (int i = threadIdx.x; i < group; i += kThreads) before = add4(before, group_sums[i]);
+    for (int i = group * kScanGroup + threadIdx.x; i < tile; i += kThreads)
+      before = add4(before, tile_sums[i]);
     block_exscan4(before, &all, wsum);
     if (threadIdx.x < 4) {
       const int c = threadIdx.x;
@@ -424,12 +431,14 @@ __global__ __launch_bounds__(kThreads) void k_bscan(
     for (int i = threadIdx.x; i < kMaxRadixPasses * kRadixBins; i += kThreads) ghist_next[i] = 0;
 }
 
-// Tile sums of a window too large for the single pass.
+// Tile sums and group sums (zero before) of a window too large for the single
+// pass.
 template <int D>
 __global__ __launch_bounds__(kThreads) void k_bscan_reduce(const Params* __restrict__ scenes,
                                                            const int* __restrict__ count,
                                                            int total_blocks, int chunk,
-                                                           int4* __restrict__ tile_sums) {
+                                                           int4* __restrict__ tile_sums,
+                                                           int4* __restrict__ group_sums) {
   __shared__ int4 wsum[kThreads / 64];
   const Params& P = scenes[0];  // the combined window extents
   int4 acc = make_int4(0, 0, 0, 0);
@@ -439,7 +448,12 @@ __global__ __launch_bounds__(kThreads) void k_bscan_reduce(const Params* __restr
     if (first + k < total_blocks) acc = add4(acc, block_values<D>(first + k, count, P, chunk));
   int4 tot;
   block_exscan4(acc, &tot, wsum);
-  if (threadIdx.x == 0) tile_sums[blockIdx.x] = tot;
+  if (threadIdx.x < 4) {
+    const int c = threadIdx.x;
+    const int v = c == 0 ? tot.x : c == 1 ? tot.y : c == 2 ? tot.z : tot.w;
+    reinterpret_cast<int*>(&tile_sums[blockIdx.x])[c] = v;
+    if (v) atomicAdd(&reinterpret_cast<int*>(&group_sums[blockIdx.x / kScanGroup])[c], v);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1739,14 +1753,15 @@ static void launch_binning(const Params* P, SubstepBuffers& B, hipStream_t st, T
   if (!scan_in_p2g<D>(B)) {
     TimerScope ts(tm, "k_bscan", st);
     const bool two_level = nparts > kScanTilesOnePass;
+    int4* group_sums = two_level ? reinterpret_cast<int4*>(B.scan_status) : nullptr;
     if (two_level) {
       k_bscan_reduce<D><<<nparts, kThreads, 0, st>>>(P, B.count, B.total_blocks, B.chunk,
-                                                     B.tile_sums);
+                                                     B.tile_sums, group_sums);
     }
     k_bscan<D><<<nparts, kThreads, 0, st>>>(
         P, B.count, B.count_next, B.total_blocks, B.chunk, nparts, B.full_sort ? passes : 0,
         B.pstart, B.pchunk_begin, B.pchunk_cnt, B.chunks, B.active, B.totals, ghist, ghist_next,
-        B.scan_status, two_level ? B.tile_sums : nullptr, B.err, B.step);
+        B.scan_status, two_level ? B.tile_sums : nullptr, group_sums, B.err, B.step);
   }
   if (B.full_sort) {
     TimerScope ts(tm, "k_radix", st);
@@ -1774,11 +1789,11 @@ static void launch_binning(const Params* P, SubstepBuffers& B, hipStream_t st, T
   }
 }
 
-// The block scan's status words (single-pass scans only), for the transfer
-// after it to clear.
+// The block scan's published tile sums, or the group sums of a larger window
+// (in the same array, two words each), for the transfer after it to clear.
 static ScanStatus scan_status(const SubstepBuffers& B) {
   const int tiles = div_up(B.total_blocks, kScanTile);
-  return {B.scan_status, tiles <= kScanTilesOnePass ? 4 * tiles : 0};
+  return {B.scan_status, tiles <= kScanTilesOnePass ? 4 * tiles : 2 * div_up(tiles, kScanGroup)};
 }
 
 static WindowScan window_scan(const SubstepBuffers& B) {
