@@ -73,7 +73,8 @@ class BatchScene(MPMSolver):
     # readout: the library returns the whole batch in insertion order
     def particle_info(self):
         full = self._batch._particle_info_all()
-        out = {k: v[self._rows()] for k, v in full.items()}
+        # its own arrays: a view would keep those of the whole batch alive
+        out = {k: np.require(v[self._rows()], requirements="O") for k, v in full.items()}
         if self.use_emitter_id:
             out['emitter_ids'] = self._emitter_ids.copy()
         return out
@@ -262,7 +263,10 @@ class MPMSolverBatch:
         return {'position': x, 'velocity': v, 'material': m, 'color': c}
 
     def particle_info(self):
-        """``particle_info()`` of every scene from one readback."""
+        """``particle_info()`` of every scene from one readback.  The arrays of
+        a scene whose particles were added in one run are views of the batch's
+        (writable, no two overlap), which live as long as any of them; copy
+        what is kept longer than the rest."""
         full = self._particle_info_all()
         return [{k: v[s._rows()] for k, v in full.items()} for s in self.scenes]
 
