@@ -12,6 +12,7 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -155,7 +156,7 @@ struct mpm_solver {
   LBState* lbs = nullptr;
   int* ghist = nullptr;
   float4* grid = nullptr;
-  int* totals = nullptr;  // 2 x 16 (substep parity)
+  int* totals = nullptr;  // 2 x 16 (substep parity), with the error bits behind them (err)
   int last_parity = 0;
   int* err = nullptr;
   unsigned* maxv = nullptr;
@@ -166,8 +167,9 @@ struct mpm_solver {
   unsigned* host_words = nullptr;
   unsigned* own_words = nullptr;
   int host_words_cap = 0;
-  // chunks of the last substep whose maxima were read (0: none yet): which of
-  // two equal ways the grid operator goes, never what it gives
+  // chunks of the last substep that the host waited for, by any call (0: none
+  // yet, or the chunk size changed): which of two equal ways the binning and the
+  // grid operator go, never what they give
   std::atomic<int> chunks_seen{0};
   // read access to the particles: device staging in insertion order and the
   // copies to the caller's memory; read_mu: readers of one handle take turns
@@ -307,12 +309,23 @@ int report_errors(mpm_solver* s, int e) {
   return MPM_OK;
 }
 
+// The totals and the error bits behind them, copied to the host together.
+struct DeviceWords {
+  int totals[2][16];
+  int err;
+};
+
+int take_words(mpm_solver* s, const DeviceWords& w) {
+  if (s->have_perm) s->chunks_seen = w.totals[s->last_parity][kTotChunks];
+  return report_errors(s, w.err);
+}
+
 int check_device_errors(mpm_solver* s) {
   HIP_TRY(hipSetDevice(s->device));
   HIP_TRY(hipStreamSynchronize(s->stream));
-  int e = 0;
-  HIP_TRY(hipMemcpy(&e, s->err, sizeof(int), hipMemcpyDeviceToHost));
-  return report_errors(s, e);
+  DeviceWords w{};
+  HIP_TRY(hipMemcpy(&w, s->totals, sizeof(w), hipMemcpyDeviceToHost));
+  return take_words(s, w);
 }
 
 // Device staging of the readers, 28 bytes a particle for mpm_particle_info and
@@ -339,12 +352,13 @@ int stage_reserve(mpm_solver* s, size_t bytes) {
   return MPM_OK;
 }
 
-// The segments and the error bits to the host, after the stream's work so far.
+// The segments, the totals and the error bits to the host, after the stream's
+// work so far.
 int read_back(mpm_solver* s, std::vector<Readback::Segment> segments) {
-  int e = 0;
-  segments.push_back({s->err, &e, sizeof(int), false});
+  DeviceWords w{};
+  segments.push_back({s->totals, &w, sizeof(w), false});
   HIP_TRY(s->readback.copy(segments, s->stream));
-  return report_errors(s, e);
+  return take_words(s, w);
 }
 
 void fill_params(Params& P, const mpm_solver* s, const SceneHost& sc, float dt, int skip) {
@@ -1043,7 +1057,7 @@ static int create_impl(const mpm_config* cfgs, int nscenes, mpm_solver** out) {
     return r;
   }
   if ((r = dalloc(&s->lbs, 1)) || (r = dalloc(&s->ghist, 2 * kMaxRadixPasses * kRadixBins)) ||
-      (r = dalloc(&s->totals, 32)) || (r = dalloc(&s->err, 1)) ||
+      (r = dalloc(&s->totals, sizeof(DeviceWords) / sizeof(int))) ||
       (r = dalloc(&s->maxv, 16 * s->persistent_groups)) ||
       (r = dalloc(&s->d_params, nscenes)) || (r = dalloc(&s->d_step, 1)) ||
       (r = dalloc(&s->d_gvmax, 1)) ||
@@ -1051,6 +1065,7 @@ static int create_impl(const mpm_config* cfgs, int nscenes, mpm_solver** out) {
     mpm_destroy(s);
     return r;
   }
+  s->err = s->totals + offsetof(DeviceWords, err) / sizeof(int);
   s->maxv_cap = 16 * s->persistent_groups;
   s->host_words_cap = 256;
   if (hipHostMalloc((void**)&s->h_params,
@@ -1065,8 +1080,7 @@ static int create_impl(const mpm_config* cfgs, int nscenes, mpm_solver** out) {
   if (hipMemsetAsync(s->lbs, 0, sizeof(LBState), s->stream) != hipSuccess ||
       hipMemsetAsync(s->ghist, 0, sizeof(int) * 2 * kMaxRadixPasses * kRadixBins, s->stream) !=
           hipSuccess ||
-      hipMemsetAsync(s->totals, 0, sizeof(int) * 32, s->stream) != hipSuccess ||
-      hipMemsetAsync(s->err, 0, sizeof(int), s->stream) != hipSuccess ||
+      hipMemsetAsync(s->totals, 0, sizeof(DeviceWords), s->stream) != hipSuccess ||
       hipStreamSynchronize(s->stream) != hipSuccess) {
     mpm_destroy(s);
     return fail(MPM_EHIP, "initialising solver buffers failed");
@@ -1111,7 +1125,6 @@ int mpm_destroy(mpm_solver* s) {
   dfree(s->grid);
   dfree(s->grid_alt);
   dfree(s->totals);
-  dfree(s->err);
   dfree(s->maxv);
   dfree(s->d_params);
   dfree(s->d_slab);
@@ -1432,7 +1445,7 @@ int mpm_read_max_velocity(mpm_solver* s, int32_t nsub, float* out) {
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(s->stream));
   if (nsub > 0) std::memcpy(out, s->host_words, sizeof(float) * nsub);
-  s->chunks_seen = (int)s->host_words[nsub + 1];
+  if (s->have_perm) s->chunks_seen = (int)s->host_words[nsub + 1];
   return report_errors(s, (int)s->host_words[nsub]);
 }
 
@@ -1964,6 +1977,7 @@ int mpm_set_tuning(mpm_solver* s, int32_t chunk, int32_t groups) {
   }
   if (chunk != 0 && chunk != s->chunk) {
     s->chunk = chunk;
+    s->chunks_seen = 0;
     if (s->cap > 0) TRY(alloc_chunk_buffers(s));
   }
   // the next substep bins from scratch (chunk boundaries changed)
