@@ -337,8 +337,9 @@ def quant_bench(x, v, m, steps, warmup, autotune=True):
 
 def small2d_bench(steps=100, repeats=3):
     """The reference's own small case: 2D, 128^2, 20,000 water particles in
-    [0.2, 0.5] x [0.4, 0.8] (seed 0), 100 substeps at default_dt -- timed
-    with HIP graph replay of substep pairs and kernel by kernel."""
+    [0.2, 0.5] x [0.4, 0.8] (seed 0), 100 substeps at default_dt -- kernel by
+    kernel (the default, whose rate is reported) and with HIP graph replay of
+    substep pairs beside it."""
     from taichi_elements_amd import MPMSolver
     from taichi_elements_amd._lib import check
     from taichi_elements_amd._lib import lib as _l
@@ -347,7 +348,7 @@ def small2d_bench(steps=100, repeats=3):
     x = (np.array([0.2, 0.4], np.float32)
          + rng.random((20000, 2), dtype=np.float32) * np.array([0.3, 0.4], np.float32))
     out = {}
-    for graphs in (True, False):
+    for graphs in (False, True):
         s = MPMSolver(res=(128, 128))
         s.set_graphs(graphs)
         s.read_restart(len(x), x, np.zeros_like(x), np.zeros(len(x), np.int32),
@@ -362,8 +363,8 @@ def small2d_bench(steps=100, repeats=3):
             best = el if best is None else min(best, el)
         out["graphs" if graphs else "kernel_by_kernel"] = 1e6 * best / steps
         del s
-    return dict(us_per_substep=out, speedup=out["kernel_by_kernel"] / out["graphs"],
-                value=20000 / (out["graphs"] * 1e-6), unit="particle-substeps/s",
+    return dict(us_per_substep=out, graphs_over_default=out["graphs"] / out["kernel_by_kernel"],
+                value=20000 / (out["kernel_by_kernel"] * 1e-6), unit="particle-substeps/s",
                 workload="2D water, 128^2, 20k particles, default_dt, 100 substeps per call")
 
 
@@ -540,7 +541,7 @@ def main():
     ap.add_argument("--no-batched", action="store_true",
                     help="skip the 64-scene batched measurement")
     ap.add_argument("--no-small2d", action="store_true",
-                    help="skip the 2D reference-sized scene (graphs vs kernel by kernel)")
+                    help="skip the 2D reference-sized scene")
     ap.add_argument("--no-quant", action="store_true",
                     help="skip the packed-storage (quant=True) legs")
     ap.add_argument("--no-g2p2g", action="store_true",
