@@ -23,6 +23,11 @@
  *    leave the simulated window are reported by the next call that
  *    synchronises (mpm_read_max_velocity, mpm_particle_info, mpm_get_state,
  *    mpm_sync).
+ *  - The readers (mpm_particle_info, mpm_get_state) keep their staging with
+ *    the handle until mpm_destroy: from the second read on up to 8 MiB of
+ *    pinned host memory, and on the device 28 and up to 36 bytes a 3D
+ *    particle, as long as that is no more than 1 GiB (a larger one is freed
+ *    after each read).
  */
 #ifndef MPM_ABI_H
 #define MPM_ABI_H
@@ -251,7 +256,10 @@ int mpm_set_graphs(mpm_solver* s, int32_t enabled);
 /* Launch tuning (no reference counterpart; the reference leaves launch
  * shapes to Taichi).  chunk: particles per transfer work item (16-1024);
  * groups: workgroups of the persistent transfer kernels (64-16384); 0 keeps
- * a value.  The next substep re-bins from scratch; results change only by
+ * a value.  p2g takes four times groups past 160k particles, and in 3D g2p
+ * (while it reads the grid from memory) and use_g2p2g (up to 768k particles)
+ * take no more than the device holds at once, 1280 or 1536 and 768: groups
+ * beyond that change p2g alone.  The next substep re-bins from scratch; results change only by
  * float32 summation order.  MPMSolver.autotune() times candidates on the
  * live scene and keeps the fastest. */
 int mpm_set_tuning(mpm_solver* s, int32_t chunk, int32_t groups);

@@ -165,8 +165,7 @@ void launch_front(const Params* P, const int* slab, SubstepBuffers& B, int raw_g
 // state pf_in: gout = adjoints of the new state, gin = adjoints of the old
 // state (both laid out like pf), gE (may be null) = adjoint of the
 // per-particle Young's modulus, gnu[0] = adjoint of nu.  gbar holds
-// total_blocks * nodes float4, abuf D*D * cap floats, nu_part
-// persistent_groups floats.
+// total_blocks * nodes float4, nu_part persistent_groups floats.
 template <int D>
 void launch_adjoint(const Params* P, const int* slab, SubstepBuffers& B, const float* pf_in,
                     const float* gout, float* gin, float* gE, float4* gbar,
@@ -200,7 +199,8 @@ void launch_scatter_i(const int* src, int64_t cap, int ncomp, const int* orig, i
 // x, v (n, D) and material in insertion order (null: not wanted).
 void launch_particle_info(int D, bool quant, bool g2p2g, const float* pf, const int* pi,
                           int64_t cap, int n, float* x, float* v, int* mat, hipStream_t st);
-// out[r] = max of part[r * stride .. + stride), r < rows; out[rows] = *err.
+// out[r] = max of part[r * stride .. + stride), r < rows; out[rows] = *err,
+// out[rows + 1] = totals[kTotChunks].
 void launch_max_rows(const unsigned* part, int rows, int stride, const int* err,
                      const int* totals, unsigned* out, hipStream_t st);
 void launch_fill_u32(unsigned* p, unsigned v, int64_t n, hipStream_t st);

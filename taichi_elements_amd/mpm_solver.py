@@ -149,7 +149,7 @@ SNAPSHOT_SAVE, SNAPSHOT_RESTORE, SNAPSHOT_RELEASE = 0, 1, 2
 def _autotune(obj, handle, dt, substeps, chunks, groups, verbose, dts):
     """Shared by MPMSolver and MPMSolverBatch: time each launch shape on
     the live particles.  Four untimed substeps after each change re-bin,
-    reorder the slots and capture the shape's substep-pair graph; the
+    reorder the slots and show the shape's number of chunks; the
     shape's time is the best of three timed runs of ``substeps``.  The
     scene is put back from a device snapshot (mpm_snapshot) before every
     candidate and at the end: the particle slots and, with use_g2p2g, the
