@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -28,30 +29,58 @@ class Readback {
     bool on_host;
   };
 
-  // Waits for the stream's work so far and for the copies.
+  // Waits for the stream's work so far and for the copies.  Without pinned
+  // memory (or host memory for the bookkeeping) they are plain ones.
   hipError_t copy(const std::vector<Segment>& segments, hipStream_t st) {
-    std::vector<Piece> pieces;
+    if (again_) {  // a single read does not pay for pinned memory (~0.2 ms per MiB)
+      bool began = false;
+      const hipError_t e = through_slots(segments, st, began);
+      if (began) return e;
+      (void)hipGetLastError();
+    }
+    again_ = true;
+    hipError_t e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return e;
+    for (const Segment& s : segments) {
+      if (s.bytes == 0) continue;
+      if (s.on_host)
+        std::memcpy(s.dst, s.src, s.bytes);
+      else if ((e = hipMemcpy(s.dst, s.src, s.bytes, hipMemcpyDeviceToHost)) != hipSuccess)
+        return e;
+    }
+    return hipSuccess;
+  }
+
+  void release() {
+    for (int k = 0; k < kSlots; k++) {
+      if (done_[k]) hipEventDestroy(done_[k]);
+      if (slot_[k]) hipHostFree(slot_[k]);
+      done_[k] = nullptr;
+      slot_[k] = nullptr;
+    }
+  }
+
+ private:
+  static constexpr int kSlots = 4;
+  static constexpr size_t kSlotBytes = 2u << 20;
+  struct Piece {
+    const char* src;
+    char* dst;
+    size_t bytes;
+    bool on_host;
+  };
+
+  // began: everything the copies need is there.
+  hipError_t through_slots(const std::vector<Segment>& segments, hipStream_t st, bool& began) {
     size_t device = 0, all = 0;
     for (const Segment& s : segments) {
       if (!s.on_host) device += s.bytes;
       all += s.bytes;
     }
-    hipError_t e;
-    if (!again_) {  // a single read does not pay for pinned memory (~0.2 ms per MiB)
-      again_ = true;
-      if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
-      for (const Segment& s : segments) {
-        if (s.bytes == 0) continue;
-        if (s.on_host)
-          std::memcpy(s.dst, s.src, s.bytes);
-        else if ((e = hipMemcpy(s.dst, s.src, s.bytes, hipMemcpyDeviceToHost)) != hipSuccess)
-          return e;
-      }
-      return hipSuccess;
-    }
-    e = reserve(device <= kSlotBytes ? 1 : kSlots);
+    hipError_t e = reserve(device <= kSlotBytes ? 1 : kSlots);
     if (e != hipSuccess) return e;
     if (device <= kSlotBytes) {  // one slot holds everything
+      began = true;
       size_t at = 0;
       for (size_t i = 0; i < segments.size();) {  // neighbours on the device in one copy
         const Segment& s = segments[i++];
@@ -75,33 +104,22 @@ class Readback {
       }
       return hipSuccess;
     }
+    std::vector<Piece> pieces;
+    std::vector<std::atomic<int>> moved;
+    try {
+      for (const Segment& s : segments)
+        for (size_t at = 0; at < s.bytes; at += kSlotBytes)
+          pieces.push_back({(const char*)s.src + at, (char*)s.dst + at,
+                            std::min(kSlotBytes, s.bytes - at), s.on_host});
+      moved = std::vector<std::atomic<int>>(pieces.size());
+    } catch (const std::bad_alloc&) {
+      return hipErrorOutOfMemory;
+    }
+    began = true;
     e = hipStreamSynchronize(st);  // no thread waits for kernels
     if (e != hipSuccess) return e;
-    for (const Segment& s : segments)
-      for (size_t at = 0; at < s.bytes; at += kSlotBytes)
-        pieces.push_back({(const char*)s.src + at, (char*)s.dst + at,
-                          std::min(kSlotBytes, s.bytes - at), s.on_host});
-    return pipeline(pieces, st, all);
+    return pipeline(pieces, moved, st, all);
   }
-
-  void release() {
-    for (int k = 0; k < kSlots; k++) {
-      if (done_[k]) hipEventDestroy(done_[k]);
-      if (slot_[k]) hipHostFree(slot_[k]);
-      done_[k] = nullptr;
-      slot_[k] = nullptr;
-    }
-  }
-
- private:
-  static constexpr int kSlots = 4;
-  static constexpr size_t kSlotBytes = 2u << 20;
-  struct Piece {
-    const char* src;
-    char* dst;
-    size_t bytes;
-    bool on_host;
-  };
 
   // The first n slots and their events.
   hipError_t reserve(int n) {
@@ -123,10 +141,10 @@ class Readback {
   // Piece k passes through slot k % kSlots.  Every mover copies its share of
   // each piece once the piece has arrived; a slot is refilled when all movers
   // are done with it.
-  hipError_t pipeline(const std::vector<Piece>& pieces, hipStream_t st, size_t bytes) {
+  hipError_t pipeline(const std::vector<Piece>& pieces, std::vector<std::atomic<int>>& moved,
+                      hipStream_t st, size_t bytes) {
     const int n = (int)pieces.size();
     std::atomic<int> arrived{0};
-    std::vector<std::atomic<int>> moved(n);
     for (auto& m : moved) m.store(0, std::memory_order_relaxed);
     const int hw = (int)std::max(2u, std::thread::hardware_concurrency());
     const int want = (int)std::min<size_t>({(size_t)kMovers, (size_t)hw / 2, 1 + bytes / (4u << 20)});
